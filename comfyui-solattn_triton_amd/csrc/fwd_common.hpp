@@ -64,47 +64,46 @@ struct TileDesc {
 // query blocks of the same heads, which keeps their K/V blocks in that XCD's
 // L2. Within each window of WIN consecutive dispatches on an XCD (the query
 // blocks that run there together) the query blocks are taken longest first,
-// by exact-block count: the window's counts are ranked in LDS and this
-// workgroup takes the query block whose rank is its place in the window. Same
-// L2 footprint, shorter tail per window (4-9% faster forwards at cfg 2). A
-// window spans kLptTokens query tokens: 64 dispatches at block 128, 128 at
-// block 64 (a 128-dispatch window is 3-4% faster than 64 at block 64, and
-// 256 is slower at both sizes).
+// by exact-block count: this workgroup takes the query block whose rank in the
+// window is its place there. Same L2 footprint, shorter tail per window (4-9%
+// faster forwards at cfg 2). A window spans kLptTokens query tokens: 64
+// dispatches at block 128, 128 at block 64 (a 128-dispatch window is 3-4%
+// faster than 64 at block 64, and 256 is slower at both sizes).
+//
+// The rank is found without LDS or barriers: each wave holds the window's keys
+// (count, then earlier index first; unique) in WIN / 64 registers and builds
+// the r-th largest key bit by bit from ballots, 0.4 us. (Ranking every entry
+// against every other in LDS took 1.2 us alone and 4-6 us beside the MFMA
+// waves of other workgroups.)
 constexpr int kLptTokens = 8192;
 template <int WIN>
 __device__ __forceinline__ void tile_coords_lpt(const int32_t* __restrict__ counts, int NT, int& bh,
                                                 int& qb) {
-  static_assert(WIN > 0 && (WIN & (WIN - 1)) == 0, "window offsets are taken with masks");
-  __shared__ int s_cnt[WIN];
-  __shared__ int s_pick;
+  static_assert(WIN >= 64 && (WIN & (WIN - 1)) == 0, "a window is whole waves, offsets are masks");
+  constexpr int R = WIN / 64, kIdxBits = __builtin_ctz(WIN);
   const uint32_t w = blockIdx.x, total = gridDim.x;
-  uint32_t base, r, nwin;
-  if ((total & 7u) == 0u) {
-    const uint32_t per = total >> 3, li = w >> 3;
-    base = (w & 7u) * per + (li & ~(WIN - 1u));
-    r = li & (WIN - 1u);
-    nwin = min(static_cast<uint32_t>(WIN), per - (li & ~(WIN - 1u)));
-  } else {
-    base = w & ~(WIN - 1u);
-    r = w & (WIN - 1u);
-    nwin = min(static_cast<uint32_t>(WIN), total - base);
+  // XCD x serves total / 8 query blocks, one more for the first total % 8 XCDs
+  const uint32_t x = w & 7u, li = w >> 3, q8 = total >> 3, rem = total & 7u;
+  const uint32_t per = q8 + (x < rem ? 1u : 0u), win0 = li & ~(WIN - 1u);
+  const uint32_t base = x * q8 + min(x, rem) + win0;
+  const int r = static_cast<int>(li - win0), nwin = static_cast<int>(min(static_cast<uint32_t>(WIN), per - win0));
+  const int lane = threadIdx.x & 63;
+  int key[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int i = lane + 64 * u;
+    const int c = min(max(counts[base + min(i, nwin - 1)], 0), NT);  // any counts give a permutation
+    key[u] = i < nwin ? (c << kIdxBits) | (WIN - 1 - i) : -1;
   }
-  // Strided over the workgroup so that every window slot is filled and ranked
-  // whatever the thread count; exactly one slot has rank r, so s_pick is set.
-  for (int t = threadIdx.x; t < WIN; t += blockDim.x)
-    s_cnt[t] = t < static_cast<int>(nwin) ? counts[base + t] : -1;
-  __syncthreads();
-  for (int t = threadIdx.x; t < static_cast<int>(nwin); t += blockDim.x) {
-    const int mine = s_cnt[t];
-    int rank = 0;
-    for (int u = 0; u < static_cast<int>(nwin); ++u) {
-      const int cu = s_cnt[u];
-      rank += (cu > mine) || (cu == mine && u < t);
-    }
-    if (rank == static_cast<int>(r)) s_pick = t;
+  int sel = 0;
+  for (int bit = 31 - __builtin_clz(NT) + kIdxBits; bit >= 0; --bit) {
+    const int cand = sel | (1 << bit);
+    int n = 0;
+#pragma unroll
+    for (int u = 0; u < R; ++u) n += __popcll(__ballot(key[u] >= cand));
+    if (n > r) sel = cand;
   }
-  __syncthreads();
-  const uint32_t logical = base + static_cast<uint32_t>(s_pick);
+  const uint32_t logical = base + static_cast<uint32_t>(WIN - 1 - (sel & (WIN - 1)));
   bh = static_cast<int>(logical / static_cast<uint32_t>(NT));
   qb = static_cast<int>(logical % static_cast<uint32_t>(NT));
 }

@@ -68,10 +68,14 @@ struct TileDesc {
 // window is its place there. Same L2 footprint, shorter tail per window (4-9%
 // faster forwards at cfg 2). A window spans kLptTokens query tokens: 64
 // dispatches at block 128, 128 at block 64 (a 128-dispatch window is 3-4%
-// faster than 64 at block 64, and 256 is slower at both sizes).
+// faster than 64 at block 64, and 256 is slower at both sizes). An XCD's last
+// window spans up to two of them: what runs last is what leaves CUs idle, and
+// there the order is worth more than the L2 footprint (4096 tokens at block 64,
+// 192 dispatches an XCD: call 95.5 -> 93 us; 9180 tokens 259 -> 254 us; 32760
+// tokens within noise).
 //
 // The rank is found without LDS or barriers: each wave holds the window's keys
-// (count, then earlier index first; unique) in WIN / 64 registers and builds
+// (count, then earlier index first; unique) in 2 WIN / 64 registers and builds
 // the r-th largest key bit by bit from ballots, 0.4 us. (Ranking every entry
 // against every other in LDS took 1.2 us alone and 4-6 us beside the MFMA
 // waves of other workgroups.)
@@ -80,20 +84,23 @@ template <int WIN>
 __device__ __forceinline__ void tile_coords_lpt(const int32_t* __restrict__ counts, int NT, int& bh,
                                                 int& qb) {
   static_assert(WIN >= 64 && (WIN & (WIN - 1)) == 0, "a window is whole waves, offsets are masks");
-  constexpr int R = WIN / 64, kIdxBits = __builtin_ctz(WIN);
+  constexpr int kTail = 2 * WIN, R = kTail / 64, kIdxBits = __builtin_ctz(kTail);
   const uint32_t w = blockIdx.x, total = gridDim.x;
   // XCD x serves total / 8 query blocks, one more for the first total % 8 XCDs
   const uint32_t x = w & 7u, li = w >> 3, q8 = total >> 3, rem = total & 7u;
-  const uint32_t per = q8 + (x < rem ? 1u : 0u), win0 = li & ~(WIN - 1u);
+  const uint32_t per = q8 + (x < rem ? 1u : 0u);
+  const uint32_t tail0 = per > WIN ? (per - 1u - WIN) & ~(WIN - 1u) : 0u;  // the last window: WIN < size <= 2 WIN
+  const uint32_t win0 = min(li & ~(WIN - 1u), tail0);
   const uint32_t base = x * q8 + min(x, rem) + win0;
-  const int r = static_cast<int>(li - win0), nwin = static_cast<int>(min(static_cast<uint32_t>(WIN), per - win0));
+  const int r = static_cast<int>(li - win0);
+  const int nwin = static_cast<int>(win0 == tail0 ? per - win0 : static_cast<uint32_t>(WIN));
   const int lane = threadIdx.x & 63;
   int key[R];
 #pragma unroll
   for (int u = 0; u < R; ++u) {
     const int i = lane + 64 * u;
     const int c = min(max(counts[base + min(i, nwin - 1)], 0), NT);  // any counts give a permutation
-    key[u] = i < nwin ? (c << kIdxBits) | (WIN - 1 - i) : -1;
+    key[u] = i < nwin ? (c << kIdxBits) | (kTail - 1 - i) : -1;
   }
   int sel = 0;
   for (int bit = 31 - __builtin_clz(NT) + kIdxBits; bit >= 0; --bit) {
@@ -103,7 +110,7 @@ __device__ __forceinline__ void tile_coords_lpt(const int32_t* __restrict__ coun
     for (int u = 0; u < R; ++u) n += __popcll(__ballot(key[u] >= cand));
     if (n > r) sel = cand;
   }
-  const uint32_t logical = base + static_cast<uint32_t>(WIN - 1 - (sel & (WIN - 1)));
+  const uint32_t logical = base + static_cast<uint32_t>(kTail - 1 - (sel & (kTail - 1)));
   bh = static_cast<int>(logical / static_cast<uint32_t>(NT));
   qb = static_cast<int>(logical % static_cast<uint32_t>(NT));
 }

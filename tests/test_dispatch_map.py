@@ -70,33 +70,37 @@ def test_dispatch_map_longest_first_within_window(threads, WINDOW):
 
 def _select(counts, WINDOW, NT):
     """The kernel's selection: XCD shares of total // 8 (+1 for the first
-    total % 8), unique keys (count clamped to [0, NT], earlier index first),
-    the r-th largest key built bit by bit."""
-    total, bits = len(counts), WINDOW.bit_length() - 1
+    total % 8), windows of WINDOW dispatches with a last one of up to two,
+    unique keys (count clamped to [0, NT], earlier index first), the r-th
+    largest key built bit by bit."""
+    total, idx = len(counts), 2 * WINDOW
+    bits = idx.bit_length() - 1
     out = np.empty(total, dtype=np.int64)
     for w in range(total):
         x, li, q8, rem = w & 7, w >> 3, total >> 3, total & 7
-        per, win0 = q8 + (x < rem), li & ~(WINDOW - 1)
-        base = x * q8 + min(x, rem) + win0
-        r, nwin = li - win0, min(WINDOW, per - win0)
-        assert 0 <= r < nwin and 0 <= base and base + nwin <= total
-        key = [(min(max(counts[base + i], 0), NT) << bits) | (WINDOW - 1 - i) for i in range(nwin)]
+        per = q8 + (x < rem)
+        tail0 = (per - 1 - WINDOW) & ~(WINDOW - 1) if per > WINDOW else 0
+        win0 = min(li & ~(WINDOW - 1), tail0)
+        base, r = x * q8 + min(x, rem) + win0, li - win0
+        nwin = per - win0 if win0 == tail0 else WINDOW
+        assert 0 <= r < nwin <= idx and 0 <= base and base + nwin <= total
+        key = [(min(max(counts[base + i], 0), NT) << bits) | (idx - 1 - i) for i in range(nwin)]
         sel = 0
         for bit in range(NT.bit_length() - 1 + bits, -1, -1):
             if sum(k >= sel | (1 << bit) for k in key) > r:
                 sel |= 1 << bit
-        out[w] = base + WINDOW - 1 - (sel & (WINDOW - 1))
+        out[w] = base + idx - 1 - (sel & (idx - 1))
     return out
 
 
-@pytest.mark.parametrize("total", [1, 7, 8, 9, 63, 65, 513, 1031, 2056])
+@pytest.mark.parametrize("total", [1, 7, 8, 9, 65, 513, 8 * 64, 8 * 128 + 8, 8 * 192, 2056, 3079])
 @pytest.mark.parametrize("window", [64, 128])
 def test_window_selection(total, window):
     """A permutation for any counts (negative and beyond NT too) and any grid;
-    for whole XCD shares, the entry that ranking the window gives."""
+    for XCD shares of one window, the entry that ranking the window gives."""
     rng = np.random.default_rng(total + window)
     counts = rng.integers(-2, 12, size=total).tolist()
     assert sorted(_select(counts, window, 8).tolist()) == list(range(total))
-    if total % 8 == 0:
+    if total % 8 == 0 and total // 8 <= window:
         counts = rng.integers(0, 9, size=total).tolist()
         assert np.array_equal(_select(counts, window, 8), _mapping(counts, 256, window))

@@ -41,7 +41,9 @@ namespace bf16fwd {
 // one P word, the operands are read two MFMAs ahead, and the lazy tile max
 // works the same way (also catching the first exact tile when no plain tile
 // came before it: running max -inf, p = inf).
-template <typename Mid>
+// POOLED: tile n is a pooled tile of whole blocks (its masked scores -inf):
+// each key weighs BLK in the row sum, which adds the fp32 p.
+template <int BLK, bool POOLED, typename Mid>
 __device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32x16 (&sn)[2],
                                           uint32_t kl, uint32_t vl, const bf16x8 (&q)[8],
                                           float c, int lane, Mid&& mid) {
@@ -64,7 +66,8 @@ __device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32
       mfma_v(sn[i & 1], ka[i % 3], q[i >> 1]);
     const int ks = i >> 2, w = i & 3;
     const int r = 8 * (ks & 1) + 2 * w;
-    pw[ks][w] = exp_pair(sc[ks >> 1][r], sc[ks >> 1][r + 1], c, neg, psum);
+    pw[ks][w] = POOLED ? exp_pair_f32sum(sc[ks >> 1][r], sc[ks >> 1][r + 1], c, neg, psum)
+                       : exp_pair(sc[ks >> 1][r], sc[ks >> 1][r + 1], c, neg, psum);
   }
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks)
@@ -78,15 +81,24 @@ __device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32
     if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
       st.m = m_new;
       psum = 0.f;
-      psum = exp8<0>(sc[0], c, -m_new, pb[0], psum);
-      psum = exp8<8>(sc[0], c, -m_new, pb[1], psum);
-      psum = exp8<0>(sc[1], c, -m_new, pb[2], psum);
-      psum = exp8<8>(sc[1], c, -m_new, pb[3], psum);
+      if constexpr (POOLED) {
+#pragma unroll
+        for (int r = 0; r < 32; ++r) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r >> 4][r & 15], c, -m_new));
+          pb[r >> 3][r & 7] = static_cast<__bf16>(p);
+          psum += p;
+        }
+      } else {
+        psum = exp8<0>(sc[0], c, -m_new, pb[0], psum);
+        psum = exp8<8>(sc[0], c, -m_new, pb[1], psum);
+        psum = exp8<0>(sc[1], c, -m_new, pb[2], psum);
+        psum = exp8<8>(sc[1], c, -m_new, pb[3], psum);
+      }
       mfma_fence(st.acc);  // the rescale reads O
       rescale(st, alpha);
     }
   }
-  st.l = fmaf(st.l, alpha, psum);
+  st.l = fmaf(st.l, alpha, POOLED ? psum * static_cast<float>(BLK) : psum);
   mid();
   va[0] = v_op_x(vl, 0, 0);
   va[1] = v_op_x(vl, 0, 1);
@@ -207,19 +219,15 @@ __device__ __forceinline__ void step3(SoftmaxState& st, const f32x16 (&sc)[2], f
   st.l = fmaf(st.l, alpha, psum);
 }
 
-// Tile n of this kernel's order: pooled tiles, the ragged exact tile (if
-// any), then the full exact tiles in ascending key order.
-template <int BLK>
-__device__ __forceinline__ TileDesc desc(const TileList& tl, int n, int nrag, int T, int NT) {
-  if (n < tl.npool) return pooled_desc(tl, n, NT);
-  if (n < tl.npool + nrag) return exact_desc<BLK>(tl, tl.nexact - 1, T, NT);
-  return exact_desc<BLK>(tl, n - tl.npool - nrag, T, NT);
-}
-
 // Block 64 forward (workgroups of 2 waves). K and V are single buffered
 // (32 KiB), so four workgroups and two waves per SIMD fit a CU; the pipeline
 // step waits twice (K refilled after the QK phase, V after P.V). Tile order:
-// pooled tiles, the ragged exact tile (if any), then the full exact tiles.
+// with T not a multiple of 64, the tile of the short last block through the
+// plain path (as a ragged exact tile, or inside its pooled tile, where it
+// weighs its own length); then the pooled and the full exact tiles through the
+// pipeline. (Pooled tiles on the plain path, each with its own waits and no
+// overlap, took 4.1 us against 1.7 us of a pipelined exact tile: 15% of a
+// workgroup's time at 32760 tokens.)
 template <int BLK>
 __global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))
 fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
@@ -242,10 +250,10 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
 
   const int ntiles = build_tile_list<BLK>(tl, mask, row, NT, W, T);
   if (ntiles == 0) return;  // cannot happen for routed masks: the diagonal is exact
-  // The last exact tile is ragged when block NT-1 is exact and T is not a
-  // multiple of 64 (exact blocks are listed in ascending order).
-  const int nrag = ragged_tiles(tl, NT, T);
-  const int nplain = tl.npool + nrag;
+  const int nplain = T % kKeys != 0 ? 1 : 0;
+  const bool rag = ragged_tiles(tl, NT, T) != 0;  // the plain tile is exact, else pooled
+  const int npool = tl.npool - (nplain && !rag ? 1 : 0);  // pipelined pooled tiles, first in order
+  const int npipe = ntiles - nplain;
 
   const KVSource src{k + b * sk_b + h * sk_h, sk_t, v + b * sv_b + h * sv_h, sv_t,
                      kc + (static_cast<int64_t>(b) * npad * H + h) * kD,
@@ -254,120 +262,129 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
   off.init(sk_t, sv_t);
   const uint32_t kb = lds_addr(kbuf), vb = lds_addr(vbuf);  // LDS byte addresses
   const uint32_t kl = k_lane(kb, col, half), vl = v_lane(vb, lane);  // this lane's operands
-  const auto first_of = [&](int n) { return exact_first<BLK>(tl, n - nplain); };
+  // Pipelined tile n: pooled tiles, then the full exact tiles.
+  const auto first_of = [&](int n) { return exact_first<BLK>(tl, n - npool); };
   const auto issue_k_at = [&](int first) {
     issue_full<NTHREADS>(kb, src.k + static_cast<int64_t>(first) * src.sk, src.sk, off.k);
   };
   const auto issue_v_at = [&](int first) {
     issue_full<NTHREADS>(vb, src.v + static_cast<int64_t>(first) * src.sv, src.sv, off.v);
   };
-  const auto issue_k = [&](int n) { issue_k_at(first_of(n)); };
-  const auto issue_v = [&](int n) { issue_v_at(first_of(n)); };
-  const auto issue_tile = [&](int n) {
-    if (n >= nplain) {
-      issue_k(n);
-      issue_v(n);
+  const auto issue_pipe = [&](int n, int kv) {
+    if (n >= npool) {
+      if (kv == 0) issue_k_at(first_of(n)); else issue_v_at(first_of(n));
     } else {
-      const TileDesc td = desc<BLK>(tl, n, nrag, T, NT);
-      issue_generic<NTHREADS>(kb, 0, td, src);
-      issue_generic<NTHREADS>(vb, 1, td, src);
+      issue_generic<NTHREADS>(kv == 0 ? kb : vb, kv, pooled_desc(tl, n, NT), src);
     }
   };
-  issue_tile(0);
+  const auto plain_desc = [&] {
+    return rag ? exact_desc<BLK>(tl, tl.nexact - 1, T, NT) : pooled_desc(tl, tl.npool - 1, NT);
+  };
+  if (nplain) {
+    issue_generic<NTHREADS>(kb, 0, plain_desc(), src);
+    issue_generic<NTHREADS>(vb, 1, plain_desc(), src);
+  } else {
+    issue_pipe(0, 0);
+    issue_pipe(0, 1);
+  }
 
-  // This wave's 32 query rows as the B operand of S^T = K Q^T.
+  // This wave's 32 query rows as the B operand of S^T = K Q^T (rows past T
+  // repeat row T - 1 and are not stored).
   const int qrow = qb * BLK + wave * 32 + col;
   bf16x8 qreg[8];
   {
-    const uint16_t* qp = q + b * sq_b + static_cast<int64_t>(qrow) * sq_t + h * sq_h + half * 8;
+    const uint16_t* qp = q + b * sq_b + static_cast<int64_t>(min(qrow, T - 1)) * sq_t + h * sq_h + half * 8;
 #pragma unroll
-    for (int cc = 0; cc < 8; ++cc) {
-      uint4 r = make_uint4(0u, 0u, 0u, 0u);
-      if (qrow < T) r = *reinterpret_cast<const uint4*>(qp + cc * 16);
-      qreg[cc] = __builtin_bit_cast(bf16x8, r);
-    }
+    for (int cc = 0; cc < 8; ++cc)
+      qreg[cc] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + cc * 16));
   }
 
   SoftmaxState st;
   st.init();
 
-  // ---- plain tiles (pooled, ragged). The next tile's K is copied once
-  // every wave has its scores (it lands during the softmax and P.V), its V
-  // once every wave is done with P.V (it lands during the next QK).
-  const auto issue_tile_kv = [&](int n, int kv) {
-    if (n >= nplain) {
-      if (kv == 0) issue_k(n); else issue_v(n);
-    } else {
-      issue_generic<NTHREADS>(kv == 0 ? kb : vb, kv, desc<BLK>(tl, n, nrag, T, NT), src);
-    }
-  };
-  for (int n = 0; n < nplain; ++n) {
-    wait_vmcnt<CopyOffsets<NTHREADS>::U>();  // K(n); V(n) may be in flight
+  // ---- the short last block's tile. The first pipelined K is copied once
+  // every wave has its scores (it lands during the softmax and P.V), its V once
+  // every wave is done with P.V (it lands during the next QK).
+  if (nplain) {
+    wait_tile_copies();
     __syncthreads();
     f32x16 s[2];
     qk_tile(kl, qreg, s);
-    wait_tile_copies();  // V(n)
-    __syncthreads();     // every wave is done with K(n)
-    if (n + 1 < ntiles) issue_tile_kv(n + 1, 0);
-    finish_tile<BLK>(st, s, vl, desc<BLK>(tl, n, nrag, T, NT), c, lane, NT, T);
-    __syncthreads();     // every wave is done with V(n)
-    if (n + 1 < ntiles) issue_tile_kv(n + 1, 1);
+    __syncthreads();  // every wave is done with K
+    if (npipe > 0) issue_pipe(0, 0);
+    finish_tile<BLK>(st, s, vl, plain_desc(), c, lane, NT, T);
+    __syncthreads();  // every wave is done with V
+    if (npipe > 0) issue_pipe(0, 1);
   }
 
-  // ---- full exact tiles, pipelined; tile F was issued. K(n+2) past the last
-  // tile is clamped to it: a redundant copy that nothing reads afterwards,
-  // which keeps the loop free of branches.
-  const int F = nplain;
-  if (F < ntiles) {
+  // ---- pooled and full exact tiles, pipelined; tile 0 was issued. K(n+2) past
+  // the last tile is clamped to it: a redundant copy that nothing reads
+  // afterwards, which keeps the exact loop free of branches.
+  if (npipe > 0) {
     f32x16 sa[2], sb[2];
-    int n = F;
+    int n = 0;
     wait_tile_copies();
     __syncthreads();
     qk_tile(kl, qreg, sa);
-    mfma_fence(sa);   // the step's softmax reads S(F) through asm
+    mfma_fence(sa);   // the step's softmax reads S(0) through asm
     __syncthreads();  // kbuf is free
-    if (F + 1 < ntiles) issue_k(F + 1);
+    if (1 < npipe) issue_pipe(1, 0);
     wait_tile_copies();
-    __syncthreads();  // K(F+1) and V(F) in LDS
-    // Step n computes S(n+1) and needs n + 1 < ntiles. On entry kbuf holds
-    // K(n+1), vbuf V(n) (copy possibly in flight). The first token rows of
-    // the step's two copies were read from the LDS list in the step before
-    // (kf, vf), so no copy waits on an LDS read.
-    int kf = first_of(min(n + 2, ntiles - 1)), vf = first_of(n + 1);
-    const auto step = [&](f32x16 (&sc)[2], f32x16 (&sn)[2]) {
-      fast_step(st, sc, sn, kl, vl, qreg, c, lane, [&] {
+    __syncthreads();  // K(1) and V(0) in LDS
+    // Step n computes S(n+1) and needs n + 1 < npipe. On entry kbuf holds
+    // K(n+1), vbuf V(n) (copy possibly in flight).
+    while (n < npool && n + 1 < npipe) {
+      mask_scores(sa, tl.pmask[n]);
+      fast_step<BLK, true>(st, sa, sb, kl, vl, qreg, c, lane, [&] {
         wait_tile_copies();  // V(n)
         __syncthreads();     // every wave is done with K(n+1)
-        issue_k_at(kf);      // K(min(n + 2, ntiles - 1))
+        issue_pipe(min(n + 2, npipe - 1), 0);
       });
-      asm volatile("" ::: "memory");  // the list reads stay behind the MFMA stream
-      const int kf_next = first_of(min(n + 3, ntiles - 1));
-      const int vf_next = first_of(min(n + 2, ntiles - 1));
+      asm volatile("" ::: "memory");
       wait_tile_copies();  // K(n+2)
       __syncthreads();     // every wave is done with V(n)
-      issue_v_at(vf);      // V(n + 1)
-      kf = kf_next;
-      vf = vf_next;
+      issue_pipe(n + 1, 1);
+      sa[0] = sb[0];
+      sa[1] = sb[1];
       ++n;
-    };
-    // Pairs of steps, so the S buffers swap roles without register copies.
-    while (n + 2 < ntiles) {
-      step(sa, sb);
-      step(sb, sa);
     }
+    if (n >= npool) {
+      // The first token rows of an exact step's two copies are read from the
+      // LDS list in the step before (kf, vf), so no copy waits on an LDS read.
+      int kf = first_of(min(n + 2, npipe - 1)), vf = first_of(min(n + 1, npipe - 1));
+      const auto step = [&](f32x16 (&sc)[2], f32x16 (&sn)[2]) {
+        fast_step<BLK, false>(st, sc, sn, kl, vl, qreg, c, lane, [&] {
+          wait_tile_copies();  // V(n)
+          __syncthreads();     // every wave is done with K(n+1)
+          issue_k_at(kf);      // K(min(n + 2, npipe - 1))
+        });
+        asm volatile("" ::: "memory");  // the list reads stay behind the MFMA stream
+        const int kf_next = first_of(min(n + 3, npipe - 1));
+        const int vf_next = first_of(min(n + 2, npipe - 1));
+        wait_tile_copies();  // K(n+2)
+        __syncthreads();     // every wave is done with V(n)
+        issue_v_at(vf);      // V(n + 1)
+        kf = kf_next;
+        vf = vf_next;
+        ++n;
+      };
+      // Pairs of steps, so the S buffers swap roles without register copies.
+      while (n + 2 < npipe) {
+        step(sa, sb);
+        step(sb, sa);
+      }
+      if (n + 1 < npipe) {
+        step(sa, sb);
+        sa[0] = sb[0];
+        sa[1] = sb[1];
+      }
+    }
+    wait_tile_copies();
+    __syncthreads();
+    mfma_fence(st.acc);  // O from the asm MFMAs, read by the plain path
+    // the last tile: exact, or pooled for a mask row without a full exact block
     const TileDesc full{0, 0, kKeys, ~0ull};
-    if (n + 1 < ntiles) {
-      step(sa, sb);
-      wait_tile_copies();
-      __syncthreads();
-      mfma_fence(st.acc);  // O from the asm MFMAs, read by the plain path
-      finish_tile<BLK>(st, sb, vl, full, c, lane, NT, T);
-    } else {
-      wait_tile_copies();
-      __syncthreads();
-      mfma_fence(st.acc);
-      finish_tile<BLK>(st, sa, vl, full, c, lane, NT, T);
-    }
+    finish_tile<BLK>(st, sa, vl, n < npool ? pooled_desc(tl, n, NT) : full, c, lane, NT, T);
   }
   wait_tile_copies();
 

@@ -509,6 +509,25 @@ __device__ __forceinline__ uint32_t exp_pair(float s0, float s1, float c, float 
       : "v"(s0), "v"(s1), "v"(c), "v"(neg), "s"(0x3F803F80u));
   return p;
 }
+// The same with the fp32 p added to the sum (pooled keys, whose row sum is
+// weighted by the block length).
+__device__ __forceinline__ uint32_t exp_pair_f32sum(float s0, float s1, float c, float neg,
+                                                    float& sum) {
+  uint32_t p;
+  float t0, t1;
+  asm volatile(
+      "v_fma_f32 %2, %4, %6, %7\n\t"
+      "v_fma_f32 %3, %5, %6, %7\n\t"
+      "v_exp_f32 %2, %2\n\t"
+      "v_exp_f32 %3, %3\n\t"
+      "s_nop 0\n\t"
+      "v_cvt_pk_bf16_f32 %0, %2, %3\n\t"
+      "v_add_f32 %1, %1, %2\n\t"
+      "v_add_f32 %1, %1, %3"
+      : "=&v"(p), "+v"(sum), "=&v"(t0), "=&v"(t1)
+      : "v"(s0), "v"(s1), "v"(c), "v"(neg));
+  return p;
+}
 // ------------------------------------------------------------ online softmax
 struct SoftmaxState {
   float m;          // running max, in the exp2 domain (score * c)
@@ -570,6 +589,26 @@ __device__ __forceinline__ void rescale(SoftmaxState& st, float alpha) {
   }
 }
 
+// Scores of the tile's keys outside amask (wave-uniform) become -inf. The two
+// lane halves hold different keys, so each element's keep bits are spread to a
+// lane mask by scalar instructions, leaving one v_cndmask per element.
+__device__ __forceinline__ void mask_scores(f32x16 (&s)[2], uint64_t amask) {
+  if (amask == ~0ull) return;
+  const uint32_t w[2] = {  // read from LDS by every lane: make it scalar
+      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(amask))),
+      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(amask >> 32)))};
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int k0 = 8 * (r >> 2) + (r & 3);  // the key (of 32) of lanes 0-31; lanes 32-63: k0 + 4
+      const uint32_t lo = static_cast<uint32_t>(static_cast<int32_t>(w[m] << (31 - k0)) >> 31);
+      const uint32_t hi = static_cast<uint32_t>(static_cast<int32_t>(w[m] << (27 - k0)) >> 31);
+      const uint64_t keep = (static_cast<uint64_t>(hi) << 32) | lo;
+      s[m][r] = __builtin_amdgcn_inverse_ballot_w64(keep) ? s[m][r] : -INFINITY;
+    }
+}
+
 // Softmax and P.V of one bf16 tile whose scores are in s (the plain path:
 // pooled, ragged and last tiles). Masked keys get -inf; pooled keys weigh
 // len_j in the row sum (/root/reference/_tri_fwd.py:302-307); P is rounded to
@@ -581,15 +620,7 @@ template <int BLK, typename VTile>
 __device__ __forceinline__ void finish_tile(SoftmaxState& st, f32x16 (&s)[2], VTile vt,
                                             const TileDesc& td, float c, int lane, int NT, int T) {
   const int half = lane >> 5;
-  if (td.amask != ~0ull) {
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const uint32_t bits = static_cast<uint32_t>(td.amask >> (32 * m + 4 * half));
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        s[m][r] = ((bits >> (8 * (r >> 2) + (r & 3))) & 1u) ? s[m][r] : -INFINITY;
-    }
-  }
+  mask_scores(s, td.amask);
   float mx = -INFINITY;
 #pragma unroll
   for (int m = 0; m < 2; ++m)
@@ -601,17 +632,26 @@ __device__ __forceinline__ void finish_tile(SoftmaxState& st, f32x16 (&s)[2], VT
   bf16x8 pb[4];
   float psum = 0.f;
   if (td.pooled) {
-    const int kl_last = NT - 1 - td.first;
-    const float tail = static_cast<float>(T - (NT - 1) * BLK);
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int kl = 32 * m + 8 * (r >> 2) + 4 * half + (r & 3);
         const float p = __builtin_amdgcn_exp2f(fmaf(s[m][r], c, neg));
         pb[2 * m + (r >> 3)][r & 7] = static_cast<__bf16>(p);
-        psum = fmaf(p, kl == kl_last ? tail : static_cast<float>(BLK), psum);
+        psum += p;
+        s[m][r] = p;
       }
+    psum *= static_cast<float>(BLK);
+    const int kl_last = NT - 1 - td.first;  // a short last block weighs its own length
+    const int tail = T - (NT - 1) * BLK;
+    if (tail != BLK && kl_last < kKeys) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * m + 8 * (r >> 2) + 4 * half + (r & 3) == kl_last)
+            psum = fmaf(s[m][r], static_cast<float>(tail - BLK), psum);
+    }
   } else {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {

@@ -8,15 +8,14 @@
 //                 (/root/reference/_tri_fwd.py:288-308);
 //   exact tiles   64 tokens of an exact block (/root/reference/_tri_fwd.py:310-340).
 // All tiles feed one online softmax per query row, which is exact under any
-// tile order (up to fp32 rounding). The full exact tiles run through a
-// software pipeline, the pooled tiles and the ragged last exact tile through a
-// plain path:
+// tile order (up to fp32 rounding). The full exact tiles (block 64: the pooled
+// tiles too) run through a software pipeline, the others through a plain path:
 //   block 128 (fwd_bf16_kernel): K and V double buffered, two workgroups per
 //     CU; exact tiles first, three-stage step n = S(n+1) = K(n+1) Q^T, O +=
 //     P(n-1) V(n-1) and the softmax of S(n) in one instruction stream;
-//   block 64 (fwd_bf16_sbuf_kernel): K and V single buffered, four workgroups
-//     per CU; plain tiles first, two-stage step n = S(n+1) with the softmax of
-//     tile n interleaved, then O += P(n) V(n).
+//   block 64 (fwd_bf16_sbuf_kernel): K and V as two half tiles of 32 keys, four
+//     workgroups per CU; the short last block's tile first, then the same
+//     three-stage step over the half tiles of pooled and exact tiles.
 // Both pipelined steps are hand-ordered: inline-asm MFMAs and softmax exp
 // pairs in a fixed interleave (fwd_common.hpp), which the compiler's own
 // schedule did not give.
@@ -33,89 +32,93 @@
 namespace solattn {
 namespace bf16fwd {
 
-// Pipelined step over full exact tile n (scores in sc): S(n+1) from the K tile
-// kn goes to sn, interleaved with the softmax of tile n; `mid` runs before
-// P(n) . V(n).
-// kl, vl: this lane's operand addresses (k_lane, v_lane) in K(n+1) and V(n).
-// Hand-ordered as step3 below: each score MFMA is followed by the exps of
-// one P word, the operands are read two MFMAs ahead, and the lazy tile max
-// works the same way (also catching the first exact tile when no plain tile
-// came before it: running max -inf, p = inf).
-// POOLED: tile n is a pooled tile of whole blocks (its masked scores -inf):
-// each key weighs BLK in the row sum, which adds the fp32 p.
-template <int BLK, bool POOLED, typename Mid>
-__device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32x16 (&sn)[2],
-                                          uint32_t kl, uint32_t vl, const bf16x8 (&q)[8],
-                                          float c, int lane, Mid&& mid) {
-  bf16x8 ka[3], va[3], pb[4];
-  uint32_t pw[4][4];
+// Three-stage step of the block-64 forward over half tiles of 32 keys: S(n+1) =
+// K(n+1) Q^T (8 MFMAs), O += P(n-1) V(n-1) (8 MFMAs) and the softmax of S(n)
+// (8 pairs of exps) in one hand-ordered stream, as step3 below: slot i issues
+// score MFMA i, the exps of P(n) word i, then P.V MFMA i, each operand read two
+// slots ahead; the tile max is lazy and the O rescale follows the products.
+// QK = false drops the score product (the last half tile), PV = false the value
+// product (the first). POOLED: the keys of n are pooled keys of whole blocks
+// (masked scores -inf), each weighing BLK in the row sum, which adds the fp32 p.
+// kl, vl: this lane's operand addresses in K(n+1) and V(n-1).
+template <int BLK, bool POOLED, bool QK, bool PV>
+__device__ __forceinline__ void half_step(SoftmaxState& st, const f32x16& sc, f32x16& sn,
+                                          const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
+                                          uint32_t vl, const bf16x8 (&q)[8], float c) {
+  static_assert(kMaxSlack >= 8.f, "the lazy test relies on 255 < 2^kMaxSlack");
+  bf16x8 ka[3], va[3];
+  uint32_t pw[2][4];
   float psum = 0.f;
   const float neg = -st.m;
-  ka[0] = k_op_x(kl, 0, 0);
-  ka[1] = k_op_x(kl, 1, 0);
+  if constexpr (QK) {
+    ka[0] = k_op_x(kl, 0, 0);
+    ka[1] = k_op_x(kl, 0, 1);
+  }
+  if constexpr (PV) {
+    va[0] = v_op_x(vl, 0, 0);
+    va[1] = v_op_x(vl, 0, 1);
+  }
   asm volatile("" ::: "memory");
+  const auto unit = [&](int i) {
+    pw[i >> 2][i & 3] = POOLED ? exp_pair_f32sum(sc[2 * i], sc[2 * i + 1], c, neg, psum)
+                               : exp_pair(sc[2 * i], sc[2 * i + 1], c, neg, psum);
+  };
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + 2 < 16) {
-      ka[(i + 2) % 3] = k_op_x(kl, (i + 2) & 1, (i + 2) >> 1);
+  for (int i = 0; i < 8; ++i) {
+    if (i + 2 < 8) {
+      if constexpr (QK) ka[(i + 2) % 3] = k_op_x(kl, 0, i + 2);
+      if constexpr (PV) va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
       asm volatile("" ::: "memory");
     }
-    if (i < 2)
-      mfma_v0(sn[i & 1], ka[i % 3], q[i >> 1]);
-    else
-      mfma_v(sn[i & 1], ka[i % 3], q[i >> 1]);
-    const int ks = i >> 2, w = i & 3;
-    const int r = 8 * (ks & 1) + 2 * w;
-    pw[ks][w] = POOLED ? exp_pair_f32sum(sc[ks >> 1][r], sc[ks >> 1][r + 1], c, neg, psum)
-                       : exp_pair(sc[ks >> 1][r], sc[ks >> 1][r + 1], c, neg, psum);
+    if constexpr (QK) {
+      if (i == 0)
+        mfma_v0(sn, ka[0], q[0]);
+      else
+        mfma_v(sn, ka[i % 3], q[i]);
+      unit(i);
+    }
+    if constexpr (PV) {
+      if (i == 0)
+        mfma_v_first(st.acc[0], va[0], pp[0]);
+      else if (QK && i == 7)
+        mfma_v_tie(st.acc[3], va[1], pp[1], sn);  // va[7 % 3]
+      else
+        mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
+    }
+    if constexpr (!QK) unit(i);
+    if (i == 0) __builtin_amdgcn_s_setprio(1);
   }
+  __builtin_amdgcn_s_setprio(0);
+  if constexpr (QK && !PV) mfma_fence(sn);
+  if constexpr (!QK) mfma_fence(st.acc);
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    pb[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
+  for (int ks = 0; ks < 2; ++ks)
+    pn[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
   float alpha = 1.f;
   if (__any(!(psum <= 255.f))) {  // (also catches inf / NaN)
     float mx = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
     const float m_new = new_max(st.m, xhalf_max(mx) * c, alpha);
     if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
       st.m = m_new;
       psum = 0.f;
       if constexpr (POOLED) {
 #pragma unroll
-        for (int r = 0; r < 32; ++r) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r >> 4][r & 15], c, -m_new));
-          pb[r >> 3][r & 7] = static_cast<__bf16>(p);
+        for (int r = 0; r < 16; ++r) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r], c, -m_new));
+          pn[r >> 3][r & 7] = static_cast<__bf16>(p);
           psum += p;
         }
       } else {
-        psum = exp8<0>(sc[0], c, -m_new, pb[0], psum);
-        psum = exp8<8>(sc[0], c, -m_new, pb[1], psum);
-        psum = exp8<0>(sc[1], c, -m_new, pb[2], psum);
-        psum = exp8<8>(sc[1], c, -m_new, pb[3], psum);
+        psum = exp8<0>(sc, c, -m_new, pn[0], psum);
+        psum = exp8<8>(sc, c, -m_new, pn[1], psum);
       }
-      mfma_fence(st.acc);  // the rescale reads O
+      if constexpr (PV) mfma_fence(st.acc);  // the rescale reads O
       rescale(st, alpha);
     }
   }
   st.l = fmaf(st.l, alpha, POOLED ? psum * static_cast<float>(BLK) : psum);
-  mid();
-  va[0] = v_op_x(vl, 0, 0);
-  va[1] = v_op_x(vl, 0, 1);
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + 2 < 16) {
-      va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
-      asm volatile("" ::: "memory");
-    }
-    if (i == 0)
-      mfma_v_first(st.acc[0], va[0], pb[0]);
-    else if (i == 15)
-      mfma_v_tie(st.acc[3], va[0], pb[3], sn);  // va[15 % 3]
-    else
-      mfma_v(st.acc[i & 3], va[i % 3], pb[i >> 2]);
-  }
 }
 
 // Three-stage step: S(n+1) = K(n+1) Q^T, O += P(n-1) V(n-1) and the softmax of
@@ -219,15 +222,22 @@ __device__ __forceinline__ void step3(SoftmaxState& st, const f32x16 (&sc)[2], f
   st.l = fmaf(st.l, alpha, psum);
 }
 
-// Block 64 forward (workgroups of 2 waves). K and V are single buffered
-// (32 KiB), so four workgroups and two waves per SIMD fit a CU; the pipeline
-// step waits twice (K refilled after the QK phase, V after P.V). Tile order:
-// with T not a multiple of 64, the tile of the short last block through the
-// plain path (as a ragged exact tile, or inside its pooled tile, where it
+// Block 64 forward (workgroups of 2 waves). K and V hold two half tiles of 32
+// keys each (32 KiB), so four workgroups and two waves per SIMD fit a CU. Tile
+// order: with T not a multiple of 64, the tile of the short last block through
+// the plain path (as a ragged exact tile, or inside its pooled tile, where it
 // weighs its own length); then the pooled and the full exact tiles through the
-// pipeline. (Pooled tiles on the plain path, each with its own waits and no
-// overlap, took 4.1 us against 1.7 us of a pipelined exact tile: 15% of a
-// workgroup's time at 32760 tokens.)
+// pipeline, two half steps a tile.
+//
+// Bound: at 32760 tokens the tile copies (without them, results wrong by
+// construction, the two-stage form of this kernel ran 19% faster; with all of
+// them hitting L2, 8%), then the MFMAs at the power-limited clock; at 4096
+// tokens (1.5 workgroups a slot) the workgroup's own latency. Half tiles
+// against the two-stage step over whole tiles (K copied behind 16 bare P.V
+// MFMAs, V behind QK and the exps): every copy gets a whole step, the MFMAs of
+// both products hide the exps, and the scores take 32 registers less. Calls:
+// 32760 tokens 2835 -> 2737 us, 12133 packed 623 -> 606, 4096 91.2 -> 87.4,
+// 9180 with 64-channel heads 247.5 -> 239.5.
 template <int BLK>
 __global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))
 fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
@@ -262,20 +272,28 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
   off.init(sk_t, sv_t);
   const uint32_t kb = lds_addr(kbuf), vb = lds_addr(vbuf);  // LDS byte addresses
   const uint32_t kl = k_lane(kb, col, half), vl = v_lane(vb, lane);  // this lane's operands
-  // Pipelined tile n: pooled tiles, then the full exact tiles.
-  const auto first_of = [&](int n) { return exact_first<BLK>(tl, n - npool); };
-  const auto issue_k_at = [&](int first) {
-    issue_full<NTHREADS>(kb, src.k + static_cast<int64_t>(first) * src.sk, src.sk, off.k);
+  // Half hh of pipelined tile t (pooled tiles, then the full exact tiles) into
+  // K or V half buffer hh.
+  const auto first_of = [&](int t) { return exact_first<BLK>(tl, max(t - npool, 0)); };
+  const auto issue_k_at = [&](int first, int hh) {
+    issue_half<NTHREADS>(kb + hh * kHalfBytes, src.k + static_cast<int64_t>(first + 32 * hh) * src.sk,
+                         src.sk, off.k);
   };
-  const auto issue_v_at = [&](int first) {
-    issue_full<NTHREADS>(vb, src.v + static_cast<int64_t>(first) * src.sv, src.sv, off.v);
+  const auto issue_v_at = [&](int first, int hh) {
+    issue_half<NTHREADS>(vb + hh * kHalfBytes, src.v + static_cast<int64_t>(first + 32 * hh) * src.sv,
+                         src.sv, off.v);
   };
-  const auto issue_pipe = [&](int n, int kv) {
-    if (n >= npool) {
-      if (kv == 0) issue_k_at(first_of(n)); else issue_v_at(first_of(n));
+  const auto issue_any = [&](int t, int kv, int hh) {
+    if (t >= npool) {
+      if (kv == 0) issue_k_at(first_of(t), hh); else issue_v_at(first_of(t), hh);
     } else {
-      issue_generic<NTHREADS>(kv == 0 ? kb : vb, kv, pooled_desc(tl, n, NT), src);
+      issue_generic_half<NTHREADS>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, t, NT), hh, src);
     }
+  };
+  const auto issue_start = [&] {  // what the first half steps need
+    issue_any(0, 0, 0);
+    issue_any(0, 0, 1);
+    issue_any(0, 1, 0);
   };
   const auto plain_desc = [&] {
     return rag ? exact_desc<BLK>(tl, tl.nexact - 1, T, NT) : pooled_desc(tl, tl.npool - 1, NT);
@@ -284,8 +302,7 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
     issue_generic<NTHREADS>(kb, 0, plain_desc(), src);
     issue_generic<NTHREADS>(vb, 1, plain_desc(), src);
   } else {
-    issue_pipe(0, 0);
-    issue_pipe(0, 1);
+    issue_start();
   }
 
   // This wave's 32 query rows as the B operand of S^T = K Q^T (rows past T
@@ -302,89 +319,99 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
   SoftmaxState st;
   st.init();
 
-  // ---- the short last block's tile. The first pipelined K is copied once
-  // every wave has its scores (it lands during the softmax and P.V), its V once
-  // every wave is done with P.V (it lands during the next QK).
+  // ---- the short last block's tile
   if (nplain) {
     wait_tile_copies();
     __syncthreads();
     f32x16 s[2];
     qk_tile(kl, qreg, s);
-    __syncthreads();  // every wave is done with K
-    if (npipe > 0) issue_pipe(0, 0);
     finish_tile<BLK>(st, s, vl, plain_desc(), c, lane, NT, T);
-    __syncthreads();  // every wave is done with V
-    if (npipe > 0) issue_pipe(0, 1);
+    __syncthreads();  // every wave is done with K and V
+    if (npipe > 0) issue_start();
   }
 
-  // ---- pooled and full exact tiles, pipelined; tile 0 was issued. K(n+2) past
-  // the last tile is clamped to it: a redundant copy that nothing reads
-  // afterwards, which keeps the exact loop free of branches.
+  // ---- pooled and full exact tiles, pipelined by half tiles n = 2t, 2t + 1. On
+  // entry to step n: S(n) and P(n-1) in registers, K(n+1) and V(n-1) in LDS; the
+  // step copies K(n+2) over K(n) and V(n) over V(n-2), so a copy has a whole step
+  // to land. K of the tile past the last is clamped to it: a redundant copy that
+  // nothing reads.
   if (npipe > 0) {
-    f32x16 sa[2], sb[2];
-    int n = 0;
+    f32x16 sa, sb;
+    bf16x8 pa[2], pb[2];
     wait_tile_copies();
     __syncthreads();
-    qk_tile(kl, qreg, sa);
-    mfma_fence(sa);   // the step's softmax reads S(0) through asm
-    __syncthreads();  // kbuf is free
-    if (1 < npipe) issue_pipe(1, 0);
-    wait_tile_copies();
-    __syncthreads();  // K(1) and V(0) in LDS
-    // Step n computes S(n+1) and needs n + 1 < npipe. On entry kbuf holds
-    // K(n+1), vbuf V(n) (copy possibly in flight).
-    while (n < npool && n + 1 < npipe) {
-      mask_scores(sa, tl.pmask[n]);
-      fast_step<BLK, true>(st, sa, sb, kl, vl, qreg, c, lane, [&] {
-        wait_tile_copies();  // V(n)
-        __syncthreads();     // every wave is done with K(n+1)
-        issue_pipe(min(n + 2, npipe - 1), 0);
-      });
-      asm volatile("" ::: "memory");
-      wait_tile_copies();  // K(n+2)
-      __syncthreads();     // every wave is done with V(n)
-      issue_pipe(n + 1, 1);
-      sa[0] = sb[0];
-      sa[1] = sb[1];
-      ++n;
+    {
+      const f32x16 zero = {};
+#pragma unroll
+      for (int cc = 0; cc < 8; ++cc) sa = mfma_bf16(k_op_x(kl, 0, cc), qreg[cc], cc == 0 ? zero : sa);
     }
-    if (n >= npool) {
-      // The first token rows of an exact step's two copies are read from the
-      // LDS list in the step before (kf, vf), so no copy waits on an LDS read.
-      int kf = first_of(min(n + 2, npipe - 1)), vf = first_of(min(n + 1, npipe - 1));
-      const auto step = [&](f32x16 (&sc)[2], f32x16 (&sn)[2]) {
-        fast_step<BLK, false>(st, sc, sn, kl, vl, qreg, c, lane, [&] {
-          wait_tile_copies();  // V(n)
-          __syncthreads();     // every wave is done with K(n+1)
-          issue_k_at(kf);      // K(min(n + 2, npipe - 1))
-        });
-        asm volatile("" ::: "memory");  // the list reads stay behind the MFMA stream
-        const int kf_next = first_of(min(n + 3, npipe - 1));
-        const int vf_next = first_of(min(n + 2, npipe - 1));
-        wait_tile_copies();  // K(n+2)
-        __syncthreads();     // every wave is done with V(n)
-        issue_v_at(vf);      // V(n + 1)
-        kf = kf_next;
-        vf = vf_next;
-        ++n;
-      };
-      // Pairs of steps, so the S buffers swap roles without register copies.
-      while (n + 2 < npipe) {
-        step(sa, sb);
-        step(sb, sa);
-      }
-      if (n + 1 < npipe) {
-        step(sa, sb);
-        sa[0] = sb[0];
-        sa[1] = sb[1];
+    mfma_fence(sa);   // the steps read the scores through asm
+    __syncthreads();  // every wave is done with K(0)
+    const uint32_t kl1 = kl + kHalfBytes, vl1 = vl + kHalfBytes;
+    const int last = npipe - 1;
+    int t = 0;
+    const auto land = [&] {
+      wait_tile_copies();
+      __syncthreads();
+    };
+    // half steps 0 (its V came with the first copies) and 1
+    if (npool > 0) {
+      issue_any(min(1, last), 0, 0);
+      mask_scores(sa, static_cast<uint32_t>(tl.pmask[0]));
+      half_step<BLK, true, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
+      land();
+      issue_any(min(1, last), 0, 1);
+      issue_any(0, 1, 1);
+      mask_scores(sb, static_cast<uint32_t>(tl.pmask[0] >> 32));
+      half_step<BLK, true, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      land();
+      for (t = 1; t < npool; ++t) {
+        issue_any(min(t + 1, last), 0, 0);
+        issue_any(t, 1, 0);
+        mask_scores(sa, static_cast<uint32_t>(tl.pmask[t]));
+        half_step<BLK, true, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
+        land();
+        issue_any(min(t + 1, last), 0, 1);
+        issue_any(t, 1, 1);
+        mask_scores(sb, static_cast<uint32_t>(tl.pmask[t] >> 32));
+        half_step<BLK, true, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+        land();
       }
     }
-    wait_tile_copies();
-    __syncthreads();
-    mfma_fence(st.acc);  // O from the asm MFMAs, read by the plain path
-    // the last tile: exact, or pooled for a mask row without a full exact block
-    const TileDesc full{0, 0, kKeys, ~0ull};
-    finish_tile<BLK>(st, sa, vl, n < npool ? pooled_desc(tl, n, NT) : full, c, lane, NT, T);
+    // The first token rows of tiles t and t + 1 are read from the LDS list an
+    // iteration ahead, so no copy waits on an LDS read.
+    int f0 = first_of(min(t, last)), f1 = first_of(min(t + 1, last));
+    if (npool == 0) {
+      issue_k_at(f1, 0);
+      half_step<BLK, false, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
+      land();
+      issue_k_at(f1, 1);
+      issue_v_at(f0, 1);
+      half_step<BLK, false, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      f0 = f1;
+      f1 = first_of(min(2, last));
+      land();
+      t = 1;
+    }
+    for (; t < npipe; ++t) {
+      issue_k_at(f1, 0);
+      issue_v_at(f0, 0);
+      half_step<BLK, false, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
+      asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
+      const int f2 = first_of(min(t + 2, last));
+      land();
+      issue_k_at(f1, 1);
+      issue_v_at(f0, 1);
+      half_step<BLK, false, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      land();
+      f0 = f1;
+      f1 = f2;
+    }
+    // P.V of the last half tile
+    mfma_fence(st.acc);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      st.acc[i & 3] = mfma_bf16(v_op_x(vl1, i >> 2, i & 3), pb[i >> 2], st.acc[i & 3]);
   }
   wait_tile_copies();
 

@@ -332,6 +332,38 @@ __device__ __forceinline__ void issue_full(uint32_t dst, const uint16_t* base, i
   }
 }
 
+// The same for half a tile (32 keys): rows [32 hh, 32 hh + 32) of the tile `td`
+// (issue_generic_half) or a base at the half's first row (issue_half).
+constexpr uint32_t kHalfBytes = kTileBytes / 2;
+template <int NTHREADS>
+__device__ __forceinline__ void issue_generic_half(uint32_t dst, int kv, const TileDesc& td, int hh,
+                                                   const KVSource& src) {
+  constexpr int U = CopyOffsets<NTHREADS>::U / 2;
+  const uint32_t l0 = dst + wave_id() * 64 * 16;
+  const uint16_t* b = kv == 0 ? (td.pooled ? src.kc : src.k) : (td.pooled ? src.vc : src.v);
+  const int64_t stride = td.pooled ? src.skc : (kv == 0 ? src.sk : src.sv);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int e = threadIdx.x + NTHREADS * u;
+    const int row = 32 * hh + (e >> 4), pc = e & 15;
+    const int srow = td.first + (row < td.nvalid ? row : 0);
+    const int chunk = kv == 0 ? swz_k(row, pc) : swz_v(row, pc);
+    g2l16(b + static_cast<int64_t>(srow) * stride + chunk * 8, l0 + NTHREADS * u * 16);
+  }
+}
+template <int NTHREADS>
+__device__ __forceinline__ void issue_half(uint32_t dst, const uint16_t* base, int64_t stride,
+                                           const uint32_t (&off)[CopyOffsets<NTHREADS>::P]) {
+  using CO = CopyOffsets<NTHREADS>;
+  const uint32_t l0 = dst + wave_id() * 64 * 16;
+  const char* b = reinterpret_cast<const char*>(base);
+#pragma unroll
+  for (int u = 0; u < CO::U / 2; ++u) {
+    const char* row_base = b + static_cast<int64_t>(u / CO::P) * 16 * stride * 2;
+    g2l16_s(row_base, off[u % CO::P], l0 + NTHREADS * u * 16);
+  }
+}
+
 // ------------------------------------------------------------ bf16 MFMA tiles
 __device__ __forceinline__ f32x16 mfma_bf16(const bf16x8& a, const bf16x8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -479,7 +511,15 @@ __device__ __forceinline__ void mfma_v_tie(f32x16& d, const bf16x8& a, const bf1
                : "+v"(d), "+v"(s[0]), "+v"(s[1])
                : "v"(a), "v"(b));
 }
+__device__ __forceinline__ void mfma_v_tie(f32x16& d, const bf16x8& a, const bf16x8& b, f32x16& s) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\ts_nop 3"
+               : "+v"(d), "+v"(s)
+               : "v"(a), "v"(b));
+}
 // 16 wait states after the MFMAs that wrote x; readers of x come after it.
+__device__ __forceinline__ void mfma_fence(f32x16& x) {
+  asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x));
+}
 template <int N>
 __device__ __forceinline__ void mfma_fence(f32x16 (&x)[N]) {
   static_assert(N == 2 || N == 4, "fence sizes");
@@ -592,21 +632,22 @@ __device__ __forceinline__ void rescale(SoftmaxState& st, float alpha) {
 // Scores of the tile's keys outside amask (wave-uniform) become -inf. The two
 // lane halves hold different keys, so each element's keep bits are spread to a
 // lane mask by scalar instructions, leaving one v_cndmask per element.
+__device__ __forceinline__ void mask_scores(f32x16& s, uint32_t keep32) {
+  const uint32_t w = static_cast<uint32_t>(  // read from LDS by every lane: make it scalar
+      __builtin_amdgcn_readfirstlane(static_cast<int>(keep32)));
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int k0 = 8 * (r >> 2) + (r & 3);  // the key (of 32) of lanes 0-31; lanes 32-63: k0 + 4
+    const uint32_t lo = static_cast<uint32_t>(static_cast<int32_t>(w << (31 - k0)) >> 31);
+    const uint32_t hi = static_cast<uint32_t>(static_cast<int32_t>(w << (27 - k0)) >> 31);
+    const uint64_t keep = (static_cast<uint64_t>(hi) << 32) | lo;
+    s[r] = __builtin_amdgcn_inverse_ballot_w64(keep) ? s[r] : -INFINITY;
+  }
+}
 __device__ __forceinline__ void mask_scores(f32x16 (&s)[2], uint64_t amask) {
   if (amask == ~0ull) return;
-  const uint32_t w[2] = {  // read from LDS by every lane: make it scalar
-      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(amask))),
-      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(amask >> 32)))};
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int k0 = 8 * (r >> 2) + (r & 3);  // the key (of 32) of lanes 0-31; lanes 32-63: k0 + 4
-      const uint32_t lo = static_cast<uint32_t>(static_cast<int32_t>(w[m] << (31 - k0)) >> 31);
-      const uint32_t hi = static_cast<uint32_t>(static_cast<int32_t>(w[m] << (27 - k0)) >> 31);
-      const uint64_t keep = (static_cast<uint64_t>(hi) << 32) | lo;
-      s[m][r] = __builtin_amdgcn_inverse_ballot_w64(keep) ? s[m][r] : -INFINITY;
-    }
+  mask_scores(s[0], static_cast<uint32_t>(amask));
+  mask_scores(s[1], static_cast<uint32_t>(amask >> 32));
 }
 
 // Softmax and P.V of one bf16 tile whose scores are in s (the plain path:

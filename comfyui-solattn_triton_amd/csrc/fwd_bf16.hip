@@ -8,17 +8,12 @@
 //                 (/root/reference/_tri_fwd.py:288-308);
 //   exact tiles   64 tokens of an exact block (/root/reference/_tri_fwd.py:310-340).
 // All tiles feed one online softmax per query row, which is exact under any
-// tile order (up to fp32 rounding). The full exact tiles (block 64: the pooled
-// tiles too) run through a software pipeline, the others through a plain path:
-//   block 128 (fwd_bf16_kernel): K and V double buffered, two workgroups per
-//     CU; exact tiles first, three-stage step n = S(n+1) = K(n+1) Q^T, O +=
-//     P(n-1) V(n-1) and the softmax of S(n) in one instruction stream;
-//   block 64 (fwd_bf16_sbuf_kernel): K and V as two half tiles of 32 keys, four
-//     workgroups per CU; the short last block's tile first, then the same
-//     three-stage step over the half tiles of pooled and exact tiles.
-// Both pipelined steps are hand-ordered: inline-asm MFMAs and softmax exp
-// pairs in a fixed interleave (fwd_common.hpp), which the compiler's own
-// schedule did not give.
+// tile order (up to fp32 rounding). The pooled and the full exact tiles run
+// through a software pipeline of half tiles (32 keys): step n computes S(n+1) =
+// K(n+1) Q^T, O += P(n-1) V(n-1) and the softmax of S(n) in one instruction
+// stream, hand-ordered from inline-asm MFMAs and softmax exp pairs
+// (fwd_common.hpp), which the compiler's own schedule did not give. The tile of
+// a short last block goes through a plain path first.
 //
 // MFMA dataflow (v_mfma_f32_32x32x16_bf16): S^T = K . Q^T puts one query row
 // per lane column, so row max / sum need one cross-lane step (lanes 32 apart,
@@ -32,16 +27,26 @@
 namespace solattn {
 namespace bf16fwd {
 
-// Three-stage step of the block-64 forward over half tiles of 32 keys: S(n+1) =
-// K(n+1) Q^T (8 MFMAs), O += P(n-1) V(n-1) (8 MFMAs) and the softmax of S(n)
-// (8 pairs of exps) in one hand-ordered stream, as step3 below: slot i issues
-// score MFMA i, the exps of P(n) word i, then P.V MFMA i, each operand read two
-// slots ahead; the tile max is lazy and the O rescale follows the products.
-// QK = false drops the score product (the last half tile), PV = false the value
-// product (the first). POOLED: the keys of n are pooled keys of whole blocks
-// (masked scores -inf), each weighing BLK in the row sum, which adds the fp32 p.
-// kl, vl: this lane's operand addresses in K(n+1) and V(n-1).
-template <int BLK, bool POOLED, bool QK, bool PV>
+// Three-stage step over half tiles of 32 keys: S(n+1) = K(n+1) Q^T (8 MFMAs),
+// O += P(n-1) V(n-1) (8 MFMAs) and the softmax of S(n) (8 pairs of exps) in one
+// hand-ordered stream: slot i issues score MFMA i, the exps of P(n) word i, then
+// P.V MFMA i; the K and V operands of slot i + 2 are read at the top of slot i
+// (the empty asm with a memory clobber keeps the reads there). O is rescaled to
+// the new running max after the P(n-1) V(n-1) products. PV = false: the first
+// half tile, which has no value product to add. POOLED: the keys of n are
+// pooled keys of whole blocks (masked scores -inf), each weighing BLK in the row
+// sum, which adds the fp32 p. kl, vl: this lane's operand addresses in K(n+1)
+// and V(n-1).
+// Lazy tile max: the exps use the running max as it stands, and the tile's max
+// is taken only when a lane's row sum exceeds 255. No sum above 255 means every
+// p <= 255, i.e. every score is below the running max + log2(255.5) <
+// kMaxSlack, so the tile would not have moved the max: the running max evolves
+// as with the max taken every step. The first tile of a workgroup (running max
+// -inf, p = inf or NaN) always takes that path.
+// Raised wave priority for the step's stream: the issue arbiter then prefers a
+// wave inside its MFMAs over one at its copies or barrier (without it, 6%
+// slower at block 64 and 32760 tokens).
+template <int BLK, bool POOLED, bool PV>
 __device__ __forceinline__ void half_step(SoftmaxState& st, const f32x16& sc, f32x16& sn,
                                           const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
                                           uint32_t vl, const bf16x8 (&q)[8], float c) {
@@ -50,47 +55,38 @@ __device__ __forceinline__ void half_step(SoftmaxState& st, const f32x16& sc, f3
   uint32_t pw[2][4];
   float psum = 0.f;
   const float neg = -st.m;
-  if constexpr (QK) {
-    ka[0] = k_op_x(kl, 0, 0);
-    ka[1] = k_op_x(kl, 0, 1);
-  }
+  ka[0] = k_op_x(kl, 0, 0);
+  ka[1] = k_op_x(kl, 0, 1);
   if constexpr (PV) {
     va[0] = v_op_x(vl, 0, 0);
     va[1] = v_op_x(vl, 0, 1);
   }
   asm volatile("" ::: "memory");
-  const auto unit = [&](int i) {
-    pw[i >> 2][i & 3] = POOLED ? exp_pair_f32sum(sc[2 * i], sc[2 * i + 1], c, neg, psum)
-                               : exp_pair(sc[2 * i], sc[2 * i + 1], c, neg, psum);
-  };
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     if (i + 2 < 8) {
-      if constexpr (QK) ka[(i + 2) % 3] = k_op_x(kl, 0, i + 2);
+      ka[(i + 2) % 3] = k_op_x(kl, 0, i + 2);
       if constexpr (PV) va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
       asm volatile("" ::: "memory");
     }
-    if constexpr (QK) {
-      if (i == 0)
-        mfma_v0(sn, ka[0], q[0]);
-      else
-        mfma_v(sn, ka[i % 3], q[i]);
-      unit(i);
-    }
+    if (i == 0)
+      mfma_v0(sn, ka[0], q[0]);
+    else
+      mfma_v(sn, ka[i % 3], q[i]);
+    pw[i >> 2][i & 3] = POOLED ? exp_pair_f32sum(sc[2 * i], sc[2 * i + 1], c, neg, psum)
+                               : exp_pair(sc[2 * i], sc[2 * i + 1], c, neg, psum);
     if constexpr (PV) {
       if (i == 0)
         mfma_v_first(st.acc[0], va[0], pp[0]);
-      else if (QK && i == 7)
+      else if (i == 7)
         mfma_v_tie(st.acc[3], va[1], pp[1], sn);  // va[7 % 3]
       else
         mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
     }
-    if constexpr (!QK) unit(i);
     if (i == 0) __builtin_amdgcn_s_setprio(1);
   }
   __builtin_amdgcn_s_setprio(0);
-  if constexpr (QK && !PV) mfma_fence(sn);
-  if constexpr (!QK) mfma_fence(st.acc);
+  if constexpr (!PV) mfma_fence(sn);
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks)
     pn[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
@@ -121,126 +117,28 @@ __device__ __forceinline__ void half_step(SoftmaxState& st, const f32x16& sc, f3
   st.l = fmaf(st.l, alpha, POOLED ? psum * static_cast<float>(BLK) : psum);
 }
 
-// Three-stage step: S(n+1) = K(n+1) Q^T, O += P(n-1) V(n-1) and the softmax of
-// S(n) -> P(n) share one instruction stream, so the softmax's VALU work
-// overlaps 32 MFMAs instead of 16. O is rescaled to the new running max after
-// the P(n-1) V(n-1) products; P(n) V(n) is left to the next step. QK = false
-// drops the score product (last tile), PV = false the value product (first).
-// The two key halves of S(n+1) accumulate alternately (MFMA i adds channel
-// chunk i/2 to half i%2), so consecutive score MFMAs are independent (with the
-// halves one after the other, each a chain of 8, the loop ran 1.3-2% slower).
-// kl, vl: this lane's operand addresses (k_lane, v_lane) in K(n+1) and V(n-1).
-// The step is one hand-ordered stream (fwd_common.hpp: mfma_v*, exp_pair):
-// slot i (16 per step) issues the MFMA of score chunk i, the exps of P(n)
-// word i (two scores of S(n)), then the MFMA of P.V operand i; the K and V
-// operands of slot i + 2 are read at the top of slot i (the empty asm with a
-// memory clobber keeps the reads there, so each has two slots to land).
-// Measured on a stand-alone copy of the loop: 1346 against 1250 TFLOP/s, the
-// compiler's order having issued the MFMAs four at a time with the softmax
-// between the groups.
-// Lazy tile max: the exps use the running max as it stands, and the tile's max
-// is taken only when a lane's row sum exceeds 255. No sum above 255 means every
-// p <= 255, i.e. every score is below the running max + log2(255.5) <
-// kMaxSlack, so the tile would not have moved the max: the running max evolves
-// as with the max taken every step. The first exact tile of a workgroup
-// (running max -inf, p = inf) always takes that path.
-template <bool QK, bool PV>
-__device__ __forceinline__ void step3(SoftmaxState& st, const f32x16 (&sc)[2], f32x16 (&sn)[2],
-                                      const bf16x8 (&pp)[4], bf16x8 (&pn)[4], uint32_t kl,
-                                      uint32_t vl, const bf16x8 (&q)[8], float c) {
-  static_assert(kMaxSlack >= 8.f, "the lazy test relies on 255 < 2^kMaxSlack");
-  bf16x8 ka[3], va[3];
-  uint32_t pw[4][4];
-  float psum = 0.f;
-  const float neg = -st.m;
-  if constexpr (QK) {
-    ka[0] = k_op_x(kl, 0, 0);
-    ka[1] = k_op_x(kl, 1, 0);
-  }
-  if constexpr (PV) {
-    va[0] = v_op_x(vl, 0, 0);
-    va[1] = v_op_x(vl, 0, 1);
-  }
-  asm volatile("" ::: "memory");
-  const auto unit = [&](int i) {
-    const int ks = i >> 2, w = i & 3;
-    const int r = 8 * (ks & 1) + 2 * w;
-    pw[ks][w] = exp_pair(sc[ks >> 1][r], sc[ks >> 1][r + 1], c, neg, psum);
-  };
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + 2 < 16) {
-      if constexpr (QK) ka[(i + 2) % 3] = k_op_x(kl, (i + 2) & 1, (i + 2) >> 1);
-      if constexpr (PV) va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
-      asm volatile("" ::: "memory");
-    }
-    if constexpr (QK) {
-      // the two key halves of S(n+1) alternate (consecutive MFMAs independent)
-      if (i < 2)
-        mfma_v0(sn[i & 1], ka[i % 3], q[i >> 1]);
-      else
-        mfma_v(sn[i & 1], ka[i % 3], q[i >> 1]);
-      unit(i);
-    }
-    if constexpr (PV) {
-      if (i == 0)
-        mfma_v_first(st.acc[0], va[0], pp[0]);
-      else if (QK && i == 15)
-        mfma_v_tie(st.acc[3], va[0], pp[3], sn);  // va[15 % 3]
-      else
-        mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
-    }
-    if constexpr (!QK) unit(i);
-    // Raised wave priority for the rest of the step: the issue arbiter then
-    // prefers a wave inside its MFMA stream over one at its copies / barrier
-    // (about 1-2% at cfg 2).
-    if (i == 0) __builtin_amdgcn_s_setprio(1);
-  }
-  __builtin_amdgcn_s_setprio(0);
-  if constexpr (QK && !PV) mfma_fence(sn);
-  if constexpr (!QK) mfma_fence(st.acc);  // the plain path's builtin MFMAs follow
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    pn[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
-  float alpha = 1.f;
-  if (__any(!(psum <= 255.f))) {  // (also catches inf / NaN)
-    float mx = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
-    const float m_new = new_max(st.m, xhalf_max(mx) * c, alpha);
-    if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
-      st.m = m_new;
-      psum = 0.f;
-      psum = exp8<0>(sc[0], c, -m_new, pn[0], psum);
-      psum = exp8<8>(sc[0], c, -m_new, pn[1], psum);
-      psum = exp8<0>(sc[1], c, -m_new, pn[2], psum);
-      psum = exp8<8>(sc[1], c, -m_new, pn[3], psum);
-      if constexpr (PV) mfma_fence(st.acc);  // the rescale reads O
-      rescale(st, alpha);
-    }
-  }
-  st.l = fmaf(st.l, alpha, psum);
-}
-
-// Block 64 forward (workgroups of 2 waves). K and V hold two half tiles of 32
-// keys each (32 KiB), so four workgroups and two waves per SIMD fit a CU. Tile
-// order: with T not a multiple of 64, the tile of the short last block through
-// the plain path (as a ragged exact tile, or inside its pooled tile, where it
-// weighs its own length); then the pooled and the full exact tiles through the
+// The forward. Workgroups of 2 waves at block 64 (four per CU), 4 at block 128
+// (two per CU): two waves per SIMD. K and V hold two half tiles of 32 keys each
+// (32 KiB). Tile order: the tile of a short last block, if any, through the
+// plain path (as a ragged exact tile, or inside its pooled tile, where it weighs
+// its own length); then the pooled and the full exact tiles through the
 // pipeline, two half steps a tile.
 //
-// Bound: at 32760 tokens the tile copies (without them, results wrong by
-// construction, the two-stage form of this kernel ran 19% faster; with all of
-// them hitting L2, 8%), then the MFMAs at the power-limited clock; at 4096
-// tokens (1.5 workgroups a slot) the workgroup's own latency. Half tiles
-// against the two-stage step over whole tiles (K copied behind 16 bare P.V
-// MFMAs, V behind QK and the exps): every copy gets a whole step, the MFMAs of
-// both products hide the exps, and the scores take 32 registers less. Calls:
-// 32760 tokens 2835 -> 2737 us, 12133 packed 623 -> 606, 4096 91.2 -> 87.4,
-// 9180 with 64-channel heads 247.5 -> 239.5.
+// Bound: at 32760 tokens the MFMAs at the power-limited clock and the tile
+// copies (block 64: without them, results wrong by construction, the two-stage
+// form of this kernel ran 19% faster; with all of them hitting L2, 8%); at 4096
+// tokens (1.5 workgroups a slot at block 64) the workgroup's own latency.
+// Half tiles against a two-stage step over whole tiles at block 64 (K copied
+// behind 16 bare P.V MFMAs, V behind QK and the exps): every copy gets a whole
+// step, the MFMAs of both products hide the exps, and the scores take 32
+// registers less, so the pooled tiles fit the pipeline. Calls: 32760 tokens 2835
+// -> 2737 us, 12133 packed 623 -> 606, 4096 91.2 -> 87.4. At block 128 against a
+// three-stage step over whole tiles, double buffered in 64 KiB, with plain
+// pooled tiles: 32760 tokens 2370 -> 2325 us, 75600 tokens 21.2 -> 21.0 ms; four
+// half buffers with copies two steps ahead were slower (2400 us).
 template <int BLK>
 __global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))
-fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
+fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
                 const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_t, int64_t sk_h,
                 const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
                 const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t npad,
@@ -260,9 +158,11 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
 
   const int ntiles = build_tile_list<BLK>(tl, mask, row, NT, W, T);
   if (ntiles == 0) return;  // cannot happen for routed masks: the diagonal is exact
-  const int nplain = T % kKeys != 0 ? 1 : 0;
-  const bool rag = ragged_tiles(tl, NT, T) != 0;  // the plain tile is exact, else pooled
-  const int npool = tl.npool - (nplain && !rag ? 1 : 0);  // pipelined pooled tiles, first in order
+  // The plain tile: a ragged exact one, or the pooled tile of a short last block.
+  const bool rag = ragged_tiles(tl, NT, T) != 0;
+  const bool tail = T % BLK != 0 && tl.last != NT - 1;
+  const int nplain = rag || tail ? 1 : 0;
+  const int npool = tl.npool - (tail ? 1 : 0);  // pipelined pooled tiles, first in order
   const int npipe = ntiles - nplain;
 
   const KVSource src{k + b * sk_b + h * sk_h, sk_t, v + b * sv_b + h * sv_h, sv_t,
@@ -358,23 +258,23 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
     if (npool > 0) {
       issue_any(min(1, last), 0, 0);
       mask_scores(sa, static_cast<uint32_t>(tl.pmask[0]));
-      half_step<BLK, true, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
+      half_step<BLK, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
       land();
       issue_any(min(1, last), 0, 1);
       issue_any(0, 1, 1);
       mask_scores(sb, static_cast<uint32_t>(tl.pmask[0] >> 32));
-      half_step<BLK, true, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      half_step<BLK, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
       land();
       for (t = 1; t < npool; ++t) {
         issue_any(min(t + 1, last), 0, 0);
         issue_any(t, 1, 0);
         mask_scores(sa, static_cast<uint32_t>(tl.pmask[t]));
-        half_step<BLK, true, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
+        half_step<BLK, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
         land();
         issue_any(min(t + 1, last), 0, 1);
         issue_any(t, 1, 1);
         mask_scores(sb, static_cast<uint32_t>(tl.pmask[t] >> 32));
-        half_step<BLK, true, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+        half_step<BLK, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
         land();
       }
     }
@@ -383,11 +283,11 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
     int f0 = first_of(min(t, last)), f1 = first_of(min(t + 1, last));
     if (npool == 0) {
       issue_k_at(f1, 0);
-      half_step<BLK, false, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
+      half_step<BLK, false, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
       land();
       issue_k_at(f1, 1);
       issue_v_at(f0, 1);
-      half_step<BLK, false, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      half_step<BLK, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
       f0 = f1;
       f1 = first_of(min(2, last));
       land();
@@ -396,13 +296,13 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
     for (; t < npipe; ++t) {
       issue_k_at(f1, 0);
       issue_v_at(f0, 0);
-      half_step<BLK, false, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
+      half_step<BLK, false, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
       asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
       const int f2 = first_of(min(t + 2, last));
       land();
       issue_k_at(f1, 1);
       issue_v_at(f0, 1);
-      half_step<BLK, false, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      half_step<BLK, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
       land();
       f0 = f1;
       f1 = f2;
@@ -412,188 +312,6 @@ fwd_bf16_sbuf_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       st.acc[i & 3] = mfma_bf16(v_op_x(vl1, i >> 2, i & 3), pb[i >> 2], st.acc[i & 3]);
-  }
-  wait_tile_copies();
-
-  store_rows(st, o + b * so_b + h * so_h, so_t, qrow, T, half);
-}
-
-// Block 128 forward with the three-stage pipeline. Tile order: the full
-// exact tiles first (list tiles 0 .. nfast-1, ascending keys), then the
-// ragged exact tile (if any) and the pooled tiles. K and V are double
-// buffered (64 KiB, two workgroups per CU). The full exact phase runs first
-// so that the plain phase's registers are not live across its loop.
-template <int BLK>
-__global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))
-fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
-                     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_t, int64_t sk_h,
-                     const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
-                     const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t npad,
-                     const int32_t* __restrict__ counts, const uint32_t* __restrict__ mask, int T, int H, int NT, int W, float c,
-                     uint16_t* __restrict__ o, int64_t so_b, int64_t so_t, int64_t so_h) {
-  constexpr int NTHREADS = BLK * 2;
-  constexpr int kCopiesPerTile = 2 * CopyOffsets<NTHREADS>::U;
-  __shared__ __align__(256) uint16_t kbuf[2][kTileElems];
-  __shared__ __align__(256) uint16_t vbuf[2][kTileElems];
-  __shared__ TileList tl;
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = lane & 31, half = lane >> 5;
-  int bh, qb;
-  tile_coords_lpt<kLptTokens / BLK>(counts, NT, bh, qb);
-  const int b = bh / H, h = bh % H;
-  const int64_t row = static_cast<int64_t>(bh) * NT + qb;
-
-  const int ntiles = build_tile_list<BLK>(tl, mask, row, NT, W, T);
-  if (ntiles == 0) return;  // cannot happen for routed masks: the diagonal is exact
-  const int nrag = ragged_tiles(tl, NT, T);
-  // Full exact tiles (list tiles 0 .. nfast-1) run through the pipeline when
-  // there are at least two; a lone one runs as the first plain tile.
-  const int nfast = ntiles - tl.npool - nrag;
-  const int nlone = nfast == 1 ? 1 : 0;
-  const int npipe = nfast - nlone;
-  const int nplain = nlone + nrag + tl.npool;
-
-  const KVSource src{k + b * sk_b + h * sk_h, sk_t, v + b * sv_b + h * sv_h, sv_t,
-                     kc + (static_cast<int64_t>(b) * npad * H + h) * kD,
-                     static_cast<int64_t>(H) * kD, vc + (static_cast<int64_t>(b) * npad * H + h) * kD};
-  CopyOffsets<NTHREADS> off;
-  off.init(sk_t, sv_t);
-  const uint32_t kb = lds_addr(kbuf[0]), vb = lds_addr(vbuf[0]);  // LDS byte addresses
-  const auto issue_k_at = [&](int first, int buf) {
-    issue_full<NTHREADS>(kb + buf * kTileBytes, src.k + static_cast<int64_t>(first) * src.sk, src.sk, off.k);
-  };
-  const auto issue_v_at = [&](int first, int buf) {
-    issue_full<NTHREADS>(vb + buf * kTileBytes, src.v + static_cast<int64_t>(first) * src.sv, src.sv, off.v);
-  };
-  const auto issue_k = [&](int e, int buf) { issue_k_at(exact_first<BLK>(tl, e), buf); };
-  const auto issue_v = [&](int e, int buf) { issue_v_at(exact_first<BLK>(tl, e), buf); };
-  // Plain tile p: the lone full exact tile (p < nlone), the ragged exact tile
-  // (p < nlone + nrag), then the pooled tiles.
-  const auto plain_desc = [&](int p) {
-    if (p < nlone) return exact_desc<BLK>(tl, 0, T, NT);
-    if (p < nlone + nrag) return exact_desc<BLK>(tl, tl.nexact - 1, T, NT);
-    return pooled_desc(tl, p - nlone - nrag, NT);
-  };
-  const auto issue_plain_k = [&](int p, int buf) {
-    issue_generic<NTHREADS>(kb + buf * kTileBytes, 0, plain_desc(p), src);
-  };
-  const auto issue_plain_v = [&](int p, int buf) {
-    issue_generic<NTHREADS>(vb + buf * kTileBytes, 1, plain_desc(p), src);
-  };
-  if (npipe > 0) {
-    issue_k(0, 0);
-    issue_v(0, 0);
-    issue_k(1, 1);
-  } else {
-    issue_plain_k(0, 0);
-    issue_plain_v(0, 0);
-  }
-
-  // This wave's 32 query rows as the B operand of S^T = K Q^T.
-  const int qrow = qb * BLK + wave * 32 + col;
-  bf16x8 qreg[8];
-  {
-    const uint16_t* qp = q + b * sq_b + static_cast<int64_t>(qrow) * sq_t + h * sq_h + half * 8;
-#pragma unroll
-    for (int cc = 0; cc < 8; ++cc) {
-      uint4 r = make_uint4(0u, 0u, 0u, 0u);
-      if (qrow < T) r = *reinterpret_cast<const uint4*>(qp + cc * 16);
-      qreg[cc] = __builtin_bit_cast(bf16x8, r);
-    }
-  }
-
-  SoftmaxState st;
-  st.init();
-  int pbuf = 0;  // buffer of plain tile 0
-  // This lane's operand addresses in K / V buffer 0 (buffer 1 is kTileBytes on).
-  const uint32_t kl0 = k_lane(kb, col, half);
-  const uint32_t vl0 = v_lane(vb, lane);
-
-  // ---- full exact tiles. On entry to step n (0 < n < npipe): S(n) and
-  // P(n-1) in registers, K(n+1) and V(n-1) in LDS; the step copies K(n+2)
-  // over K(n) and V(n) over V(n-2). K(n+2) past the last tile is clamped to
-  // it: a redundant copy into a buffer nothing reads afterwards.
-  if (npipe > 0) {
-    f32x16 sa[2], sb[2];
-    wait_tile_copies();
-    __syncthreads();
-    qk_tile(kl0, qreg, sa);
-    mfma_fence(sa);   // the step's softmax reads S(0) through asm
-    __syncthreads();  // every wave is done with K(0)
-    {
-      const int E = npipe;
-      bf16x8 pa[4], pb[4];
-      issue_k(min(2, E - 1), 0);
-      // First token rows of the tiles the next step copies, read from the LDS
-      // list one step ahead: each step issues its copies from scalars it
-      // already holds instead of waiting on an LDS read first.
-      int kf = exact_first<BLK>(tl, min(3, E - 1)), vf = exact_first<BLK>(tl, 1);
-      step3<true, false>(st, sa, sb, pb, pa, kl0 + kTileBytes, 0u, qreg, c);
-      wait_tile_copies();
-      __syncthreads();
-      int n = 1;  // S(n) in sb, P(n-1) in pa
-      const auto gstep = [&](const f32x16 (&sc)[2], f32x16 (&sn)[2], const bf16x8 (&pp)[4],
-                             bf16x8 (&pn)[4]) {
-        issue_k_at(kf, n & 1);  // K(min(n + 2, E - 1))
-        issue_v_at(vf, n & 1);  // V(n)
-        step3<true, true>(st, sc, sn, pp, pn, kl0 + ((n + 1) & 1) * kTileBytes,
-                                vl0 + ((n - 1) & 1) * kTileBytes, qreg, c);
-        // after the MFMA stream, so the read's latency overlaps the copy wait
-        // and the barrier below rather than delaying this step's first MFMAs
-        asm volatile("" ::: "memory");
-        kf = exact_first<BLK>(tl, min(n + 3, E - 1));
-        vf = exact_first<BLK>(tl, n + 1);
-        wait_tile_copies();
-        __syncthreads();
-        ++n;
-      };
-      // Last tile n = E-1: no K left. Plain tile 0 is copied into the buffers
-      // of tile n-1 while P(n-1) V(n-1), the softmax of S(n) and P(n) V(n) run.
-      const auto last = [&](const f32x16 (&sc)[2], f32x16 (&dummy)[2], const bf16x8 (&pp)[4],
-                            bf16x8 (&pn)[4]) {
-        pbuf = (n - 1) & 1;
-        issue_v_at(vf, n & 1);  // V(n)
-        if (nplain > 0) issue_plain_k(0, pbuf);
-        step3<false, true>(st, sc, dummy, pp, pn, 0u, vl0 + pbuf * kTileBytes, qreg, c);
-        if (nplain > 0)
-          wait_vmcnt<kCopiesPerTile / 2>();  // V(n) landed; plain K(0) may be in flight
-        else
-          wait_tile_copies();
-        __syncthreads();  // every wave is done with V(n-1)
-        if (nplain > 0) issue_plain_v(0, pbuf);
-        pv_tile(vl0 + (n & 1) * kTileBytes, pn, lane, st.acc);
-      };
-      // Pairs of steps, so the S and P buffers swap roles without copies.
-      while (n + 2 < E) {
-        gstep(sb, sa, pa, pb);
-        gstep(sa, sb, pb, pa);
-      }
-      if (n + 1 < E) {
-        gstep(sb, sa, pa, pb);
-        last(sa, sb, pb, pa);
-      } else {
-        last(sb, sa, pa, pb);
-      }
-      __syncthreads();  // every wave is done with V(E-1) before plain tile 1 lands there
-    }
-  }
-
-  // ---- ragged and pooled tiles; plain tile p sits in buffers (pbuf + p) & 1
-  for (int p = 0; p < nplain; ++p) {
-    const int cur = (pbuf + p) & 1;
-    if (p + 1 < nplain) {
-      issue_plain_k(p + 1, cur ^ 1);
-      issue_plain_v(p + 1, cur ^ 1);
-      wait_vmcnt<kCopiesPerTile>();  // tile p landed; tile p+1 stays in flight
-    } else {
-      wait_tile_copies();
-    }
-    __syncthreads();
-    f32x16 s[2];
-    qk_tile(kl0 + cur * kTileBytes, qreg, s);
-    finish_tile<BLK>(st, s, vl0 + cur * kTileBytes, plain_desc(p), c, lane, NT, T);
-    __syncthreads();
   }
   wait_tile_copies();
 
@@ -622,16 +340,10 @@ extern "C" int solattn_fwd_bf16(const uint16_t* q, int64_t sq_b, int64_t sq_t, i
   const float c = scale * kLog2e;
   const uint32_t grid = static_cast<uint32_t>(B * H * NT);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (block == 128) {
-    hipLaunchKernelGGL((bf16fwd::fwd_bf16_kernel<128>), dim3(grid), dim3(256), blist_lds_bytes(NT), s,
-                       q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc, vc, npad,
-                       counts, mask, static_cast<int>(T), static_cast<int>(H),
-                       static_cast<int>(NT), W, c, o, so_b, so_t, so_h);
-  } else {
-    hipLaunchKernelGGL((bf16fwd::fwd_bf16_sbuf_kernel<64>), dim3(grid), dim3(128), blist_lds_bytes(NT), s, q,
-                       sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc, vc, npad,
-                       counts, mask, static_cast<int>(T), static_cast<int>(H),
-                       static_cast<int>(NT), W, c, o, so_b, so_t, so_h);
-  }
+  hipLaunchKernelGGL(block == 128 ? bf16fwd::fwd_bf16_kernel<128> : bf16fwd::fwd_bf16_kernel<64>,
+                     dim3(grid), dim3(static_cast<uint32_t>(block) * 2), blist_lds_bytes(NT), s, q, sq_b,
+                     sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc, vc, npad, counts, mask,
+                     static_cast<int>(T), static_cast<int>(H), static_cast<int>(NT), W, c, o, so_b, so_t,
+                     so_h);
   return check_launch("fwd_bf16");
 }

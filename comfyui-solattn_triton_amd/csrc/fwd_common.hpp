@@ -505,12 +505,6 @@ __device__ __forceinline__ void mfma_v_first(f32x16& d, const bf16x8& a, const b
   asm volatile("s_nop 2\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
 }
 // An MFMA that also passes s through: readers of s come after it.
-__device__ __forceinline__ void mfma_v_tie(f32x16& d, const bf16x8& a, const bf16x8& b,
-                                           f32x16 (&s)[2]) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %3, %4, %0\n\ts_nop 3"
-               : "+v"(d), "+v"(s[0]), "+v"(s[1])
-               : "v"(a), "v"(b));
-}
 __device__ __forceinline__ void mfma_v_tie(f32x16& d, const bf16x8& a, const bf16x8& b, f32x16& s) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\ts_nop 3"
                : "+v"(d), "+v"(s)

@@ -413,7 +413,7 @@ __device__ __forceinline__ void fast_step_bf16pv(SoftmaxState& st, const f32x16 
 // LDS). The last score MFMA is followed by two exp pairs and a P.V MFMA before
 // the int32 scores are read. QK = false: the last tile (no scores to make);
 // PV = false: the first. Lazy tile max, hazards and the final O rescale as
-// in the BF16 forward's step3. qc: the factor of sc's scores.
+// in the BF16 forward's half_step. qc: the factor of sc's scores.
 template <bool QK, bool PV, bool UKS>
 __device__ __forceinline__ void step3_i8(SoftmaxState& st, const f32x16 (&sc)[2], float qc,
                                          f32x16 (&sn)[2], const bf16x8 (&pp)[4], bf16x8 (&pn)[4],

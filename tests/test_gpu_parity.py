@@ -513,3 +513,38 @@ def test_head_dim_64(pkg, dev, mode, case):
         err, cos = compare_rows(out.float().cpu().numpy(), port, block)
         print(f"[d64 {case} bf16] max|err|={err:.3e} cos={cos:.6f}", flush=True)
         assert err < BF16_MAXABS and cos >= BF16_COS
+
+
+@pytest.mark.parametrize("block,T", [(64, 64 * 70 + 17), (64, 64 * 64), (128, 128 * 66 + 64), (128, 128 * 65 + 90)])
+def test_fwd_bf16_hand_set_masks(pkg, dev, block, T):
+    """Tile orders the router never gives: rows with no exact block (pooled tiles
+    only, a partial chunk and a short last block among them), with the last block
+    alone, with the first alone, with every second block. Against float64: P and
+    the outputs are rounded to bf16 (2^-9 each) under values of order 1, far
+    inside BF16_MAXABS."""
+    prep, tri = _mods(pkg)[0], _mods(pkg)[1]
+    q, k, v = (randn_bf16((1, T, 1, 128), s) for s in (90, 91, 92))
+    r = prep.route(q.to(dev), k.to(dev), v.to(dev), scale=128 ** -0.5, tau=0.9, block=block)
+    NT = r.counts.shape[-1]
+    exact = torch.zeros(4, NT, dtype=torch.bool)
+    exact[1, NT - 1] = exact[2, 0] = True
+    exact[3, ::2] = True
+    rows = exact[torch.arange(NT) % 4]  # [query block, key block]
+    j = torch.arange(NT)
+    words = torch.zeros(NT, r.mask.shape[-1], dtype=torch.int64)
+    words.index_add_(1, j >> 5, rows.long() << (j & 31))
+    mask = torch.where(words >= 2 ** 31, words - 2 ** 32, words).to(torch.int32).to(dev)
+    r = r._replace(mask=mask.reshape(r.mask.shape).contiguous(),
+                   counts=rows.sum(-1).to(torch.int32).to(dev).reshape(r.counts.shape))
+    print(f"[hand masks] block={block} T={T}", flush=True)
+    out = tri.forward_bf16(q.to(dev), k.to(dev), v.to(dev), r).float().cpu()[0, :, 0]
+    lens = torch.full((NT,), float(block), dtype=torch.float64)
+    lens[-1] = T - (NT - 1) * block
+    qd, kd, vd = (t[0, :, 0].double() for t in (q, k, v))
+    kc, vc = (t[0, :NT, 0].double().cpu() for t in (r.kc, r.vc))
+    on = rows[torch.arange(T) // block]
+    s = (qd @ kd.t() * 128 ** -0.5).masked_fill(~on[:, torch.arange(T) // block], -torch.inf).exp()
+    p = (qd @ kc.t() * 128 ** -0.5).masked_fill(on, -torch.inf).exp()
+    ref = (s @ vd + p @ vc) / (s.sum(1) + p @ lens)[:, None]
+    assert float((out - ref).abs().max()) < BF16_MAXABS
+    assert cosine(out.numpy(), ref.numpy()) >= BF16_COS

@@ -36,8 +36,8 @@ def sol_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float 
              use_tma: bool = False, block: int = BLOCK) -> torch.Tensor:
     """Run Sol-Attn on BTHD bf16 inputs; returns a fresh BTHD bf16 tensor.
 
-    Head dims below 128 (multiples of 8) run zero-padded to 128 inside the
-    library call. Each query block attends exactly to its routed blocks (score above the
+    Head dims below 128 (multiples of 8) run as they are (64) or zero-padded to
+    64 or 128 inside the library call. Each query block attends exactly to its routed blocks (score above the
     Gaussian threshold mu + tau*sigma, the diagonal band |i-j| <= 1 and the
     ``sink_blocks`` KV range) and to one pooled key/value per remaining block;
     query blocks inside ``sink_q`` attend everything exactly.

@@ -43,26 +43,31 @@ uint64_t spread3(uint64_t v) {
   return out;
 }
 
-// Head dims the one-call pipelines take: multiples of 8 up to the kernels'
-// 128; smaller heads are zero-padded to 128 in the workspace.
+// Head dims the one-call pipelines take: multiples of 8 up to 128. The BF16
+// kernels run 64 and 128 channels, the INT8 kernels 128; other heads are
+// zero-padded to the next of these in the workspace. (64-channel heads padded
+// to 128 moved and multiplied twice what they hold, after three copies: 240
+// against 150 us for 9180 tokens of 16 heads at block 64.)
 constexpr int64_t kKernelD = 128;
+inline int64_t kernel_head_dim(int64_t D, bool int8) { return !int8 && D <= 64 ? 64 : kKernelD; }
 inline bool pipeline_head_dim_ok(int64_t D) { return D >= 8 && D <= kKernelD && D % 8 == 0; }
 
 // Carves the pipeline's intermediates out of one workspace.
 struct Layout {
   int64_t NT, npad, W, TP;
+  int64_t Dk;  // the kernels' head dim
   int64_t kc, vc, qbar, kc_mean, kc_var, thr, counts, mask;   // byte offsets
   int64_t vamax, vscale, qi, qs, ki, ks, vi;                          // INT8 only
-  int64_t qp, kp, vp, op;  // zero-padded [B, T, H, 128] q, k, v, o (head dims < 128)
+  int64_t qp, kp, vp, op;  // zero-padded [B, T, H, Dk] q, k, v, o (head dims below 128)
   bool padded;
   int64_t total;
   Layout(int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, bool int8) {
-    const int64_t Dk = kKernelD;
+    Dk = kernel_head_dim(D, int8);
     NT = cdiv(T, block);
     npad = cdiv(NT, 64) * 64;
     W = cdiv(NT, 32);
     TP = T;
-    padded = D != Dk;
+    padded = D != kKernelD;  // heads of 64 too: strides the kernels refuse go through copies
     int64_t off = 0;
     auto take = [&](int64_t bytes) {
       const int64_t at = off;
@@ -157,14 +162,16 @@ struct Call {
   int64_t skv_lo, skv_hi, sq_lo, sq_hi;
 };
 
-// Runs fn on the call as the D = 128 kernels see it: unchanged when D is 128,
-// else on zero-padded copies of q, k, v in the workspace with the output
+// Runs fn on the call as the kernels see it: unchanged when D is theirs (L.Dk;
+// at 64 also with token strides in the kernels' range, which copies take out of
+// the caller's hands), else on zero-padded copies of q, k, v in the workspace with the output
 // sliced back into the caller's o afterwards (zero channels add exact zeros
 // to every dot product and sum).
 template <typename F>
 int with_kernel_head_dim(const Layout& L, void* ws, const Call& c, hipStream_t s, F&& fn) {
-  if (!L.padded) return fn(c);
-  const int64_t Dk = kKernelD, st = c.H * Dk, sb = c.T * st;
+  const auto direct = [](int64_t st) { return st >= 0 && st < (1ll << 24); };
+  if (!L.padded || (c.D == L.Dk && direct(c.sq_t) && direct(c.sk_t) && direct(c.sv_t))) return fn(c);
+  const int64_t Dk = L.Dk, st = c.H * Dk, sb = c.T * st;
   Call p = c;
   uint16_t* qp = at<uint16_t>(ws, L.qp);
   uint16_t* kp = at<uint16_t>(ws, L.kp);
@@ -187,23 +194,25 @@ int with_kernel_head_dim(const Layout& L, void* ws, const Call& c, hipStream_t s
 // out of ws (256-byte aligned, at least L.total bytes; nothing in it needs to
 // start zeroed: every byte a later stage reads is written by an earlier one).
 int run_bf16_pipeline(const Layout& L, void* ws, const Call& call, solattn_stream_t stream) {
-  return with_kernel_head_dim(L, ws, call, reinterpret_cast<hipStream_t>(stream), [&](const Call& c) {
-    int rc = solattn_pool(c.q, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h, c.v, c.sv_b,
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  return with_kernel_head_dim(L, ws, call, hs, [&](const Call& c) {
+    int rc = pool_checked(c.q, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h, c.v, c.sv_b,
                           c.sv_t, c.sv_h, c.B, c.T, c.H, c.D, c.block, at<uint16_t>(ws, L.kc),
-                          at<uint16_t>(ws, L.vc), L.npad, at<float>(ws, L.qbar), nullptr, stream);
+                          at<uint16_t>(ws, L.vc), L.npad, at<float>(ws, L.qbar), nullptr, nullptr, nullptr,
+                          0, hs);
     if (rc) return rc;
-    rc = solattn_moments(at<uint16_t>(ws, L.kc), L.npad, c.B, L.NT, c.H, c.D, 0,
-                         at<float>(ws, L.kc_mean), at<float>(ws, L.kc_var), nullptr, nullptr, stream);
+    rc = moments(at<uint16_t>(ws, L.kc), L.npad, c.B, L.NT, c.H, c.D, 0, at<float>(ws, L.kc_mean),
+                 at<float>(ws, L.kc_var), nullptr, nullptr, hs);
     if (rc) return rc;
-    rc = solattn_route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.npad,
-                       at<float>(ws, L.kc_mean), at<float>(ws, L.kc_var), c.B, c.T, c.H, c.D,
-                       c.block, c.scale, c.tau, 0, c.skv_lo, c.skv_hi, c.sq_lo, c.sq_hi,
-                       at<float>(ws, L.thr), at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), stream);
+    rc = route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.npad, at<float>(ws, L.kc_mean),
+               at<float>(ws, L.kc_var), c.B, c.T, c.H, c.D, c.block, c.scale, c.tau, 0, c.skv_lo,
+               c.skv_hi, c.sq_lo, c.sq_hi, at<float>(ws, L.thr), at<int32_t>(ws, L.counts),
+               at<uint32_t>(ws, L.mask), hs);
     if (rc) return rc;
-    return solattn_fwd_bf16(c.q, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h, c.v, c.sv_b,
-                            c.sv_t, c.sv_h, at<uint16_t>(ws, L.kc), at<uint16_t>(ws, L.vc), L.npad,
-                            at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), c.B, c.T, c.H, c.D, c.block, c.scale, c.o,
-                            c.so_b, c.so_t, c.so_h, stream);
+    return fwd_bf16(c.q, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h, c.v, c.sv_b,
+                    c.sv_t, c.sv_h, at<uint16_t>(ws, L.kc), at<uint16_t>(ws, L.vc), L.npad,
+                    at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), c.B, c.T, c.H, c.D, c.block,
+                    c.scale, c.o, c.so_b, c.so_t, c.so_h, hs);
   });
 }
 
@@ -226,13 +235,12 @@ int run_int8_pipeline(const Layout& L, void* ws, const Call& call, int int8_pv,
                           qk_block ? nullptr : at<int8_t>(ws, L.qi),
                           qk_block ? nullptr : at<float>(ws, L.qs), L.TP, hs);
     if (rc) return rc;
-    rc = solattn_moments(at<uint16_t>(ws, L.kc), L.npad, c.B, L.NT, c.H, c.D, 1,
-                         at<float>(ws, L.kc_mean), at<float>(ws, L.kc_var), vamax, vscale, stream);
+    rc = moments(at<uint16_t>(ws, L.kc), L.npad, c.B, L.NT, c.H, c.D, 1, at<float>(ws, L.kc_mean),
+                 at<float>(ws, L.kc_var), vamax, vscale, hs);
     if (rc) return rc;
-    rc = solattn_route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.npad, nullptr,
-                       at<float>(ws, L.kc_var), c.B, c.T, c.H, c.D, c.block, c.scale, c.tau, 1,
-                       c.skv_lo, c.skv_hi, c.sq_lo, c.sq_hi, at<float>(ws, L.thr),
-                       at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), stream);
+    rc = route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.npad, nullptr, at<float>(ws, L.kc_var),
+               c.B, c.T, c.H, c.D, c.block, c.scale, c.tau, 1, c.skv_lo, c.skv_hi, c.sq_lo, c.sq_hi,
+               at<float>(ws, L.thr), at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), hs);
     if (rc) return rc;
     rc = quant_qkv(qk_block ? c.q : nullptr, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h,
                    c.v, c.sv_b, c.sv_t, c.sv_h, c.B, c.T, c.H, c.D, at<float>(ws, L.kc_mean),

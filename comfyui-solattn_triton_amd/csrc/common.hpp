@@ -102,19 +102,26 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// The pooling pass (prep.hip) with, when qi != null, the per-token INT8 of q
-// (codes qi [B, TP, H, 128], scales qs [B, TP, H]) in the same read;
-// pool_checked validates the arguments as solattn_pool does.
+// The stages of the one-call pipelines for head dims 128 and (BF16 only) 64;
+// arguments are validated as in the public entry points, which take 128 alone.
+// pool_checked: the pooling pass (prep.hip) with, when qi != null, the per-token
+// INT8 of q (codes qi [B, TP, H, 128], scales qs [B, TP, H]) in the same read.
 int pool_checked(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
                  int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b,
                  int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t D,
                  int64_t block, uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar,
                  float* vamax_part, int8_t* qi, float* qs, int64_t TP, hipStream_t s);
-int launch_pool(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
-                int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b,
-                int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t block,
-                uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar, float* vamax_part,
-                int8_t* qi, float* qs, int64_t TP, hipStream_t s);
+int moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H, int64_t D, int centre,
+            float* kc_mean, float* kc_var, const float* vamax_part, float* vscale, hipStream_t s);
+int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_mean, const float* kc_var,
+          int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
+          int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr,
+          int32_t* counts, uint32_t* mask, hipStream_t s);
+int fwd_bf16(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
+             int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b, int64_t sv_t,
+             int64_t sv_h, const uint16_t* kc, const uint16_t* vc, int64_t npad, const int32_t* counts,
+             const uint32_t* mask, int64_t B, int64_t T, int64_t H, int64_t D, int64_t block,
+             float scale, uint16_t* o, int64_t so_b, int64_t so_t, int64_t so_h, hipStream_t s);
 
 // The INT8 preparation with one read of q, k and v (prep.hip): pooled keys,
 // centred kc, moments, V scale, Q/K/V codes; as solattn_prep_int8, whose

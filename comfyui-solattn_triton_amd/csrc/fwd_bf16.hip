@@ -46,42 +46,50 @@ namespace bf16fwd {
 // Raised wave priority for the step's stream: the issue arbiter then prefers a
 // wave inside its MFMAs over one at its copies or barrier (without it, 6%
 // slower at block 64 and 32760 tokens).
-template <int BLK, bool POOLED, bool PV>
-__device__ __forceinline__ void half_step(SoftmaxState& st, const f32x16& sc, f32x16& sn,
+// 64 channels halve the MFMAs: one of each product per two slots.
+template <int BLK, int D, bool POOLED, bool PV>
+__device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x16& sc, f32x16& sn,
                                           const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
-                                          uint32_t vl, const bf16x8 (&q)[8], float c) {
+                                          uint32_t vl, const bf16x8 (&q)[D / 16], float c) {
   static_assert(kMaxSlack >= 8.f, "the lazy test relies on 255 < 2^kMaxSlack");
+  constexpr int ND = D / 32, NM = D / 16;  // MFMAs of each product
+  constexpr int SLOTS = 8 / NM;            // slots per MFMA of each
   bf16x8 ka[3], va[3];
   uint32_t pw[2][4];
   float psum = 0.f;
   const float neg = -st.m;
-  ka[0] = k_op_x(kl, 0, 0);
-  ka[1] = k_op_x(kl, 0, 1);
+  ka[0] = k_op_x<D>(kl, 0, 0);
+  ka[1] = k_op_x<D>(kl, 0, 1);
   if constexpr (PV) {
-    va[0] = v_op_x(vl, 0, 0);
-    va[1] = v_op_x(vl, 0, 1);
+    va[0] = v_op_x<D>(vl, 0, 0);
+    va[1] = v_op_x<D>(vl, 0, 1);
   }
   asm volatile("" ::: "memory");
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    if (i + 2 < 8) {
-      ka[(i + 2) % 3] = k_op_x(kl, 0, i + 2);
-      if constexpr (PV) va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
-      asm volatile("" ::: "memory");
+    const int j = i / SLOTS;  // MFMA j of each product: scores first, P.V after the slots' exps
+    if (i % SLOTS == 0) {
+      if (j + 2 < NM) {
+        ka[(j + 2) % 3] = k_op_x<D>(kl, 0, j + 2);
+        if constexpr (PV) va[(j + 2) % 3] = v_op_x<D>(vl, (j + 2) / ND, (j + 2) % ND);
+        asm volatile("" ::: "memory");
+      }
+      if (j == 0)
+        mfma_v0(sn, ka[0], q[0]);
+      else
+        mfma_v(sn, ka[j % 3], q[j]);
     }
-    if (i == 0)
-      mfma_v0(sn, ka[0], q[0]);
-    else
-      mfma_v(sn, ka[i % 3], q[i]);
     pw[i >> 2][i & 3] = POOLED ? exp_pair_f32sum(sc[2 * i], sc[2 * i + 1], c, neg, psum)
                                : exp_pair(sc[2 * i], sc[2 * i + 1], c, neg, psum);
     if constexpr (PV) {
-      if (i == 0)
-        mfma_v_first(st.acc[0], va[0], pp[0]);
-      else if (i == 7)
-        mfma_v_tie(st.acc[3], va[1], pp[1], sn);  // va[7 % 3]
-      else
-        mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
+      if (i % SLOTS == SLOTS - 1) {
+        if (j == 0)
+          mfma_v_first(st.acc[0], va[0], pp[0]);
+        else if (j == NM - 1)
+          mfma_v_tie(st.acc[ND - 1], va[j % 3], pp[1], sn);
+        else
+          mfma_v(st.acc[j % ND], va[j % 3], pp[j / ND]);
+      }
     }
     if (i == 0) __builtin_amdgcn_s_setprio(1);
   }
@@ -136,8 +144,8 @@ __device__ __forceinline__ void half_step(SoftmaxState& st, const f32x16& sc, f3
 // three-stage step over whole tiles, double buffered in 64 KiB, with plain
 // pooled tiles: 32760 tokens 2370 -> 2325 us, 75600 tokens 21.2 -> 21.0 ms; four
 // half buffers with copies two steps ahead were slower (2400 us).
-template <int BLK>
-__global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))
+template <int BLK, int D>
+__global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2)))
 fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
                 const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_t, int64_t sk_h,
                 const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
@@ -145,8 +153,9 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
                 const int32_t* __restrict__ counts, const uint32_t* __restrict__ mask, int T, int H, int NT, int W, float c,
                 uint16_t* __restrict__ o, int64_t so_b, int64_t so_t, int64_t so_h) {
   constexpr int NTHREADS = BLK * 2;
-  __shared__ __align__(256) uint16_t kbuf[kTileElems];
-  __shared__ __align__(256) uint16_t vbuf[kTileElems];
+  constexpr uint32_t kHalfBytes = kKeys * D;  // half a tile: 32 rows of 2 D bytes
+  __shared__ __align__(256) uint16_t kbuf[kKeys * D];
+  __shared__ __align__(256) uint16_t vbuf[kKeys * D];
   __shared__ TileList tl;
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -166,28 +175,28 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
   const int npipe = ntiles - nplain;
 
   const KVSource src{k + b * sk_b + h * sk_h, sk_t, v + b * sv_b + h * sv_h, sv_t,
-                     kc + (static_cast<int64_t>(b) * npad * H + h) * kD,
-                     static_cast<int64_t>(H) * kD, vc + (static_cast<int64_t>(b) * npad * H + h) * kD};
-  CopyOffsets<NTHREADS> off;
+                     kc + (static_cast<int64_t>(b) * npad * H + h) * D,
+                     static_cast<int64_t>(H) * D, vc + (static_cast<int64_t>(b) * npad * H + h) * D};
+  CopyOffsets<NTHREADS, D> off;
   off.init(sk_t, sv_t);
   const uint32_t kb = lds_addr(kbuf), vb = lds_addr(vbuf);  // LDS byte addresses
-  const uint32_t kl = k_lane(kb, col, half), vl = v_lane(vb, lane);  // this lane's operands
+  const uint32_t kl = k_lane<D>(kb, col, half), vl = v_lane<D>(vb, lane);  // this lane's operands
   // Half hh of pipelined tile t (pooled tiles, then the full exact tiles) into
   // K or V half buffer hh.
   const auto first_of = [&](int t) { return exact_first<BLK>(tl, max(t - npool, 0)); };
   const auto issue_k_at = [&](int first, int hh) {
-    issue_half<NTHREADS>(kb + hh * kHalfBytes, src.k + static_cast<int64_t>(first + 32 * hh) * src.sk,
+    issue_half<NTHREADS, D>(kb + hh * kHalfBytes, src.k + static_cast<int64_t>(first + 32 * hh) * src.sk,
                          src.sk, off.k);
   };
   const auto issue_v_at = [&](int first, int hh) {
-    issue_half<NTHREADS>(vb + hh * kHalfBytes, src.v + static_cast<int64_t>(first + 32 * hh) * src.sv,
+    issue_half<NTHREADS, D>(vb + hh * kHalfBytes, src.v + static_cast<int64_t>(first + 32 * hh) * src.sv,
                          src.sv, off.v);
   };
   const auto issue_any = [&](int t, int kv, int hh) {
     if (t >= npool) {
       if (kv == 0) issue_k_at(first_of(t), hh); else issue_v_at(first_of(t), hh);
     } else {
-      issue_generic_half<NTHREADS>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, t, NT), hh, src);
+      issue_generic_half<NTHREADS, D>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, t, NT), hh, src);
     }
   };
   const auto issue_start = [&] {  // what the first half steps need
@@ -199,8 +208,8 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     return rag ? exact_desc<BLK>(tl, tl.nexact - 1, T, NT) : pooled_desc(tl, tl.npool - 1, NT);
   };
   if (nplain) {
-    issue_generic<NTHREADS>(kb, 0, plain_desc(), src);
-    issue_generic<NTHREADS>(vb, 1, plain_desc(), src);
+    issue_generic<NTHREADS, D>(kb, 0, plain_desc(), src);
+    issue_generic<NTHREADS, D>(vb, 1, plain_desc(), src);
   } else {
     issue_start();
   }
@@ -208,15 +217,15 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
   // This wave's 32 query rows as the B operand of S^T = K Q^T (rows past T
   // repeat row T - 1 and are not stored).
   const int qrow = qb * BLK + wave * 32 + col;
-  bf16x8 qreg[8];
+  bf16x8 qreg[D / 16];
   {
     const uint16_t* qp = q + b * sq_b + static_cast<int64_t>(min(qrow, T - 1)) * sq_t + h * sq_h + half * 8;
 #pragma unroll
-    for (int cc = 0; cc < 8; ++cc)
+    for (int cc = 0; cc < D / 16; ++cc)
       qreg[cc] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + cc * 16));
   }
 
-  SoftmaxState st;
+  SoftmaxStateOf<D / 32> st;
   st.init();
 
   // ---- the short last block's tile
@@ -224,7 +233,7 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     wait_tile_copies();
     __syncthreads();
     f32x16 s[2];
-    qk_tile(kl, qreg, s);
+    qk_tile<D>(kl, qreg, s);
     finish_tile<BLK>(st, s, vl, plain_desc(), c, lane, NT, T);
     __syncthreads();  // every wave is done with K and V
     if (npipe > 0) issue_start();
@@ -243,7 +252,7 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     {
       const f32x16 zero = {};
 #pragma unroll
-      for (int cc = 0; cc < 8; ++cc) sa = mfma_bf16(k_op_x(kl, 0, cc), qreg[cc], cc == 0 ? zero : sa);
+      for (int cc = 0; cc < D / 16; ++cc) sa = mfma_bf16(k_op_x<D>(kl, 0, cc), qreg[cc], cc == 0 ? zero : sa);
     }
     mfma_fence(sa);   // the steps read the scores through asm
     __syncthreads();  // every wave is done with K(0)
@@ -258,23 +267,23 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     if (npool > 0) {
       issue_any(min(1, last), 0, 0);
       mask_scores(sa, static_cast<uint32_t>(tl.pmask[0]));
-      half_step<BLK, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
+      half_step<BLK, D, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
       land();
       issue_any(min(1, last), 0, 1);
       issue_any(0, 1, 1);
       mask_scores(sb, static_cast<uint32_t>(tl.pmask[0] >> 32));
-      half_step<BLK, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      half_step<BLK, D, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
       land();
       for (t = 1; t < npool; ++t) {
         issue_any(min(t + 1, last), 0, 0);
         issue_any(t, 1, 0);
         mask_scores(sa, static_cast<uint32_t>(tl.pmask[t]));
-        half_step<BLK, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
+        half_step<BLK, D, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
         land();
         issue_any(min(t + 1, last), 0, 1);
         issue_any(t, 1, 1);
         mask_scores(sb, static_cast<uint32_t>(tl.pmask[t] >> 32));
-        half_step<BLK, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+        half_step<BLK, D, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
         land();
       }
     }
@@ -283,11 +292,11 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     int f0 = first_of(min(t, last)), f1 = first_of(min(t + 1, last));
     if (npool == 0) {
       issue_k_at(f1, 0);
-      half_step<BLK, false, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
+      half_step<BLK, D, false, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
       land();
       issue_k_at(f1, 1);
       issue_v_at(f0, 1);
-      half_step<BLK, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      half_step<BLK, D, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
       f0 = f1;
       f1 = first_of(min(2, last));
       land();
@@ -296,13 +305,13 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     for (; t < npipe; ++t) {
       issue_k_at(f1, 0);
       issue_v_at(f0, 0);
-      half_step<BLK, false, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
+      half_step<BLK, D, false, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
       asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
       const int f2 = first_of(min(t + 2, last));
       land();
       issue_k_at(f1, 1);
       issue_v_at(f0, 1);
-      half_step<BLK, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
+      half_step<BLK, D, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
       land();
       f0 = f1;
       f1 = f2;
@@ -310,8 +319,10 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     // P.V of the last half tile
     mfma_fence(st.acc);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      st.acc[i & 3] = mfma_bf16(v_op_x(vl1, i >> 2, i & 3), pb[i >> 2], st.acc[i & 3]);
+    for (int i = 0; i < D / 16; ++i) {
+      const int ks = i / (D / 32), dt = i % (D / 32);
+      st.acc[dt] = mfma_bf16(v_op_x<D>(vl1, ks, dt), pb[ks], st.acc[dt]);
+    }
   }
   wait_tile_copies();
 
@@ -323,6 +334,32 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
 
 using namespace solattn;
 
+namespace solattn {
+
+int fwd_bf16(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
+             int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b, int64_t sv_t,
+             int64_t sv_h, const uint16_t* kc, const uint16_t* vc, int64_t npad, const int32_t* counts,
+             const uint32_t* mask, int64_t B, int64_t T, int64_t H, int64_t D, int64_t block,
+             float scale, uint16_t* o, int64_t so_b, int64_t so_t, int64_t so_h, hipStream_t s) {
+  SOLATTN_REQUIRE(D == 64 || D == kD, SOLATTN_EUNSUPPORTED, "fwd_bf16: head_dim %lld", (long long)D);
+  if (int rc = check_fwd_args(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc,
+                              vc, npad, counts, mask, B, T, H, block, o, so_b, so_t, so_h, "fwd_bf16"))
+    return rc;
+  const int64_t NT = cdiv(T, block);
+  const int W = static_cast<int>(cdiv(NT, 32));
+  const float c = scale * kLog2e;
+  const uint32_t grid = static_cast<uint32_t>(B * H * NT);
+  const auto kern = D == 64 ? (block == 128 ? bf16fwd::fwd_bf16_kernel<128, 64> : bf16fwd::fwd_bf16_kernel<64, 64>)
+                            : (block == 128 ? bf16fwd::fwd_bf16_kernel<128, 128> : bf16fwd::fwd_bf16_kernel<64, 128>);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(static_cast<uint32_t>(block) * 2), blist_lds_bytes(NT), s, q,
+                     sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc, vc, npad, counts,
+                     mask, static_cast<int>(T), static_cast<int>(H), static_cast<int>(NT), W, c, o, so_b,
+                     so_t, so_h);
+  return check_launch("fwd_bf16");
+}
+
+}  // namespace solattn
+
 extern "C" int solattn_fwd_bf16(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
                                 const uint16_t* k, int64_t sk_b, int64_t sk_t, int64_t sk_h,
                                 const uint16_t* v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
@@ -331,19 +368,7 @@ extern "C" int solattn_fwd_bf16(const uint16_t* q, int64_t sq_b, int64_t sq_t, i
                                 int64_t block, float scale, uint16_t* o, int64_t so_b,
                                 int64_t so_t, int64_t so_h, solattn_stream_t stream) {
   clear_error();
-  if (int rc = check_fwd_args(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc,
-                              vc, npad, counts, mask, B, T, H, D, block, o, so_b, so_t,
-                              so_h, "fwd_bf16"))
-    return rc;
-  const int64_t NT = cdiv(T, block);
-  const int W = static_cast<int>(cdiv(NT, 32));
-  const float c = scale * kLog2e;
-  const uint32_t grid = static_cast<uint32_t>(B * H * NT);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(block == 128 ? bf16fwd::fwd_bf16_kernel<128> : bf16fwd::fwd_bf16_kernel<64>,
-                     dim3(grid), dim3(static_cast<uint32_t>(block) * 2), blist_lds_bytes(NT), s, q, sq_b,
-                     sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc, vc, npad, counts, mask,
-                     static_cast<int>(T), static_cast<int>(H), static_cast<int>(NT), W, c, o, so_b, so_t,
-                     so_h);
-  return check_launch("fwd_bf16");
+  SOLATTN_REQUIRE(D == kD, SOLATTN_EUNSUPPORTED, "fwd_bf16: head_dim %lld != 128", (long long)D);
+  return fwd_bf16(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, kc, vc, npad, counts,
+                  mask, B, T, H, D, block, scale, o, so_b, so_t, so_h, reinterpret_cast<hipStream_t>(stream));
 }

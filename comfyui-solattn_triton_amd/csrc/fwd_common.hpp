@@ -18,7 +18,7 @@
 namespace solattn {
 
 constexpr int kKeys = 64;             // keys per tile
-constexpr int kD = 128;               // head dim
+constexpr int kD = 128;               // head dim (the BF16 forward also has a 64-channel form)
 constexpr int kMaxNT = 16384;         // query/key blocks per head
 constexpr int kMaxPool = kMaxNT / 64; // pooled tiles per query block
 constexpr float kMaxSlack = 8.f;      // lazy running max (log2 units)
@@ -229,11 +229,20 @@ __device__ __forceinline__ int exact_first(const TileList& tl, int e) {
 //      lanes = 16 rows of one chunk per cycle, all in different chunks;
 //   V: physical chunk = chunk ^ 4*(row & 3): a ds_read_b64_tr_b16 serves 32
 //      lanes = 4 rows x 4 consecutive chunks per cycle, all distinct.
+// At 64 channels a row is 128 bytes, so two rows make a bank sweep and the row's
+// parity already picks a half: the same rules on row >> 1.
 constexpr int kTileElems = kKeys * kD;  // one K or V tile in LDS (16 KiB)
 constexpr uint32_t kTileBytes = kTileElems * 2;
 
-__device__ __forceinline__ int swz_k(int row, int chunk) { return chunk ^ (row & 15); }
-__device__ __forceinline__ int swz_v(int row, int chunk) { return chunk ^ ((row & 3) << 2); }
+template <int D = kD>
+__device__ __forceinline__ int swz_k(int row, int chunk) {
+  static_assert(D == 64 || D == 128, "head dims of the tiles");
+  return chunk ^ (D == 128 ? (row & 15) : ((row >> 1) & 7));
+}
+template <int D = kD>
+__device__ __forceinline__ int swz_v(int row, int chunk) {
+  return chunk ^ (D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2);
+}
 
 // Global -> LDS copies (global_load_lds_*): lane i's bytes land at
 // lds + size * i, with lds a wave-uniform LDS byte address (M0). They are
@@ -280,39 +289,42 @@ __device__ __forceinline__ void wait_vmcnt() {
 // tile, each lane computing its own source rows: rows past nvalid re-read row
 // 0 of the tile (finite data that the softmax masks out). U copies per lane.
 // dst is the tile's LDS byte address.
-template <int NTHREADS>
+template <int NTHREADS, int D = kD>
 __device__ __forceinline__ void issue_generic(uint32_t dst, int kv, const TileDesc& td,
                                               const KVSource& src) {
-  constexpr int U = kKeys * 16 / NTHREADS;
+  constexpr int C = D / 8, U = kKeys * C / NTHREADS;
   const uint32_t l0 = dst + wave_id() * 64 * 16;
   const uint16_t* b = kv == 0 ? (td.pooled ? src.kc : src.k) : (td.pooled ? src.vc : src.v);
   const int64_t stride = td.pooled ? src.skc : (kv == 0 ? src.sk : src.sv);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int e = threadIdx.x + NTHREADS * u;
-    const int row = e >> 4, pc = e & 15;
+    const int row = e / C, pc = e % C;
     const int srow = td.first + (row < td.nvalid ? row : 0);
-    const int chunk = kv == 0 ? swz_k(row, pc) : swz_v(row, pc);
+    const int chunk = kv == 0 ? swz_k<D>(row, pc) : swz_v<D>(row, pc);
     g2l16(b + static_cast<int64_t>(srow) * stride + chunk * 8, l0 + NTHREADS * u * 16);
   }
 }
 
 // Per-lane byte offsets of the 16-byte chunks this lane copies into a full
-// bf16 K or V tile. Copy u covers rows (NTHREADS/16)u ..; lanes repeat their
-// swizzle every P copies (P = 256 / NTHREADS), so the offset of copy u is
-// off[u % P] + (u / P) * 16 * row stride, the second term wave-uniform.
-template <int NTHREADS>
+// bf16 K or V tile. A copy covers kRows rows; lanes repeat their swizzle every
+// P copies (16 rows), so the offset of copy u is off[u % P] + (u / P) * P *
+// kRows * row stride, the second term wave-uniform.
+template <int NTHREADS, int D = kD>
 struct CopyOffsets {
-  static constexpr int U = kKeys * 16 / NTHREADS;  // copies per lane per K or V tile
-  static constexpr int P = 256 / NTHREADS;
+  static constexpr int C = D / 8;                 // chunks per row
+  static constexpr int kRows = NTHREADS / C;      // rows per copy
+  static constexpr int U = kKeys / kRows;         // copies per lane per K or V tile
+  static constexpr int P = kRows < 16 ? 16 / kRows : 1;
+  static constexpr int kStep = P * kRows;         // rows per P copies
   uint32_t k[P], v[P];
   __device__ __forceinline__ void init(int64_t sk, int64_t sv) {
 #pragma unroll
     for (int u = 0; u < P; ++u) {
       const int e = threadIdx.x + NTHREADS * u;
-      const int row = e >> 4, pc = e & 15;
-      k[u] = static_cast<uint32_t>((row * sk + swz_k(row, pc) * 8) * 2);
-      v[u] = static_cast<uint32_t>((row * sv + swz_v(row, pc) * 8) * 2);
+      const int row = e / C, pc = e % C;
+      k[u] = static_cast<uint32_t>((row * sk + swz_k<D>(row, pc) * 8) * 2);
+      v[u] = static_cast<uint32_t>((row * sv + swz_v<D>(row, pc) * 8) * 2);
     }
   }
 };
@@ -327,39 +339,38 @@ __device__ __forceinline__ void issue_full(uint32_t dst, const uint16_t* base, i
   const char* b = reinterpret_cast<const char*>(base);
 #pragma unroll
   for (int u = 0; u < CO::U; ++u) {
-    const char* row_base = b + static_cast<int64_t>(u / CO::P) * 16 * stride * 2;
+    const char* row_base = b + static_cast<int64_t>(u / CO::P) * CO::kStep * stride * 2;
     g2l16_s(row_base, off[u % CO::P], l0 + NTHREADS * u * 16);
   }
 }
 
 // The same for half a tile (32 keys): rows [32 hh, 32 hh + 32) of the tile `td`
 // (issue_generic_half) or a base at the half's first row (issue_half).
-constexpr uint32_t kHalfBytes = kTileBytes / 2;
-template <int NTHREADS>
+template <int NTHREADS, int D>
 __device__ __forceinline__ void issue_generic_half(uint32_t dst, int kv, const TileDesc& td, int hh,
                                                    const KVSource& src) {
-  constexpr int U = CopyOffsets<NTHREADS>::U / 2;
+  constexpr int C = D / 8, U = CopyOffsets<NTHREADS, D>::U / 2;
   const uint32_t l0 = dst + wave_id() * 64 * 16;
   const uint16_t* b = kv == 0 ? (td.pooled ? src.kc : src.k) : (td.pooled ? src.vc : src.v);
   const int64_t stride = td.pooled ? src.skc : (kv == 0 ? src.sk : src.sv);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int e = threadIdx.x + NTHREADS * u;
-    const int row = 32 * hh + (e >> 4), pc = e & 15;
+    const int row = 32 * hh + e / C, pc = e % C;
     const int srow = td.first + (row < td.nvalid ? row : 0);
-    const int chunk = kv == 0 ? swz_k(row, pc) : swz_v(row, pc);
+    const int chunk = kv == 0 ? swz_k<D>(row, pc) : swz_v<D>(row, pc);
     g2l16(b + static_cast<int64_t>(srow) * stride + chunk * 8, l0 + NTHREADS * u * 16);
   }
 }
-template <int NTHREADS>
+template <int NTHREADS, int D>
 __device__ __forceinline__ void issue_half(uint32_t dst, const uint16_t* base, int64_t stride,
-                                           const uint32_t (&off)[CopyOffsets<NTHREADS>::P]) {
-  using CO = CopyOffsets<NTHREADS>;
+                                           const uint32_t (&off)[CopyOffsets<NTHREADS, D>::P]) {
+  using CO = CopyOffsets<NTHREADS, D>;
   const uint32_t l0 = dst + wave_id() * 64 * 16;
   const char* b = reinterpret_cast<const char*>(base);
 #pragma unroll
   for (int u = 0; u < CO::U / 2; ++u) {
-    const char* row_base = b + static_cast<int64_t>(u / CO::P) * 16 * stride * 2;
+    const char* row_base = b + static_cast<int64_t>(u / CO::P) * CO::kStep * stride * 2;
     g2l16_s(row_base, off[u % CO::P], l0 + NTHREADS * u * 16);
   }
 }
@@ -400,32 +411,36 @@ __device__ __forceinline__ bf16x8 v_op(const uint16_t* vt, int ks, int dt, int l
 }
 
 // Operand addressing by XOR. In a 256-byte-aligned K tile the operand (m, cc)
-// of a lane sits at (k_lane ^ (cc << 5)) + m * 8192, because the swizzle
-// c ^ (row & 15) only flips chunk bits that cc's chunk index 2cc + half
-// shares with bits 5-7 of the address. In a V tile the transposed operand
-// (ks, dt) rows row0 / row0 + 8 sit at (v_lane ^ (dt << 6)) + ks * 4096 and
-// 2048 further (swizzle c ^ ((row & 3) << 2) flips address bits 6-7). One
-// lane address per tile replaces one per (cc) or (dt).
+// of a lane sits at (k_lane ^ (cc << 5)) + 32 m rows, because the swizzle
+// c ^ (row & 15) (64 channels: c ^ (row >> 1 & 7)) only flips chunk bits that
+// cc's chunk index 2cc + half shares with bits 5-7 of the address. In a V tile
+// the transposed operand (ks, dt) rows row0 / row0 + 8 sit at (v_lane ^ (dt <<
+// 6)) + 16 ks rows and 8 rows further (the swizzle flips address bits 6-7, at 64
+// channels bit 6). One lane address per tile replaces one per (cc) or (dt).
+template <int D = kD>
 __device__ __forceinline__ uint32_t k_lane(uint32_t tile, int col, int half) {
-  return tile + col * 256 + 16 * (half ^ (col & 15));
+  return tile + col * (2 * D) + 16 * swz_k<D>(col, half);
 }
+template <int D = kD>
 __device__ __forceinline__ uint32_t v_lane(uint32_t tile, int lane) {
   const int g = lane >> 4, sl = lane & 15;
   const int row0 = 4 * (g >> 1) + (sl >> 2);
   const int cp = 2 * (g & 1) + ((sl & 3) >> 1);
-  return tile + row0 * 256 + 64 * (row0 & 3) + 16 * cp + 8 * (sl & 1);
+  return tile + row0 * (2 * D) + 16 * swz_v<D>(row0, cp) + 8 * (sl & 1);
 }
+template <int D = kD>
 __device__ __forceinline__ bf16x8 k_op_x(uint32_t kl, int m, int cc) {
-  const uint32_t a = (kl ^ static_cast<uint32_t>(cc << 5)) + m * 8192;
+  const uint32_t a = (kl ^ static_cast<uint32_t>(cc << 5)) + m * (64 * D);
   return *reinterpret_cast<const __attribute__((address_space(3))) bf16x8*>(static_cast<uintptr_t>(a));
 }
+template <int D = kD>
 __device__ __forceinline__ bf16x8 v_op_x(uint32_t vl, int ks, int dt) {
   typedef short v4i16 __attribute__((ext_vector_type(4)));
-  const uint32_t a = (vl ^ static_cast<uint32_t>(dt << 6)) + ks * 4096;
+  const uint32_t a = (vl ^ static_cast<uint32_t>(dt << 6)) + ks * (32 * D);
   const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       reinterpret_cast<__attribute__((address_space(3))) v4i16*>(static_cast<uintptr_t>(a)));
   const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      reinterpret_cast<__attribute__((address_space(3))) v4i16*>(static_cast<uintptr_t>(a + 2048)));
+      reinterpret_cast<__attribute__((address_space(3))) v4i16*>(static_cast<uintptr_t>(a + 16 * D)));
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
@@ -441,32 +456,32 @@ __device__ __forceinline__ void qk_tile(const uint16_t* kt, const bf16x8 (&q)[8]
   }
 }
 
-// O^T += V^T . P^T over the tile's 16 (key step, channel tile) operands, each
-// read three operands ahead of its MFMA.
 // The same from the lane address kl = k_lane(tile, col, half) of a
 // 256-byte-aligned K tile: no per-chunk addresses to keep live.
-__device__ __forceinline__ void qk_tile(uint32_t kl, const bf16x8 (&q)[8], f32x16 (&s)[2]) {
+template <int D>
+__device__ __forceinline__ void qk_tile(uint32_t kl, const bf16x8 (&q)[D / 16], f32x16 (&s)[2]) {
   const f32x16 zero = {};
 #pragma unroll
-  for (int cc = 0; cc < 8; ++cc) {
-    const bf16x8 a0 = k_op_x(kl, 0, cc);
-    const bf16x8 a1 = k_op_x(kl, 1, cc);
+  for (int cc = 0; cc < D / 16; ++cc) {
+    const bf16x8 a0 = k_op_x<D>(kl, 0, cc);
+    const bf16x8 a1 = k_op_x<D>(kl, 1, cc);
     s[0] = mfma_bf16(a0, q[cc], cc == 0 ? zero : s[0]);
     s[1] = mfma_bf16(a1, q[cc], cc == 0 ? zero : s[1]);
   }
 }
 
-// O^T += V^T . P^T over one tile; vop(ks, dt) gives the V^T operand.
-template <typename VOp>
-__device__ __forceinline__ void pv_tile_with(VOp&& vop, const bf16x8 (&pb)[4], f32x16 (&o)[4]) {
-  constexpr int L = 3;
-  bf16x8 va[16];
+// O^T += V^T . P^T over one tile's (key step, channel tile) operands, each read
+// three operands ahead of its MFMA; vop(ks, dt) gives the V^T operand.
+template <int ND, typename VOp>
+__device__ __forceinline__ void pv_tile_with(VOp&& vop, const bf16x8 (&pb)[4], f32x16 (&o)[ND]) {
+  constexpr int L = 3, N = 4 * ND;
+  bf16x8 va[N];
 #pragma unroll
-  for (int i = 0; i < L; ++i) va[i] = vop(i >> 2, i & 3);
+  for (int i = 0; i < L; ++i) va[i] = vop(i / ND, i % ND);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + L < 16) va[i + L] = vop((i + L) >> 2, (i + L) & 3);
-    o[i & 3] = mfma_bf16(va[i], pb[i >> 2], o[i & 3]);
+  for (int i = 0; i < N; ++i) {
+    if (i + L < N) va[i + L] = vop((i + L) / ND, (i + L) % ND);
+    o[i % ND] = mfma_bf16(va[i], pb[i / ND], o[i % ND]);
   }
 }
 __device__ __forceinline__ void pv_tile(const uint16_t* vt, const bf16x8 (&pb)[4], int lane,
@@ -474,9 +489,10 @@ __device__ __forceinline__ void pv_tile(const uint16_t* vt, const bf16x8 (&pb)[4
   pv_tile_with([&](int ks, int dt) { return v_op(vt, ks, dt, lane); }, pb, o);
 }
 // From the lane address vl = v_lane(tile, lane) of a 256-byte-aligned V tile.
+template <int ND>
 __device__ __forceinline__ void pv_tile(uint32_t vl, const bf16x8 (&pb)[4], int /*lane*/,
-                                        f32x16 (&o)[4]) {
-  pv_tile_with([&](int ks, int dt) { return v_op_x(vl, ks, dt); }, pb, o);
+                                        f32x16 (&o)[ND]) {
+  pv_tile_with([&](int ks, int dt) { return v_op_x<32 * ND>(vl, ks, dt); }, pb, o);
 }
 
 // ------------------------------------------- hand-ordered MFMA / softmax stream
@@ -516,7 +532,7 @@ __device__ __forceinline__ void mfma_fence(f32x16& x) {
 }
 template <int N>
 __device__ __forceinline__ void mfma_fence(f32x16 (&x)[N]) {
-  static_assert(N == 2 || N == 4, "fence sizes");
+  static_assert(N == 2 || N == 4, "fence sizes");  // (two scores or O tiles, four O tiles)
   if constexpr (N == 2)
     asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0]), "+v"(x[1]));
   else
@@ -563,19 +579,21 @@ __device__ __forceinline__ uint32_t exp_pair_f32sum(float s0, float s1, float c,
   return p;
 }
 // ------------------------------------------------------------ online softmax
-struct SoftmaxState {
+template <int ND>  // channel tiles: head dim / 32
+struct SoftmaxStateOf {
   float m;          // running max, in the exp2 domain (score * c)
   float l;          // partial row sum over this lane's keys
-  f32x16 acc[4];    // O^T: channel 32dt + 8(r/4) + 4*half + (r%4), query row `col`
+  f32x16 acc[ND];   // O^T: channel 32dt + 8(r/4) + 4*half + (r%4), query row `col`
   __device__ __forceinline__ void init() {
     m = -INFINITY;
     l = 0.f;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
   }
 };
+using SoftmaxState = SoftmaxStateOf<kD / 32>;
 
 // x combined with the value of the lane 32 apart (one v_permlane32_swap).
 __device__ __forceinline__ float xhalf_max(float x) {
@@ -614,10 +632,11 @@ __device__ __forceinline__ float exp8(const f32x16& s, float c, float neg, bf16x
   return sum;
 }
 
-__device__ __forceinline__ void rescale(SoftmaxState& st, float alpha) {
+template <int ND>
+__device__ __forceinline__ void rescale(SoftmaxStateOf<ND>& st, float alpha) {
   if (__any(alpha != 1.f)) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) st.acc[dt][r] *= alpha;
   }
@@ -651,8 +670,8 @@ __device__ __forceinline__ void mask_scores(f32x16 (&s)[2], uint64_t amask) {
 // pipelined path).
 // vt: the V tile, as a pointer or as the lane address v_lane(tile, lane) of a
 // 256-byte-aligned tile (see pv_tile).
-template <int BLK, typename VTile>
-__device__ __forceinline__ void finish_tile(SoftmaxState& st, f32x16 (&s)[2], VTile vt,
+template <int BLK, int ND, typename VTile>
+__device__ __forceinline__ void finish_tile(SoftmaxStateOf<ND>& st, f32x16 (&s)[2], VTile vt,
                                             const TileDesc& td, float c, int lane, int NT, int T) {
   const int half = lane >> 5;
   mask_scores(s, td.amask);
@@ -704,14 +723,15 @@ __device__ __forceinline__ void finish_tile(SoftmaxState& st, f32x16 (&s)[2], VT
 // value) made the epilogue 2.5 us of every workgroup's life, 3.3 us beside
 // other workgroups: calls of 1000 / 4096 / 32760 tokens at block 64 went from
 // 34.9 / 100.5 / 2954 to 33.0 / 97.0 / 2930 us, same bits.
-__device__ __forceinline__ void store_rows(const SoftmaxState& st, uint16_t* __restrict__ obase,
+template <int ND>
+__device__ __forceinline__ void store_rows(const SoftmaxStateOf<ND>& st, uint16_t* __restrict__ obase,
                                            int64_t so_t, int qrow, int T, int half) {
   const float inv = 1.f / xhalf_sum(st.l);
   if (qrow >= T) return;
   uint16_t* orow = obase + static_cast<int64_t>(qrow) * so_t;
   // the two lanes of a row swap halves so each writes 16 contiguous bytes
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
+  for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
     for (int ip = 0; ip < 2; ++ip) {
       uint32_t w[2][2];
@@ -737,9 +757,8 @@ __device__ __forceinline__ void store_rows(const SoftmaxState& st, uint16_t* __r
 inline int check_fwd_common(const void* q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
                             const void* kc, const void* vc, int64_t npad, const int32_t* counts,
                             const uint32_t* mask, int64_t B, int64_t T,
-                            int64_t H, int64_t D, int64_t block, const void* o, int64_t so_b,
+                            int64_t H, int64_t block, const void* o, int64_t so_b,
                             int64_t so_t, int64_t so_h, const char* what) {
-  SOLATTN_REQUIRE(D == kD, SOLATTN_EUNSUPPORTED, "%s: head_dim %lld != 128", what, (long long)D);
   SOLATTN_REQUIRE(block == 64 || block == 128, SOLATTN_EUNSUPPORTED, "%s: block %lld not in {64, 128}",
                   what, (long long)block);
   SOLATTN_REQUIRE(B > 0 && T > 0 && H > 0, SOLATTN_EINVAL, "%s: bad sizes", what);
@@ -766,10 +785,10 @@ inline int check_fwd_args(const void* q, int64_t sq_b, int64_t sq_t, int64_t sq_
                           int64_t sk_b, int64_t sk_t, int64_t sk_h, const void* v, int64_t sv_b,
                           int64_t sv_t, int64_t sv_h, const void* kc, const void* vc, int64_t npad,
                           const int32_t* counts, const uint32_t* mask,
-                          int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, const void* o,
+                          int64_t B, int64_t T, int64_t H, int64_t block, const void* o,
                           int64_t so_b, int64_t so_t, int64_t so_h, const char* what) {
-  if (int rc = check_fwd_common(q, sq_b, sq_t, sq_h, kc, vc, npad, counts, mask, B, T, H, D,
-                                block, o, so_b, so_t, so_h, what))
+  if (int rc = check_fwd_common(q, sq_b, sq_t, sq_h, kc, vc, npad, counts, mask, B, T, H, block, o,
+                                so_b, so_t, so_h, what))
     return rc;
   SOLATTN_REQUIRE(k && v, SOLATTN_EINVAL, "%s: null k/v", what);
   // Lane offsets within a 64-row tile are kept in 32 bits.

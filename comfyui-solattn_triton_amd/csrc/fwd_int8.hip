@@ -1378,8 +1378,9 @@ int fwd_int8(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const 
              int64_t T, int64_t H, int64_t D, int64_t block, float scale, int int8_pv,
              uint16_t* o, int64_t so_b, int64_t so_t, int64_t so_h, solattn_stream_t stream,
              bool uniform_ks, bool ks_head_major) {
-  if (int rc = check_fwd_common(q, sq_b, sq_t, sq_h, kc, vc, npad, counts, mask, B, T, H, D,
-                                block, o, so_b, so_t, so_h, "fwd_int8"))
+  SOLATTN_REQUIRE(D == kD, SOLATTN_EUNSUPPORTED, "fwd_int8: head_dim %lld != 128", (long long)D);
+  if (int rc = check_fwd_common(q, sq_b, sq_t, sq_h, kc, vc, npad, counts, mask, B, T, H, block, o,
+                                so_b, so_t, so_h, "fwd_int8"))
     return rc;
   SOLATTN_REQUIRE(TP >= T, SOLATTN_EINVAL, "fwd_int8: TP < T");
   SOLATTN_REQUIRE(int8_pv >= SOLATTN_PV_BF16 && int8_pv <= SOLATTN_PV_INT8_RUNNING, SOLATTN_EINVAL,

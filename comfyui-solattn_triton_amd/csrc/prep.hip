@@ -163,10 +163,22 @@ __device__ __forceinline__ void quant_span_rows_buf(const uint4 (&raw)[kSlotRows
   }
 }
 
+// load_span_buf for the lane's own head (64-channel heads): xl is a per-lane
+// address, rows past T re-read row T-1 (the pooling adds 0.0f for them).
+__device__ __forceinline__ void load_span_lane(const uint16_t* xl, int64_t st, int64_t r0, int64_t T,
+                                               int g, uint4 (&raw)[kSlotRows]) {
+#pragma unroll
+  for (int m = 0; m < kSlotRows; ++m)
+    raw[m] = *reinterpret_cast<const uint4*>(xl + min(r0 + g + 16 * m, T - 1) * st);
+}
+
 // QUANT: Q's rows come first and are quantised while K's and V's land, then
 // Q, K and V are pooled in that order; otherwise K, V, Q. AMAX: the per-block
-// |v| max (vamax_part).
-template <int BLK, bool QUANT, bool AMAX>
+// |v| max (vamax_part). HD: the head dim, 128 or 64. At 64 a workgroup covers
+// heads 2 blockIdx.x and 2 blockIdx.x + 1, eight lanes of each lane group a head
+// (the upper lanes of an odd last head repeat it and store nothing), so the
+// partials and their order are those of 128 channels.
+template <int BLK, bool QUANT, bool AMAX, int HD = kHeadDim>
 __global__ void __launch_bounds__(kPoolThreads)
 pool_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
             const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_t, int64_t sk_h,
@@ -177,45 +189,54 @@ pool_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t 
   constexpr int NB = kSpan / BLK;
   __shared__ __align__(16) float part[NB * kSlots * kHeadDim];
   __shared__ __align__(16) float amx[AMAX ? NB * kSlots * kHeadDim : 4];
-  const int h = blockIdx.x;
+  static_assert(HD == kHeadDim || (HD == 64 && !QUANT), "head dims of the pool");
+  constexpr int kHeads = kHeadDim / HD;  // heads per workgroup
+  const int h0 = blockIdx.x * kHeads;
   const int64_t b = blockIdx.z, r0 = static_cast<int64_t>(blockIdx.y) * kSpan;
   const PoolLane pl;
   uint4 rk[kSlotRows], rv[kSlotRows], rq[kSlotRows];
-  if (QUANT) load_span_buf(q + b * sq_b + h * sq_h, sq_t, r0, T, pl, rq);
-  load_span_buf(k + b * sk_b + h * sk_h, sk_t, r0, T, pl, rk);
-  load_span_buf(v + b * sv_b + h * sv_h, sv_t, r0, T, pl, rv);
-  if (!QUANT) load_span_buf(q + b * sq_b + h * sq_h, sq_t, r0, T, pl, rq);
-  // this thread's output: block s*NB + blk (if it exists), channel c
+  const auto load = [&](const uint16_t* x, int64_t sb, int64_t st, int64_t sh, uint4 (&raw)[kSlotRows]) {
+    if constexpr (HD == kHeadDim)
+      load_span_buf(x + b * sb + h0 * sh, st, r0, T, pl, raw);
+    else
+      load_span_lane(x + b * sb + min(h0 + pl.c8 / HD, H - 1) * sh + pl.c8 % HD, st, r0, T, pl.g, raw);
+  };
+  if (QUANT) load(q, sq_b, sq_t, sq_h, rq);
+  load(k, sk_b, sk_t, sk_h, rk);
+  load(v, sv_b, sv_t, sv_h, rv);
+  if (!QUANT) load(q, sq_b, sq_t, sq_h, rq);
+  // this thread's output: block s*NB + blk (if it exists), channel ch of head h
   const int blk = static_cast<int>(threadIdx.x) >> 7, c = static_cast<int>(threadIdx.x) & 127;
   const int j = static_cast<int>(blockIdx.y) * NB + blk;
-  const bool out = blk < NB && j < NT;
+  const int h = h0 + c / HD, ch = c % HD;
+  const bool out = blk < NB && j < NT && h < H;
   const float flen = static_cast<float>(min<int64_t>(BLK, T - static_cast<int64_t>(j) * BLK));
   const float* pc = part + blk * kSlots * kHeadDim + c;
   const auto pool_q = [&]() {
     pool_span<BLK, false>(rq, r0, T, pl, part, nullptr);
     __syncthreads();
-    if (out) qbar[((b * H + h) * NT + j) * kHeadDim + c] = tree16(pc, kHeadDim) / flen;
+    if (out) qbar[((b * H + h) * NT + j) * HD + ch] = tree16(pc, kHeadDim) / flen;
     __syncthreads();
   };
 
   if (QUANT) {
-    quant_span_rows_buf(rq, r0, T, pl, b, h, H, TP, qi, qs);
+    quant_span_rows_buf(rq, r0, T, pl, b, h0, H, TP, qi, qs);
     pool_q();
   }
   pool_span<BLK, false>(rk, r0, T, pl, part, nullptr);
   __syncthreads();
-  if (out) kc[((b * npad + j) * H + h) * kHeadDim + c] = f2bf(tree16(pc, kHeadDim) / flen);
+  if (out) kc[((b * npad + j) * H + h) * HD + ch] = f2bf(tree16(pc, kHeadDim) / flen);
   __syncthreads();
   pool_span<BLK, AMAX>(rv, r0, T, pl, part, amx);
   __syncthreads();
   if (out) {
-    vc[((b * npad + j) * H + h) * kHeadDim + c] = f2bf(tree16(pc, kHeadDim));
+    vc[((b * npad + j) * H + h) * HD + ch] = f2bf(tree16(pc, kHeadDim));
     if (AMAX) {
       const float* ac = amx + blk * kSlots * kHeadDim + c;
       float m = ac[0];
 #pragma unroll
       for (int g = 1; g < kSlots; ++g) m = fmaxf(m, ac[g * kHeadDim]);
-      vamax_part[((b * NT + j) * H + h) * kHeadDim + c] = m;
+      vamax_part[((b * NT + j) * H + h) * HD + ch] = m;
     }
   }
   if (!QUANT) {
@@ -246,7 +267,7 @@ __device__ __forceinline__ float tree8(const float (*part)[N], int d) {
 constexpr int kMomCh = 16;
 constexpr int kMomThreads = 8 * kMomCh;
 constexpr int kMomR = 32;
-template <bool CENTRE>
+template <bool CENTRE, int HD = kHeadDim>
 __global__ void __launch_bounds__(kMomThreads)
 moments_kernel(uint16_t* __restrict__ kc, int64_t npad, int NT, int H,
                float* __restrict__ kc_mean, float* __restrict__ kc_var,
@@ -262,12 +283,12 @@ moments_kernel(uint16_t* __restrict__ kc, int64_t npad, int NT, int H,
   // wave-uniform base at row r and the lane's row g + 8u, channel c at a
   // 32-bit offset (below 2^32 for H < 65536); rows past NT read 0.
   constexpr int kChunk = 8 * kMomR;
-  uint16_t* kch = kc + (static_cast<int64_t>(b) * npad * H + h) * kHeadDim;
-  const float* ah = vamax_part + (static_cast<int64_t>(b) * NT * H + h) * kHeadDim;
-  const int64_t sj = static_cast<int64_t>(H) * kHeadDim;
+  uint16_t* kch = kc + (static_cast<int64_t>(b) * npad * H + h) * HD;
+  const float* ah = vamax_part + (static_cast<int64_t>(b) * NT * H + h) * HD;
+  const int64_t sj = static_cast<int64_t>(H) * HD;
   const auto koff = [&](int u) { return static_cast<uint32_t>(((g + 8 * u) * sj + c) * 2); };
-  const auto kbytes = [&](int64_t r) { return rows_nbytes(r, NT, 2 * sj, 2 * kHeadDim, kChunk * 2 * sj); };
-  const auto abytes = [&](int64_t r) { return rows_nbytes(r, NT, 4 * sj, 4 * kHeadDim, kChunk * 4 * sj); };
+  const auto kbytes = [&](int64_t r) { return rows_nbytes(r, NT, 2 * sj, 2 * HD, kChunk * 2 * sj); };
+  const auto abytes = [&](int64_t r) { return rows_nbytes(r, NT, 4 * sj, 4 * HD, kChunk * 4 * sj); };
   const bool resident = NT <= kChunk;
   uint16_t w[kMomR];
   float s = 0.f, am = 0.f;
@@ -291,7 +312,7 @@ moments_kernel(uint16_t* __restrict__ kc, int64_t npad, int NT, int H,
   part[g][cl] = s;
   amx[g][cl] = am;
   __syncthreads();
-  const int64_t mo = (static_cast<int64_t>(b) * H + h) * kHeadDim + c;
+  const int64_t mo = (static_cast<int64_t>(b) * H + h) * HD + c;
   if (t < kMomCh) {
     const float mean = tree8(part, t) / fnt;
     smean[t] = mean;
@@ -625,7 +646,7 @@ constexpr int kMaxWords = 512;  // NT <= 16384 (the forwards' limit)
 // G > 1 serves short sequences (NT <= 128), whose rows would leave waves idle.
 // Against kc rows staged in LDS with two or four threads per row: 20.0 ->
 // 19.7 us at NT 256 and 63.0 -> 47.2 us at NT 512, same bits.
-template <int G>
+template <int G, int HD = kHeadDim>
 __global__ void __launch_bounds__(kRouteThreads)
 route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, int64_t npad,
              const float* __restrict__ kc_mean, const float* __restrict__ kc_var, int H, int NT,
@@ -636,21 +657,25 @@ route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, in
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   extern __shared__ __align__(16) uint32_t smask_lds[];
   const auto smask = [&](int i, int w) -> uint32_t& { return smask_lds[i * W + w]; };
-  __shared__ __align__(16) float sq[kQB][kHeadDim];  // the kQB query centroids
-  __shared__ __align__(16) float smk[kHeadDim];      // kc mean (mode 0)
-  __shared__ __align__(16) float svk[kHeadDim];      // kc variance
-  static_assert(kQB * kHeadDim / 4 == kRouteThreads && 2 * kHeadDim == kRouteThreads,
-                "one float4 of the centroids and one moment per thread");
+  __shared__ __align__(16) float sq[kQB][HD];  // the kQB query centroids
+  __shared__ __align__(16) float smk[HD];      // kc mean (mode 0)
+  __shared__ __align__(16) float svk[HD];      // kc variance
+  static_assert(kQB * HD / 4 <= kRouteThreads && 2 * HD <= kRouteThreads,
+                "at most one float4 of the centroids and one moment per thread");
   const int64_t bh = static_cast<int64_t>(b) * H + h;
   {
     // The centroids and moments, one load per thread. Query rows past NT (a
     // ragged last workgroup) read row NT-1; nothing of theirs is stored.
-    const int qb = t >> 5, q4 = t & 31;
-    const float4 x =
-        reinterpret_cast<const float4*>(qbar + (bh * NT + min(i0 + qb, NT - 1)) * kHeadDim)[q4];
-    const float mv = t < kHeadDim ? kc_mean[bh * kHeadDim + t] : kc_var[bh * kHeadDim + t - kHeadDim];
-    reinterpret_cast<float4*>(&sq[qb][0])[q4] = x;
-    (t < kHeadDim ? smk[t] : svk[t - kHeadDim]) = mv;
+    const int qb = t / (HD / 4), q4 = t % (HD / 4);
+    if (kQB * HD / 4 == kRouteThreads || qb < kQB) {
+      const float4 x =
+          reinterpret_cast<const float4*>(qbar + (bh * NT + min(i0 + qb, NT - 1)) * HD)[q4];
+      reinterpret_cast<float4*>(&sq[qb][0])[q4] = x;
+    }
+    if (2 * HD == kRouteThreads || t < 2 * HD) {
+      const float mv = t < HD ? kc_mean[bh * HD + t] : kc_var[bh * HD + t - HD];
+      (t < HD ? smk[t] : svk[t - HD]) = mv;
+    }
   }
   for (int e = t; e < kQB * W; e += kRouteThreads) smask_lds[e] = 0u;
   constexpr int R = kRouteThreads / G, kQG = kQB / G;  // rows per pass, query blocks per thread
@@ -659,11 +684,11 @@ route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, in
   const int ig = __builtin_amdgcn_readfirstlane(t / R) * kQG;  // the group's first query block
   const float* qrow[kQG];  // wave-uniform rows of the centroids
 #pragma unroll
-  for (int i = 0; i < kQG; ++i) qrow[i] = qbar + (bh * NT + min(i0 + ig + i, NT - 1)) * kHeadDim;
+  for (int i = 0; i < kQG; ++i) qrow[i] = qbar + (bh * NT + min(i0 + ig + i, NT - 1)) * HD;
   // kc rows through raw buffer loads: base at row j0 (wave-uniform), the lane's
   // row rr further; rows past NT read 0 (and are not active).
-  const uint16_t* kch = kc + (static_cast<int64_t>(b) * npad * H + h) * kHeadDim;
-  const int64_t sj = static_cast<int64_t>(H) * kHeadDim;
+  const uint16_t* kch = kc + (static_cast<int64_t>(b) * npad * H + h) * HD;
+  const int64_t sj = static_cast<int64_t>(H) * HD;
   const uint32_t roff = static_cast<uint32_t>(rr * sj * 2);
   __syncthreads();  // the centroids, moments and cleared mask words
   // Every wave computes the kQB thresholds (lane i: query block i0 + i), one
@@ -673,7 +698,7 @@ route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, in
     const float* qv = sq[min(lane, kQB - 1)];
     float mu = 0.f, var = 0.f;
 #pragma unroll 4
-    for (int d = 0; d < kHeadDim; d += 4) {
+    for (int d = 0; d < HD; d += 4) {
       const float4 x = *reinterpret_cast<const float4*>(qv + d);
       const float4 vk = *reinterpret_cast<const float4*>(svk + d);
       if (mode == 0) {
@@ -711,7 +736,7 @@ route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, in
     const int j = j0 + rr;
     const bool active = j < NT;
     const uint16_t* base = kch + j0 * sj;
-    const uint32_t nb = rows_nbytes(j0, NT, 2 * sj, 2 * kHeadDim, R * 2 * sj);
+    const uint32_t nb = rows_nbytes(j0, NT, 2 * sj, 2 * HD, R * 2 * sj);
     float acc[kQG];
 #pragma unroll
     for (int i = 0; i < kQG; ++i) acc[i] = 0.f;
@@ -719,11 +744,11 @@ route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, in
 #pragma unroll
     for (int u = 0; u < kChLoads; ++u) kn[u] = buffer_load16(base, nb, roff + 16 * u);
 #pragma unroll 1
-    for (int d0 = 0; d0 < kHeadDim; d0 += kCh) {
+    for (int d0 = 0; d0 < HD; d0 += kCh) {
       uint4 kr[kChLoads];
 #pragma unroll
       for (int u = 0; u < kChLoads; ++u) kr[u] = kn[u];
-      if (d0 + kCh < kHeadDim) {
+      if (d0 + kCh < HD) {
 #pragma unroll
         for (int u = 0; u < kChLoads; ++u)
           kn[u] = buffer_load16(base, nb, roff + 2 * (d0 + kCh) + 16 * u);
@@ -804,7 +829,7 @@ namespace solattn {
 
 int launch_pool(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
                 int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b,
-                int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t block,
+                int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t D, int64_t block,
                 uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar, float* vamax_part,
                 int8_t* qi, float* qs, int64_t TP, hipStream_t s) {
   const int64_t NT = cdiv(T, block);
@@ -819,10 +844,13 @@ int launch_pool(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, con
                   SOLATTN_EUNSUPPORTED, "pool: token strides must lie in [0, 2^26)");
   // heads fastest, so the workgroups in flight read whole token rows (all heads)
   // of neighbouring spans
-  dim3 grid(static_cast<uint32_t>(H), static_cast<uint32_t>(spans), static_cast<uint32_t>(B));
+  dim3 grid(static_cast<uint32_t>(cdiv(H * D, kHeadDim)), static_cast<uint32_t>(spans), static_cast<uint32_t>(B));
   const bool amax = vamax_part != nullptr;
+  SOLATTN_REQUIRE(D == kHeadDim || (!qi && !amax), SOLATTN_EUNSUPPORTED,
+                  "pool: head_dim %lld with quantisation", (long long)D);
   const auto kern =
-      block == 64
+      D == 64 ? (block == 64 ? pool_kernel<64, false, false, 64> : pool_kernel<128, false, false, 64>)
+      : block == 64
           ? (qi ? (amax ? pool_kernel<64, true, true> : pool_kernel<64, true, false>)
                 : (amax ? pool_kernel<64, false, true> : pool_kernel<64, false, false>))
           : (qi ? (amax ? pool_kernel<128, true, true> : pool_kernel<128, true, false>)
@@ -842,7 +870,7 @@ int pool_checked(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, co
                  int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t D,
                  int64_t block, uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar,
                  float* vamax_part, int8_t* qi, float* qs, int64_t TP, hipStream_t s) {
-  SOLATTN_REQUIRE(D == kHeadDim, SOLATTN_EUNSUPPORTED, "pool: head_dim %lld != 128", (long long)D);
+  SOLATTN_REQUIRE(D == kHeadDim || D == 64, SOLATTN_EUNSUPPORTED, "pool: head_dim %lld", (long long)D);
   SOLATTN_REQUIRE(block == 64 || block == 128, SOLATTN_EUNSUPPORTED, "pool: block %lld not in {64, 128}",
                   (long long)block);
   SOLATTN_REQUIRE(B > 0 && T > 0 && H > 0 && B <= 65535 && H <= 65535, SOLATTN_EINVAL,
@@ -854,8 +882,8 @@ int pool_checked(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, co
   if (int rc = check_bthd(q, sq_b, sq_t, sq_h, "pool q")) return rc;
   if (int rc = check_bthd(k, sk_b, sk_t, sk_h, "pool k")) return rc;
   if (int rc = check_bthd(v, sv_b, sv_t, sv_h, "pool v")) return rc;
-  return launch_pool(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H, block,
-                     kc, vc, npad, qbar, vamax_part, qi, qs, TP, s);
+  return launch_pool(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H, D,
+                     block, kc, vc, npad, qbar, vamax_part, qi, qs, TP, s);
 }
 
 }  // namespace solattn
@@ -867,17 +895,18 @@ extern "C" int solattn_pool(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64
                             uint16_t* vc, int64_t npad, float* qbar, float* vamax_part,
                             solattn_stream_t stream) {
   clear_error();
+  SOLATTN_REQUIRE(D == kHeadDim, SOLATTN_EUNSUPPORTED, "pool: head_dim %lld != 128", (long long)D);
   return pool_checked(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H, D,
                       block, kc, vc, npad, qbar, vamax_part, nullptr, nullptr, 0,
                       reinterpret_cast<hipStream_t>(stream));
 }
 
-extern "C" int solattn_moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H,
-                               int64_t D, int centre, float* kc_mean, float* kc_var,
-                               const float* vamax_part, float* vscale, solattn_stream_t stream) {
-  clear_error();
-  SOLATTN_REQUIRE(D == kHeadDim, SOLATTN_EUNSUPPORTED, "moments: head_dim %lld != 128",
-                  (long long)D);
+namespace solattn {
+
+int moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H, int64_t D, int centre,
+            float* kc_mean, float* kc_var, const float* vamax_part, float* vscale, hipStream_t s) {
+  SOLATTN_REQUIRE(D == kHeadDim || (D == 64 && !centre && !vamax_part), SOLATTN_EUNSUPPORTED,
+                  "moments: head_dim %lld", (long long)D);
   SOLATTN_REQUIRE(B > 0 && NT > 0 && H > 0 && npad >= NT && B <= 65535 && H <= 65535 &&
                       NT < (1ll << 31),
                   SOLATTN_EINVAL, "moments: bad sizes");
@@ -888,22 +917,18 @@ extern "C" int solattn_moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT
   SOLATTN_REQUIRE(reinterpret_cast<uintptr_t>(kc) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(vamax_part) % 16 == 0,
                   SOLATTN_EINVAL, "moments: kc and vamax_part must be 16-byte aligned");
-  hipLaunchKernelGGL(centre ? moments_kernel<true> : moments_kernel<false>,
-                     dim3(kHeadDim / kMomCh, static_cast<uint32_t>(H), static_cast<uint32_t>(B)),
-                     dim3(kMomThreads),
-                     0, reinterpret_cast<hipStream_t>(stream), kc, npad, static_cast<int>(NT),
-                     static_cast<int>(H), kc_mean, kc_var, vamax_part, vscale);
+  const auto kern = D == 64 ? moments_kernel<false, 64> : centre ? moments_kernel<true> : moments_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>(D / kMomCh), static_cast<uint32_t>(H), static_cast<uint32_t>(B)),
+                     dim3(kMomThreads), 0, s, kc, npad, static_cast<int>(NT), static_cast<int>(H), kc_mean,
+                     kc_var, vamax_part, vscale);
   return check_launch("moments");
 }
 
-extern "C" int solattn_route(const float* qbar, const uint16_t* kc, int64_t npad,
-                             const float* kc_mean, const float* kc_var, int64_t B, int64_t T,
-                             int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
-                             int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo,
-                             int64_t sink_q_hi, float* thr, int32_t* counts, uint32_t* mask,
-                             solattn_stream_t stream) {
-  clear_error();
-  SOLATTN_REQUIRE(D == kHeadDim, SOLATTN_EUNSUPPORTED, "route: head_dim %lld != 128", (long long)D);
+int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_mean, const float* kc_var,
+          int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
+          int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr,
+          int32_t* counts, uint32_t* mask, hipStream_t s) {
+  SOLATTN_REQUIRE(D == kHeadDim || D == 64, SOLATTN_EUNSUPPORTED, "route: head_dim %lld", (long long)D);
   SOLATTN_REQUIRE(block > 0 && B > 0 && T > 0 && H > 0 && B <= 65535 && H <= 65535,
                   SOLATTN_EINVAL, "route: bad sizes");
   const int64_t NT = cdiv(T, block);
@@ -920,14 +945,37 @@ extern "C" int solattn_route(const float* qbar, const uint16_t* kc, int64_t npad
   const float c2 = c * c;
   dim3 grid(static_cast<uint32_t>(cdiv(NT, kQB)), static_cast<uint32_t>(H),
             static_cast<uint32_t>(B));
-  hipLaunchKernelGGL(NT <= 64 ? route_kernel<4> : NT <= 128 ? route_kernel<2> : route_kernel<1>,
-                     grid, dim3(kRouteThreads),
-                     static_cast<size_t>(kQB * W * sizeof(uint32_t)),
-                     reinterpret_cast<hipStream_t>(stream), qbar, kc, npad,
-                     mode == 0 ? kc_mean : kc_var, kc_var, static_cast<int>(H),
+  const auto kern = D == 64 ? (NT <= 64 ? route_kernel<4, 64> : NT <= 128 ? route_kernel<2, 64> : route_kernel<1, 64>)
+                            : (NT <= 64 ? route_kernel<4> : NT <= 128 ? route_kernel<2> : route_kernel<1>);
+  hipLaunchKernelGGL(kern, grid, dim3(kRouteThreads), static_cast<size_t>(kQB * W * sizeof(uint32_t)), s,
+                     qbar, kc, npad, mode == 0 ? kc_mean : kc_var, kc_var, static_cast<int>(H),
                      static_cast<int>(NT), static_cast<int>(W), c, c2, tau, mode, sink_kv_lo,
                      sink_kv_hi, sink_q_lo, sink_q_hi, thr, counts, mask);
   return check_launch("route");
+}
+
+}  // namespace solattn
+
+extern "C" int solattn_moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H,
+                               int64_t D, int centre, float* kc_mean, float* kc_var,
+                               const float* vamax_part, float* vscale, solattn_stream_t stream) {
+  clear_error();
+  SOLATTN_REQUIRE(D == kHeadDim, SOLATTN_EUNSUPPORTED, "moments: head_dim %lld != 128",
+                  (long long)D);
+  return moments(kc, npad, B, NT, H, D, centre, kc_mean, kc_var, vamax_part, vscale,
+                 reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int solattn_route(const float* qbar, const uint16_t* kc, int64_t npad,
+                             const float* kc_mean, const float* kc_var, int64_t B, int64_t T,
+                             int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
+                             int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo,
+                             int64_t sink_q_hi, float* thr, int32_t* counts, uint32_t* mask,
+                             solattn_stream_t stream) {
+  clear_error();
+  SOLATTN_REQUIRE(D == kHeadDim, SOLATTN_EUNSUPPORTED, "route: head_dim %lld != 128", (long long)D);
+  return route(qbar, kc, npad, kc_mean, kc_var, B, T, H, D, block, scale, tau, mode, sink_kv_lo,
+               sink_kv_hi, sink_q_lo, sink_q_hi, thr, counts, mask, reinterpret_cast<hipStream_t>(stream));
 }
 
 namespace solattn {

@@ -18,10 +18,11 @@
  *    node's only eligible head size, /root/reference/__init__.py:41,178); the
  *    one-call pipelines (solattn_sol_attn*) also take head dims that are
  *    multiples of 8 below 128 (the reference kernels' D = 64 configs,
- *    /root/reference/_tri_fwd.py:209), running them zero-padded to 128 in the
- *    workspace: zero channels add exact zeros to every dot product and sum,
- *    so routing, codes and outputs are those of the unpadded problem, at the
- *    cost of a D = 128 call.
+ *    /root/reference/_tri_fwd.py:209). BF16 calls run heads of up to 64
+ *    channels on 64-channel kernels, everything else runs at 128; a head dim
+ *    that is neither is zero-padded to it in the workspace: zero channels add
+ *    exact zeros to every dot product and sum, so routing, codes and outputs
+ *    are those of the unpadded problem.
  *
  * Arithmetic contract (the CPU oracle restates the same operation order, so
  * pooled keys, thresholds, routing masks and INT8 codes are bit-exact):

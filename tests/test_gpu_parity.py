@@ -548,3 +548,23 @@ def test_fwd_bf16_hand_set_masks(pkg, dev, block, T):
     ref = (s @ vd + p @ vc) / (s.sum(1) + p @ lens)[:, None]
     assert float((out - ref).abs().max()) < BF16_MAXABS
     assert cosine(out.numpy(), ref.numpy()) >= BF16_COS
+
+
+@pytest.mark.parametrize("D", [8, 40, 64])
+@pytest.mark.parametrize("shape,block", [((2, 333, 3), 64), ((1, 777, 5), 128), ((1, 64, 1), 64),
+                                         ((1, 64 * 65 + 7, 3), 64), ((1, 128 * 20 + 64, 2), 128)])
+def test_small_heads_equal_padded_heads(pkg, dev, shape, block, D):
+    """Heads of up to 64 channels run on 64-channel kernels (two heads share a
+    pooling workgroup, the last of an odd count alone). Zero channels add exact
+    zeros to every sum, so the result is that of the heads padded to 128, bit
+    for bit; dense tensors and views of a fused qkv buffer."""
+    tri = _mods(pkg)[1]
+    B, T, H = shape
+    print(f"[small heads] D={D} shape={shape} block={block}", flush=True)
+    qkv = randn_bf16((B, T, 3, H, D), 95).to(dev)
+    views = qkv.unbind(2)
+    wide = [torch.nn.functional.pad(t, (0, 128 - D)).contiguous() for t in views]
+    want = tri.sol_attn(*wide, tau=0.8, block=block, scale=D ** -0.5)[..., :D]
+    for q, k, v in (views, [t.contiguous() for t in views]):
+        out = tri.sol_attn(q, k, v, tau=0.8, block=block, scale=D ** -0.5)
+        assert out.shape == (B, T, H, D) and torch.equal(out, want)

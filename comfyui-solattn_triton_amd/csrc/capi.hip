@@ -58,6 +58,7 @@ struct Layout {
   int64_t Dk;  // the kernels' head dim
   int64_t kc, vc, qbar, kc_mean, kc_var, thr, counts, mask;   // byte offsets
   int64_t vamax, vscale, qi, qs, ki, ks, vi;                          // INT8 only
+  int64_t kcc;  // INT8 only: the centred kc of the fused moments and routing
   int64_t qp, kp, vp, op;  // zero-padded [B, T, H, Dk] q, k, v, o (head dims below 128)
   bool padded;
   int64_t total;
@@ -82,8 +83,9 @@ struct Layout {
     thr = take(B * NT * H * 4);
     counts = take(B * H * NT * 4);
     mask = take(B * H * NT * W * 4);
-    vamax = vscale = qi = qs = ki = ks = vi = -1;
+    vamax = vscale = qi = qs = ki = ks = vi = kcc = -1;
     if (int8) {
+      if (NT <= kFusedRouteBlocks) kcc = take(B * npad * H * Dk * 2);
       vamax = take(B * NT * H * Dk * 4);
       vscale = take(B * H * Dk * 4);
       qi = take(B * TP * H * Dk);
@@ -201,16 +203,14 @@ int run_bf16_pipeline(const Layout& L, void* ws, const Call& call, solattn_strea
                           at<uint16_t>(ws, L.vc), L.npad, at<float>(ws, L.qbar), nullptr, nullptr, nullptr,
                           0, hs);
     if (rc) return rc;
-    rc = moments(at<uint16_t>(ws, L.kc), L.npad, c.B, L.NT, c.H, c.D, 0, at<float>(ws, L.kc_mean),
-                 at<float>(ws, L.kc_var), nullptr, nullptr, hs);
-    if (rc) return rc;
-    rc = route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.npad, at<float>(ws, L.kc_mean),
-               at<float>(ws, L.kc_var), c.B, c.T, c.H, c.D, c.block, c.scale, c.tau, 0, c.skv_lo,
-               c.skv_hi, c.sq_lo, c.sq_hi, at<float>(ws, L.thr), at<int32_t>(ws, L.counts),
-               at<uint32_t>(ws, L.mask), hs);
+    const uint16_t* kc = nullptr;
+    rc = moments_route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), nullptr, L.npad,
+                       at<float>(ws, L.kc_mean), at<float>(ws, L.kc_var), nullptr, nullptr, c.B, c.T,
+                       c.H, c.D, c.block, c.scale, c.tau, 0, c.skv_lo, c.skv_hi, c.sq_lo, c.sq_hi,
+                       at<float>(ws, L.thr), at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), &kc, hs);
     if (rc) return rc;
     return fwd_bf16(c.q, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h, c.v, c.sv_b,
-                    c.sv_t, c.sv_h, at<uint16_t>(ws, L.kc), at<uint16_t>(ws, L.vc), L.npad,
+                    c.sv_t, c.sv_h, kc, at<uint16_t>(ws, L.vc), L.npad,
                     at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), c.B, c.T, c.H, c.D, c.block,
                     c.scale, c.o, c.so_b, c.so_t, c.so_h, hs);
   });
@@ -235,12 +235,11 @@ int run_int8_pipeline(const Layout& L, void* ws, const Call& call, int int8_pv,
                           qk_block ? nullptr : at<int8_t>(ws, L.qi),
                           qk_block ? nullptr : at<float>(ws, L.qs), L.TP, hs);
     if (rc) return rc;
-    rc = moments(at<uint16_t>(ws, L.kc), L.npad, c.B, L.NT, c.H, c.D, 1, at<float>(ws, L.kc_mean),
-                 at<float>(ws, L.kc_var), vamax, vscale, hs);
-    if (rc) return rc;
-    rc = route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.npad, nullptr, at<float>(ws, L.kc_var),
-               c.B, c.T, c.H, c.D, c.block, c.scale, c.tau, 1, c.skv_lo, c.skv_hi, c.sq_lo, c.sq_hi,
-               at<float>(ws, L.thr), at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), hs);
+    const uint16_t* kc = nullptr;
+    rc = moments_route(at<float>(ws, L.qbar), at<uint16_t>(ws, L.kc), L.kcc < 0 ? nullptr : at<uint16_t>(ws, L.kcc),
+                       L.npad, at<float>(ws, L.kc_mean), at<float>(ws, L.kc_var), vamax, vscale, c.B, c.T, c.H,
+                       c.D, c.block, c.scale, c.tau, 1, c.skv_lo, c.skv_hi, c.sq_lo, c.sq_hi,
+                       at<float>(ws, L.thr), at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask), &kc, hs);
     if (rc) return rc;
     rc = quant_qkv(qk_block ? c.q : nullptr, c.sq_b, c.sq_t, c.sq_h, c.k, c.sk_b, c.sk_t, c.sk_h,
                    c.v, c.sv_b, c.sv_t, c.sv_h, c.B, c.T, c.H, c.D, at<float>(ws, L.kc_mean),
@@ -254,7 +253,7 @@ int run_int8_pipeline(const Layout& L, void* ws, const Call& call, int int8_pv,
     return fwd_int8(c.q, c.sq_b, c.sq_t, c.sq_h, at<int8_t>(ws, L.qi), at<float>(ws, L.qs),
                     at<int8_t>(ws, L.ki), at<float>(ws, L.ks),
                     int8_pv ? at<int8_t>(ws, L.vi) : nullptr, vscale, c.v, c.sv_b, c.sv_t, c.sv_h,
-                    L.TP, at<uint16_t>(ws, L.kc), at<uint16_t>(ws, L.vc), L.npad,
+                    L.TP, kc, at<uint16_t>(ws, L.vc), L.npad,
                     at<int32_t>(ws, L.counts), at<uint32_t>(ws, L.mask),
                     c.B, c.T, c.H, c.D, c.block, c.scale, int8_pv, c.o, c.so_b, c.so_t, c.so_h,
                     stream, qk_block != 0, /*ks_head_major=*/true);

@@ -117,6 +117,16 @@ int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_m
           int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
           int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr,
           int32_t* counts, uint32_t* mask, hipStream_t s);
+// moments (centre = mode) and route: one launch up to kFusedRouteBlocks blocks,
+// two above. The centred kc of mode 1 is written to kc_centred by the one launch
+// (its workgroups read kc side by side) and in place by the two; *kc_used is the
+// kc that the forward reads.
+constexpr int64_t kFusedRouteBlocks = 128;
+int moments_route(const float* qbar, uint16_t* kc, uint16_t* kc_centred, int64_t npad, float* kc_mean,
+                  float* kc_var, const float* vamax_part, float* vscale, int64_t B, int64_t T, int64_t H,
+                  int64_t D, int64_t block, float scale, float tau, int mode, int64_t sink_kv_lo,
+                  int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr, int32_t* counts,
+                  uint32_t* mask, const uint16_t** kc_used, hipStream_t s);
 int fwd_bf16(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
              int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b, int64_t sv_t,
              int64_t sv_h, const uint16_t* kc, const uint16_t* vc, int64_t npad, const int32_t* counts,

@@ -633,179 +633,285 @@ prep_int8_single_read_kernel(const PrepInt8Args a) {
 
 // ----------------------------------------------------------------- route --
 // Thresholds (/root/reference/_preprocess.py:149-163, /root/reference/_fused_prep.py:50-59)
-// and the routing rule of the forward (/root/reference/_tri_fwd.py:279-286),
-// for kQB query blocks per workgroup.
-constexpr int kQB = 8;
+// and the routing rule of the forward (/root/reference/_tri_fwd.py:279-286).
+//
+// A workgroup of four waves scores one head's key blocks against 4 Q query
+// blocks. kc rows come in passes of 64 R, staged in LDS kCh channels at a time
+// (whole cache lines, the next step's loads in flight); lane l scores rows l +
+// 64 u (u < R) against its wave's Q query blocks, whose centroids it reads from
+// LDS as broadcasts. A wave owns every (its query, 64 rows) mask word pair, so
+// masks and counts go out without another pass through LDS. Bound: the VALU,
+// NT^2 * HD fmas a head in the contract's order (21 us at NT 512, 24 heads) and
+// a quarter more to unpack kc. Measured, against one row per thread with the
+// centroids as scalar operands (115 SGPRs spilled to lanes, every cache line
+// fetched in eight 16-byte pieces): NT 512 46-53 -> 37-42 us, NT 591 with 40
+// heads 113 -> 85, NT 256 23 -> 19.7, NT 190 21.6 -> 17.5. Eight query blocks a
+// wave were slower (43-51 us at NT 512: half the workgroups), as was taking the
+// centroids by the fma's lane move (row_newbcast; 47-55 us).
+//
+// FUSE (every row in one pass, NT <= 64 R, kCh = HD): the workgroup also takes
+// the head's moments, in moments_kernel's order, from the rows it has staged:
+// kMoments as centre = 0; kCentred as centre = 1, with the centred kc written to
+// kc_out and the V scale from vamax_part (both by the head's first workgroup).
+// One launch for two: 3.6 + 9.1 -> 8.2 us at NT 16, 4.5 + 9.2 -> 8.7 at NT 64,
+// 7.2 + 13.0 -> 18.0 at NT 81 with the INT8 outputs.
 constexpr int kRouteThreads = 256;
 constexpr int kMaxWords = 512;  // NT <= 16384 (the forwards' limit)
-// The workgroup's threads form G groups of R = kRouteThreads / G (a multiple
-// of 64: whole waves); thread t scores key block (kc row) j0 + t % R against
-// the kQB / G query blocks of its group, its row streaming through registers
-// 32 channels at a time (the next 32 in flight); the query centroids are
-// wave-uniform, so each fma takes its q operand from an SGPR (scalar loads).
-// G > 1 serves short sequences (NT <= 128), whose rows would leave waves idle.
-// Against kc rows staged in LDS with two or four threads per row: 20.0 ->
-// 19.7 us at NT 256 and 63.0 -> 47.2 us at NT 512, same bits.
-template <int G, int HD = kHeadDim>
-__global__ void __launch_bounds__(kRouteThreads)
-route_kernel(const float* __restrict__ qbar, const uint16_t* __restrict__ kc, int64_t npad,
-             const float* __restrict__ kc_mean, const float* __restrict__ kc_var, int H, int NT,
-             int W, float c, float c2, float tau, int mode, int64_t skv_lo, int64_t skv_hi,
-             int64_t sq_lo, int64_t sq_hi, float* __restrict__ thr_out,
-             int32_t* __restrict__ counts, uint32_t* __restrict__ mask) {
-  const int i0 = blockIdx.x * kQB, h = blockIdx.y, b = blockIdx.z;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  extern __shared__ __align__(16) uint32_t smask_lds[];
-  const auto smask = [&](int i, int w) -> uint32_t& { return smask_lds[i * W + w]; };
-  __shared__ __align__(16) float sq[kQB][HD];  // the kQB query centroids
+enum RouteFuse { kNoFuse = 0, kMoments = 1, kCentred = 2 };
+
+struct RouteArgs {
+  const float* qbar;
+  const uint16_t* kc;
+  int64_t npad;
+  float *kc_mean, *kc_var;  // read, or written by FUSE
+  int H, NT, W;
+  float c, c2, tau;
+  int mode;
+  int64_t skv_lo, skv_hi, sq_lo, sq_hi;
+  float* thr;
+  int32_t* counts;
+  uint32_t* mask;
+  uint16_t* kc_out;         // kCentred
+  const float* vamax_part;  // kCentred, may be null
+  float* vscale;
+};
+
+template <int R, int Q, int HD, int FUSE>
+__global__ void __launch_bounds__(kRouteThreads) route_kernel(const RouteArgs a) {
+  constexpr int kCh = R == 4 ? 64 : HD;        // channels per LDS step
+  constexpr int kPitch = kCh + 8;              // LDS row pitch (elements): 16-byte reads of 16 rows hit all banks
+  constexpr int kRows = 64 * R, kQB = 4 * Q;
+  constexpr int kChunks = kCh / 8;             // 16-byte chunks of a row per step
+  constexpr int kLoads = kRows * kChunks / kRouteThreads;
+  static_assert(FUSE == kNoFuse || kCh == HD, "moments need whole rows");
+  const int i0 = blockIdx.x * kQB, h = blockIdx.y, b = blockIdx.z, H = a.H, NT = a.NT;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  __shared__ __align__(16) uint16_t sk[kRows * kPitch];
+  __shared__ __align__(16) float sq[kQB][HD];  // the query centroids
   __shared__ __align__(16) float smk[HD];      // kc mean (mode 0)
   __shared__ __align__(16) float svk[HD];      // kc variance
-  static_assert(kQB * HD / 4 <= kRouteThreads && 2 * HD <= kRouteThreads,
-                "at most one float4 of the centroids and one moment per thread");
   const int64_t bh = static_cast<int64_t>(b) * H + h;
-  {
-    // The centroids and moments, one load per thread. Query rows past NT (a
-    // ragged last workgroup) read row NT-1; nothing of theirs is stored.
-    const int qb = t / (HD / 4), q4 = t % (HD / 4);
-    if (kQB * HD / 4 == kRouteThreads || qb < kQB) {
-      const float4 x =
-          reinterpret_cast<const float4*>(qbar + (bh * NT + min(i0 + qb, NT - 1)) * HD)[q4];
-      reinterpret_cast<float4*>(&sq[qb][0])[q4] = x;
-    }
-    if (2 * HD == kRouteThreads || t < 2 * HD) {
-      const float mv = t < HD ? kc_mean[bh * HD + t] : kc_var[bh * HD + t - HD];
-      (t < HD ? smk[t] : svk[t - HD]) = mv;
-    }
-  }
-  for (int e = t; e < kQB * W; e += kRouteThreads) smask_lds[e] = 0u;
-  constexpr int R = kRouteThreads / G, kQG = kQB / G;  // rows per pass, query blocks per thread
-  static_assert(R % 64 == 0 && kQB % G == 0, "route groups are whole waves");
-  const int rr = t % R;
-  const int ig = __builtin_amdgcn_readfirstlane(t / R) * kQG;  // the group's first query block
-  const float* qrow[kQG];  // wave-uniform rows of the centroids
-#pragma unroll
-  for (int i = 0; i < kQG; ++i) qrow[i] = qbar + (bh * NT + min(i0 + ig + i, NT - 1)) * HD;
-  // kc rows through raw buffer loads: base at row j0 (wave-uniform), the lane's
-  // row rr further; rows past NT read 0 (and are not active).
-  const uint16_t* kch = kc + (static_cast<int64_t>(b) * npad * H + h) * HD;
+  // kc rows through raw buffer loads: base at row j0 (wave-uniform); rows past
+  // NT read 0 (and are not active).
+  const uint16_t* kch = a.kc + (static_cast<int64_t>(b) * a.npad * H + h) * HD;
   const int64_t sj = static_cast<int64_t>(H) * HD;
-  const uint32_t roff = static_cast<uint32_t>(rr * sj * 2);
-  __syncthreads();  // the centroids, moments and cleared mask words
-  // Every wave computes the kQB thresholds (lane i: query block i0 + i), one
-  // fma chain per moment in ascending d, so no barrier waits on them.
-  float th;
+  const int lrow = t / kChunks, lchunk = t % kChunks;  // this thread's loads: rows lrow + i * kRouteThreads / kChunks
+  uint4 kn[kLoads];
+  const auto load_rows = [&](int j0, int d0) {
+    const uint32_t nb = rows_nbytes(j0, NT, 2 * sj, 2 * HD, kRows * 2 * sj);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      kn[i] = buffer_load16(kch + j0 * sj, nb,
+                            static_cast<uint32_t>((lrow + i * (kRouteThreads / kChunks)) * sj * 2 + (d0 + 8 * lchunk) * 2));
+  };
+  load_rows(0, 0);
   {
-    const float* qv = sq[min(lane, kQB - 1)];
-    float mu = 0.f, var = 0.f;
-#pragma unroll 4
-    for (int d = 0; d < HD; d += 4) {
-      const float4 x = *reinterpret_cast<const float4*>(qv + d);
-      const float4 vk = *reinterpret_cast<const float4*>(svk + d);
-      if (mode == 0) {
-        const float4 mk = *reinterpret_cast<const float4*>(smk + d);
-        mu = fmaf(x.x, mk.x, mu);
-        var = fmaf(x.x * x.x, vk.x, var);
-        mu = fmaf(x.y, mk.y, mu);
-        var = fmaf(x.y * x.y, vk.y, var);
-        mu = fmaf(x.z, mk.z, mu);
-        var = fmaf(x.z * x.z, vk.z, var);
-        mu = fmaf(x.w, mk.w, mu);
-        var = fmaf(x.w * x.w, vk.w, var);
-      } else {
-        var = fmaf(x.x * x.x, vk.x, var);
-        var = fmaf(x.y * x.y, vk.y, var);
-        var = fmaf(x.z * x.z, vk.z, var);
-        var = fmaf(x.w * x.w, vk.w, var);
+    // Query rows past NT (a ragged last workgroup) read row NT-1; nothing of
+    // theirs is stored.
+    constexpr int kF4 = kQB * HD / 4;
+#pragma unroll
+    for (int e0 = 0; e0 < kF4; e0 += kRouteThreads) {
+      const int e = e0 + t;
+      if (kF4 % kRouteThreads == 0 || e < kF4) {
+        const int qb = e / (HD / 4), q4 = e % (HD / 4);
+        reinterpret_cast<float4*>(&sq[qb][0])[q4] =
+            reinterpret_cast<const float4*>(a.qbar + (bh * NT + min(i0 + qb, NT - 1)) * HD)[q4];
       }
     }
-    if (mode == 0) {
-      mu = mu * c;
-      var = var * c2;
-      const float sd = sqrtf(fmaxf(var, 0.f) + 1e-6f);
-      th = mu + tau * sd;
-    } else {
-      var = var * c2;
-      th = tau * sqrtf(var + 1e-6f);
+    if (FUSE == kNoFuse && t < 2 * HD) {
+      if (t >= HD) svk[t - HD] = a.kc_var[bh * HD + t - HD];
+      else if (a.mode == 0) smk[t] = a.kc_mean[bh * HD + t];
     }
-    if (wave == 0 && lane < kQB && i0 + lane < NT)
-      thr_out[(static_cast<int64_t>(b) * NT + i0 + lane) * H + h] = th;
   }
-  constexpr int kCh = 32;                  // channels of the row per step
-  constexpr int kChLoads = kCh / 8;        // 16-byte loads per step
-  for (int j0 = 0; j0 < NT; j0 += R) {
-    const int j = j0 + rr;
-    const bool active = j < NT;
-    const uint16_t* base = kch + j0 * sj;
-    const uint32_t nb = rows_nbytes(j0, NT, 2 * sj, 2 * HD, R * 2 * sj);
-    float acc[kQG];
+  const auto stage_rows = [&] {
 #pragma unroll
-    for (int i = 0; i < kQG; ++i) acc[i] = 0.f;
-    uint4 kn[kChLoads];  // the next channel step of this thread's row, in flight
+    for (int i = 0; i < kLoads; ++i)
+      *reinterpret_cast<uint4*>(&sk[(lrow + i * (kRouteThreads / kChunks)) * kPitch + 8 * lchunk]) = kn[i];
+  };
+
+  if constexpr (FUSE != kNoFuse) {
+    __shared__ float part[2][8][HD];
+    constexpr int kSets = kRouteThreads / HD, kGroups = 8 / kSets;  // partial groups per thread
+    const int c = t % HD, g0 = (t / HD) * kGroups;
+    const bool first = blockIdx.x == 0;
+    const float fnt = static_cast<float>(NT);
+    float am = 0.f;  // |v| max of channel c over this thread's share of the blocks
+    if (FUSE == kCentred && first && a.vamax_part) {
+      const float* ah = a.vamax_part + (static_cast<int64_t>(b) * NT * H + h) * HD + c;
+      constexpr int kBatch = 32;  // loads in flight
+      for (int j0 = t / HD; j0 < NT; j0 += kBatch * kSets) {
+        float v[kBatch];
 #pragma unroll
-    for (int u = 0; u < kChLoads; ++u) kn[u] = buffer_load16(base, nb, roff + 16 * u);
-#pragma unroll 1
-    for (int d0 = 0; d0 < HD; d0 += kCh) {
-      uint4 kr[kChLoads];
+        for (int i = 0; i < kBatch; ++i) v[i] = ah[min(j0 + i * kSets, NT - 1) * sj];
 #pragma unroll
-      for (int u = 0; u < kChLoads; ++u) kr[u] = kn[u];
-      if (d0 + kCh < HD) {
-#pragma unroll
-        for (int u = 0; u < kChLoads; ++u)
-          kn[u] = buffer_load16(base, nb, roff + 2 * (d0 + kCh) + 16 * u);
+        for (int i = 0; i < kBatch; ++i) am = fmaxf(am, v[i]);
       }
+    }
+    stage_rows();
+    __syncthreads();
 #pragma unroll
-      for (int d4 = 0; d4 < kCh / 4; ++d4) {
-        const uint4& w = kr[d4 / 2];
-        const uint32_t k01 = (d4 & 1) ? w.z : w.x, k23 = (d4 & 1) ? w.w : w.y;
-        const float k0 = lo_bf16(k01), k1 = hi_bf16(k01), k2 = lo_bf16(k23), k3 = hi_bf16(k23);
+    for (int u = 0; u < kGroups; ++u) {
+      float s = 0.f;
+#pragma unroll 8
+      for (int j = g0 + u; j < NT; j += 8) s = s + bf2f(sk[j * kPitch + c]);
+      part[0][g0 + u][c] = s;
+    }
+    __syncthreads();
+    const float mean = tree8(part[0], c) / fnt;
 #pragma unroll
-        for (int i = 0; i < kQG; ++i) {
-          const float4 qv = *reinterpret_cast<const float4*>(qrow[i] + d0 + 4 * d4);
-          acc[i] = fmaf(qv.x, k0, acc[i]);
-          acc[i] = fmaf(qv.y, k1, acc[i]);
-          acc[i] = fmaf(qv.z, k2, acc[i]);
-          acc[i] = fmaf(qv.w, k3, acc[i]);
+    for (int u = 0; u < kGroups; ++u) {
+      float s = 0.f;
+#pragma unroll 8
+      for (int j = g0 + u; j < NT; j += 8) {
+        float y = bf2f(sk[j * kPitch + c]) - mean;
+        if (FUSE == kCentred) {  // bf16 of the centred value, as moments_kernel
+          const uint16_t nb = static_cast<uint16_t>(cvt_pk_bf16(y, 0.f));
+          y = bf2f(nb);
+          sk[j * kPitch + c] = nb;
+        }
+        s = s + y * y;
+      }
+      part[1][g0 + u][c] = s;
+    }
+    __syncthreads();
+    if (t < HD) {
+      const float var = tree8(part[1], t) / fnt;
+      smk[t] = mean;
+      svk[t] = var;
+      if (first) {
+        a.kc_mean[bh * HD + t] = mean;
+        a.kc_var[bh * HD + t] = var;
+      }
+    }
+    if (FUSE == kCentred && first) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) {
+        const int j = lrow + i * (kRouteThreads / kChunks);
+        if (j < NT)
+          *reinterpret_cast<uint4*>(a.kc_out + (static_cast<int64_t>(b) * a.npad * H + h) * HD + j * sj + 8 * lchunk) =
+              *reinterpret_cast<const uint4*>(&sk[j * kPitch + 8 * lchunk]);
+      }
+      if (a.vamax_part) {
+        part[0][t / HD][c] = am;
+        __syncthreads();
+        if (t < HD) {
+          float m = part[0][0][t];
+#pragma unroll
+          for (int i = 1; i < kSets; ++i) m = fmaxf(m, part[0][i][t]);
+          const float sc = m * (1.0f / 127.0f);  // as moments_kernel
+          a.vscale[bh * HD + t] = sc < 1e-8f ? 1e-8f : sc;
         }
       }
     }
-    const bool in_skv = j >= skv_lo && j < skv_hi;
-    const int w0 = (j0 + 64 * (wave % (R / 64))) >> 5;  // this wave's 64 rows
+  }
+  __syncthreads();  // the centroids and moments (FUSE: the rows too)
+
+  // Every wave computes its Q thresholds (lane i: query block ib + i), one fma
+  // chain per moment in ascending d.
+  const int iw = wave * Q, ib = i0 + iw;
+  float th;
+  {
+    const float* qv = sq[iw + min(lane, Q - 1)];
+    float mu = 0.f, var = 0.f;
+#pragma unroll 8
+    for (int d = 0; d < HD; d += 4) {
+      const float4 x = *reinterpret_cast<const float4*>(qv + d);
+      const float4 vk = *reinterpret_cast<const float4*>(svk + d);
+      if (a.mode == 0) {
+        const float4 mk = *reinterpret_cast<const float4*>(smk + d);
+        mu = fmaf(x.x, mk.x, mu);
+        mu = fmaf(x.y, mk.y, mu);
+        mu = fmaf(x.z, mk.z, mu);
+        mu = fmaf(x.w, mk.w, mu);
+      }
+      var = fmaf(x.x * x.x, vk.x, var);
+      var = fmaf(x.y * x.y, vk.y, var);
+      var = fmaf(x.z * x.z, vk.z, var);
+      var = fmaf(x.w * x.w, vk.w, var);
+    }
+    var = var * a.c2;
+    if (a.mode == 0) {
+      mu = mu * a.c;
+      const float sd = sqrtf(fmaxf(var, 0.f) + 1e-6f);
+      th = mu + a.tau * sd;
+    } else {
+      th = a.tau * sqrtf(var + 1e-6f);
+    }
+    if (lane < Q && ib + lane < NT) a.thr[(static_cast<int64_t>(b) * NT + ib + lane) * H + h] = th;
+  }
+
+  int cnt[Q];
 #pragma unroll
-    for (int i = 0; i < kQG; ++i) {
-      const int il = ig + i;
-      const int qi = i0 + il;
-      const float r = acc[i] * c;
-      const int dij = qi > j ? qi - j : j - qi;
-      const bool q_in_sink = qi >= sq_lo && qi < sq_hi;
-      const float thr = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, th), il));
-      const bool routed = (r > thr) || dij <= 1 || in_skv;
-      const bool exact = active && qi < NT && (q_in_sink || routed);
-      const uint64_t bal = __ballot(exact);
-      if (lane == 0 && w0 < W) {
-        smask(il, w0) = static_cast<uint32_t>(bal);
-        if (w0 + 1 < W) smask(il, w0 + 1) = static_cast<uint32_t>(bal >> 32);
+  for (int i = 0; i < Q; ++i) cnt[i] = 0;
+  for (int j0 = 0; j0 < NT; j0 += kRows) {
+    float acc[R][Q];
+    const int nact = (NT - j0 + 63) >> 6;  // groups of 64 rows with a row below NT
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+#pragma unroll
+      for (int u = 0; u < R; ++u) acc[u][i] = 0.f;
+#pragma unroll 1
+    for (int d0 = 0; d0 < HD; d0 += kCh) {
+      if constexpr (FUSE == kNoFuse) {
+        if (j0 + d0 > 0) __syncthreads();  // every wave is done with the rows staged before
+        stage_rows();
+        __syncthreads();
+        const bool wrap = d0 + kCh >= HD;
+        const int jn = wrap ? j0 + kRows : j0;
+        if (jn < NT) load_rows(jn, wrap ? 0 : d0 + kCh);
+      }
+#pragma unroll 2
+      for (int d8 = 0; d8 < kChunks; ++d8) {
+        float4 qv[Q][2];  // broadcast reads: the wave's centroids
+#pragma unroll
+        for (int i = 0; i < Q; ++i) {
+          qv[i][0] = *reinterpret_cast<const float4*>(&sq[iw + i][d0 + 8 * d8]);
+          qv[i][1] = *reinterpret_cast<const float4*>(&sq[iw + i][d0 + 8 * d8 + 4]);
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          if (R > 1 && u >= nact) break;  // (uniform) a group of rows past NT
+          float x[8];
+          unpack8(*reinterpret_cast<const uint4*>(&sk[(lane + 64 * u) * kPitch + 8 * d8]), x);
+#pragma unroll
+          for (int i = 0; i < Q; ++i) {
+            acc[u][i] = fmaf(qv[i][0].x, x[0], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][0].y, x[1], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][0].z, x[2], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][0].w, x[3], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][1].x, x[4], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][1].y, x[5], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][1].z, x[6], acc[u][i]);
+            acc[u][i] = fmaf(qv[i][1].w, x[7], acc[u][i]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      const int qi = ib + i;
+      if (qi >= NT) break;
+      const float thr = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, th), i));
+      const bool q_in_sink = qi >= a.sq_lo && qi < a.sq_hi;
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int jb = j0 + 64 * u;
+        if (jb >= NT) break;
+        const int j = jb + lane;
+        const int dij = qi > j ? qi - j : j - qi;
+        const bool routed = acc[u][i] * a.c > thr || dij <= 1 || (j >= a.skv_lo && j < a.skv_hi);
+        const uint64_t bal = __ballot(j < NT && (q_in_sink || routed));
+        cnt[i] += __popcll(bal);
+        const int w0 = jb >> 5;
+        if (lane < 2 && w0 + lane < a.W)
+          a.mask[(bh * NT + qi) * a.W + w0 + lane] = static_cast<uint32_t>(lane ? bal >> 32 : bal);
       }
     }
   }
-  __syncthreads();
-
-  // Masks and exact-block counts, one query block per wave at a time.
-  for (int i = wave; i < kQB; i += kRouteThreads / 64) {
-    const int qi = i0 + i;
-    if (qi >= NT) break;
-    const int64_t row = bh * NT + qi;
-    int base = 0;
-    for (int w0 = 0; w0 < W; w0 += 64) {
-      const int w = w0 + lane;
-      const uint32_t word = w < W ? smask(i, w) : 0u;
-      if (w < W) mask[row * W + w] = word;
-      int cnt = __popc(word);
+  int mine = cnt[0];
 #pragma unroll
-      for (int s = 32; s >= 1; s >>= 1) cnt += __shfl_xor(cnt, s);
-      base += cnt;
-    }
-    if (lane == 0) counts[row] = base;
-  }
+  for (int i = 1; i < Q; ++i) mine = lane == i ? cnt[i] : mine;
+  if (lane < Q && ib + lane < NT) a.counts[bh * NT + ib + lane] = mine;
 }
 
 }  // namespace solattn
@@ -924,16 +1030,27 @@ int moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H, int64_
   return check_launch("moments");
 }
 
-int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_mean, const float* kc_var,
-          int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
-          int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr,
-          int32_t* counts, uint32_t* mask, hipStream_t s) {
+namespace {
+
+template <int HD, int FUSE>
+void launch_route(const RouteArgs& a, int64_t B, hipStream_t s) {
+  const auto go = [&](auto kern, int Q) {
+    hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>(cdiv(a.NT, 4 * Q)), static_cast<uint32_t>(a.H), static_cast<uint32_t>(B)),
+                       dim3(kRouteThreads), 0, s, a);
+  };
+  if (a.NT <= 64) go(route_kernel<1, 2, HD, FUSE>, 2);  // twice the workgroups for the fewest rows
+  else if (a.NT <= 128) go(route_kernel<2, 4, HD, FUSE>, 4);
+  else if constexpr (FUSE == kNoFuse) go(route_kernel<4, 4, HD, FUSE>, 4);
+}
+
+int check_route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_mean,
+                const float* kc_var, int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, int mode,
+                const float* thr, const int32_t* counts, const uint32_t* mask) {
   SOLATTN_REQUIRE(D == kHeadDim || D == 64, SOLATTN_EUNSUPPORTED, "route: head_dim %lld", (long long)D);
   SOLATTN_REQUIRE(block > 0 && B > 0 && T > 0 && H > 0 && B <= 65535 && H <= 65535,
                   SOLATTN_EINVAL, "route: bad sizes");
   const int64_t NT = cdiv(T, block);
-  const int64_t W = cdiv(NT, 32);
-  SOLATTN_REQUIRE(W <= kMaxWords, SOLATTN_EUNSUPPORTED, "route: %lld blocks exceed %d",
+  SOLATTN_REQUIRE(cdiv(NT, 32) <= kMaxWords, SOLATTN_EUNSUPPORTED, "route: %lld blocks exceed %d",
                   (long long)NT, kMaxWords * 32);
   SOLATTN_REQUIRE(npad >= NT, SOLATTN_EINVAL, "route: npad < NT");
   SOLATTN_REQUIRE(mode == 0 || mode == 1, SOLATTN_EINVAL, "route: mode %d", mode);
@@ -941,17 +1058,62 @@ int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_m
                   SOLATTN_EINVAL, "route: null pointer");
   SOLATTN_REQUIRE(reinterpret_cast<uintptr_t>(kc) % 16 == 0, SOLATTN_EINVAL,
                   "route: kc must be 16-byte aligned");
+  return 0;
+}
+
+RouteArgs route_args(const float* qbar, const uint16_t* kc, int64_t npad, float* kc_mean, float* kc_var,
+                     int64_t T, int64_t H, int64_t block, float scale, float tau, int mode,
+                     int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi,
+                     float* thr, int32_t* counts, uint32_t* mask) {
+  const int64_t NT = cdiv(T, block);
   const float c = scale * kLog2e;
-  const float c2 = c * c;
-  dim3 grid(static_cast<uint32_t>(cdiv(NT, kQB)), static_cast<uint32_t>(H),
-            static_cast<uint32_t>(B));
-  const auto kern = D == 64 ? (NT <= 64 ? route_kernel<4, 64> : NT <= 128 ? route_kernel<2, 64> : route_kernel<1, 64>)
-                            : (NT <= 64 ? route_kernel<4> : NT <= 128 ? route_kernel<2> : route_kernel<1>);
-  hipLaunchKernelGGL(kern, grid, dim3(kRouteThreads), static_cast<size_t>(kQB * W * sizeof(uint32_t)), s,
-                     qbar, kc, npad, mode == 0 ? kc_mean : kc_var, kc_var, static_cast<int>(H),
-                     static_cast<int>(NT), static_cast<int>(W), c, c2, tau, mode, sink_kv_lo,
-                     sink_kv_hi, sink_q_lo, sink_q_hi, thr, counts, mask);
+  return {qbar, kc, npad, kc_mean, kc_var, static_cast<int>(H), static_cast<int>(NT),
+          static_cast<int>(cdiv(NT, 32)), c, c * c, tau, mode, sink_kv_lo, sink_kv_hi, sink_q_lo,
+          sink_q_hi, thr, counts, mask, nullptr, nullptr, nullptr};
+}
+
+}  // namespace
+
+int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_mean, const float* kc_var,
+          int64_t B, int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau, int mode,
+          int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr,
+          int32_t* counts, uint32_t* mask, hipStream_t s) {
+  if (int rc = check_route(qbar, kc, npad, kc_mean, kc_var, B, T, H, D, block, mode, thr, counts, mask))
+    return rc;
+  const RouteArgs a = route_args(qbar, kc, npad, const_cast<float*>(kc_mean), const_cast<float*>(kc_var), T, H,
+                                 block, scale, tau, mode, sink_kv_lo, sink_kv_hi, sink_q_lo, sink_q_hi,
+                                 thr, counts, mask);
+  if (D == 64) launch_route<64, kNoFuse>(a, B, s);
+  else launch_route<kHeadDim, kNoFuse>(a, B, s);
   return check_launch("route");
+}
+
+int moments_route(const float* qbar, uint16_t* kc, uint16_t* kc_centred, int64_t npad, float* kc_mean,
+                  float* kc_var, const float* vamax_part, float* vscale, int64_t B, int64_t T, int64_t H,
+                  int64_t D, int64_t block, float scale, float tau, int mode, int64_t sink_kv_lo,
+                  int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, float* thr, int32_t* counts,
+                  uint32_t* mask, const uint16_t** kc_used, hipStream_t s) {
+  const int64_t NT = cdiv(T, block);
+  if (NT > kFusedRouteBlocks) {
+    *kc_used = kc;
+    if (int rc = moments(kc, npad, B, NT, H, D, mode, kc_mean, kc_var, vamax_part, vscale, s)) return rc;
+    return route(qbar, kc, npad, kc_mean, kc_var, B, T, H, D, block, scale, tau, mode, sink_kv_lo,
+                 sink_kv_hi, sink_q_lo, sink_q_hi, thr, counts, mask, s);
+  }
+  if (int rc = check_route(qbar, kc, npad, kc_mean, kc_var, B, T, H, D, block, mode, thr, counts, mask))
+    return rc;
+  SOLATTN_REQUIRE(kc_mean && (mode == 0 || (kc_centred && D == kHeadDim)) && (!vamax_part || vscale),
+                  SOLATTN_EINVAL, "moments_route: bad arguments");
+  RouteArgs a = route_args(qbar, kc, npad, kc_mean, kc_var, T, H, block, scale, tau, mode, sink_kv_lo,
+                           sink_kv_hi, sink_q_lo, sink_q_hi, thr, counts, mask);
+  a.kc_out = kc_centred;
+  a.vamax_part = vamax_part;
+  a.vscale = vscale;
+  *kc_used = mode == 1 ? kc_centred : kc;
+  if (mode == 1) launch_route<kHeadDim, kCentred>(a, B, s);
+  else if (D == 64) launch_route<64, kMoments>(a, B, s);
+  else launch_route<kHeadDim, kMoments>(a, B, s);
+  return check_launch("moments_route");
 }
 
 }  // namespace solattn

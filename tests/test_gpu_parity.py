@@ -568,3 +568,27 @@ def test_small_heads_equal_padded_heads(pkg, dev, shape, block, D):
     for q, k, v in (views, [t.contiguous() for t in views]):
         out = tri.sol_attn(q, k, v, tau=0.8, block=block, scale=D ** -0.5)
         assert out.shape == (B, T, H, D) and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("NT", [1, 2, 33, 63, 64, 65, 96, 127, 128, 129, 257])
+@pytest.mark.parametrize("mode", ["bf16", "int8_pv", "int8_bf16pv"])
+def test_one_call_equals_its_stages(pkg, dev, NT, mode):
+    """Up to 128 blocks the one calls take the moments inside the routing launch;
+    the stage-by-stage path (bit-exact against the oracle above) must give the
+    same output bits. Ragged lengths, two batches, an odd head count, sinks."""
+    prep, tri, i8, fp = _mods(pkg)[:4]
+    block = 64
+    B, T, H = 2, (NT - 1) * block + (64 if NT == 64 else 37), 3
+    q, k, v = (randn_bf16((B, T, H, 128), s).to(dev) for s in (96, 97, 98))
+    k += 0.5  # a mean that centring has to take out
+    kw = dict(tau=0.7, block=block, sink_blocks=(0, 1), sink_q=(1, 2))
+    print(f"[one call] NT={NT} mode={mode}", flush=True)
+    if mode == "bf16":
+        one = tri.sol_attn(q, k, v, **kw)
+        two = tri.forward_bf16(q, k, v, prep.route(q, k, v, scale=128 ** -0.5, **kw))
+    else:
+        pv = mode == "int8_pv"
+        one = i8.sol_attn_int8(q, k, v, int8_pv=pv, **kw)
+        r, *codes = fp.fused_preprocess_routing(q, k, v, scale=128 ** -0.5, int8_pv=pv, **kw)
+        two = i8.forward_int8(q, v, r, *codes, int8_pv=pv)
+    assert torch.equal(one, two)

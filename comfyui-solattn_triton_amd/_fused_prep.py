@@ -2,8 +2,10 @@
 
 Mirrors /root/reference/_fused_prep.py:62-98: pooled keys centred by their own
 mean (K smoothing), thresholds tau*sigma, per-token INT8 Q and smoothed K,
-per-channel INT8 V, all from the gfx950 kernels: two passes (pooling with the
-Q codes, moments, then the K and V codes), or optionally one read of Q, K and
+per-channel INT8 V, all from the gfx950 kernels: two passes in one call
+(``solattn_preprocess_int8``: pooling with the Q codes, moments, routing, then
+the K and V codes; 382 -> 318 us at 32760 tokens and block 64 against separate
+launches for the codes of Q, K and V), or optionally one read of Q, K and
 V (``solattn_prep_int8``, same bits, slower on this part).
 """
 
@@ -13,7 +15,7 @@ import torch
 
 from ._capi import LIB, QUANT_BLOCK, SolAttnError, call, ptr, stream
 from ._preprocess import (BLOCK_SIZE, GROUP_PAD, HEAD_DIM, Routing, as_kernel_input, check_inputs,
-                          num_blocks, pad_heads, route)
+                          num_blocks, pad_heads)
 
 SOLATTN_EUNSUPPORTED = -2
 
@@ -47,26 +49,34 @@ def fused_preprocess_routing(q, k, v, *, tau, scale, int8_pv=True, block=BLOCK_S
                            sink_blocks=sink_blocks, sink_q=sink_q)
         if one is not None:
             return one
-    r: Routing = route(q, k, v, scale=scale, tau=tau, block=block, int8=True, v_absmax=int8_pv,
-                       sink_blocks=sink_blocks, sink_q=sink_q)
+    check_inputs(q, k, v, block, padded_ok=False)
     q, k, v = as_kernel_input(q), as_kernel_input(k), as_kernel_input(v)
     B, T, H, D = q.shape
+    NT = num_blocks(T, block)
+    npad = (NT + GROUP_PAD - 1) // GROUP_PAD * GROUP_PAD
     dev = q.device
-    qi = torch.empty((B, T, H, D), device=dev, dtype=torch.int8)
-    ki = torch.empty_like(qi)
-    qs = torch.empty((B, T, H), device=dev, dtype=torch.float32)
-    ks = torch.empty_like(qs)
-    vi = torch.empty_like(qi) if int8_pv else None
+    f32 = dict(device=dev, dtype=torch.float32)
+    i8 = dict(device=dev, dtype=torch.int8)
+    kc = torch.empty((B, npad, H, D), device=dev, dtype=torch.bfloat16)
+    vc = torch.empty_like(kc)
+    qbar = torch.empty((B, H, NT, D), **f32)
+    kc_mean, kc_var = torch.empty((B, H, D), **f32), torch.empty((B, H, D), **f32)
+    vamax = torch.empty((B, NT, H, D), **f32) if int8_pv else None
+    vscale = torch.empty((B, H, D), **f32) if int8_pv else None
+    thr = torch.empty((B, NT, H), **f32)
+    counts = torch.empty((B, H, NT), device=dev, dtype=torch.int32)
+    mask = torch.empty((B, H, NT, (NT + 31) // 32), device=dev, dtype=torch.int32)
+    qi, ki = torch.empty((B, T, H, D), **i8), torch.empty((B, T, H, D), **i8)
+    vi = torch.empty((B, T, H, D), **i8) if int8_pv else None
+    qs, ks = torch.empty((B, T, H), **f32), torch.empty((B, T, H), **f32)
     with torch.cuda.device(dev):
-        s = stream(dev)
-        rows = "solattn_quant_rows" if quant_block is None else "solattn_quant_rows_blocked"
-        call(rows, ptr(q), q.stride(0), q.stride(1), q.stride(2), B, T, H, D, None, ptr(qi),
-             ptr(qs), T, s)
-        call(rows, ptr(k), k.stride(0), k.stride(1), k.stride(2), B, T, H, D, ptr(r.kc_mean),
-             ptr(ki), ptr(ks), T, s)
-        if int8_pv:
-            call("solattn_quant_v", ptr(v), v.stride(0), v.stride(1), v.stride(2), B, T, H, D,
-                 ptr(r.vscale), ptr(vi), T, s)
+        call("solattn_preprocess_int8", ptr(q), q.stride(0), q.stride(1), q.stride(2), ptr(k),
+             k.stride(0), k.stride(1), k.stride(2), ptr(v), v.stride(0), v.stride(1), v.stride(2),
+             B, T, H, D, block, float(scale), float(tau), int(sink_blocks[0]), int(sink_blocks[1]),
+             int(sink_q[0]), int(sink_q[1]), 0 if quant_block is None else 1, ptr(kc), ptr(vc), npad,
+             ptr(qbar), ptr(kc_mean), ptr(kc_var), ptr(vamax), ptr(vscale), ptr(thr), ptr(counts),
+             ptr(mask), ptr(qi), ptr(qs), ptr(ki), ptr(ks), ptr(vi), stream(dev))
+    r = Routing(kc, vc, thr, qbar, kc_mean, kc_var, counts, mask, vamax, vscale, block, T)
     return r, qi, qs, ki, ks, vi
 
 

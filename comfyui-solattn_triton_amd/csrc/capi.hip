@@ -116,7 +116,7 @@ using namespace solattn;
 
 extern "C" const char* solattn_last_error(void) { return g_error; }
 
-extern "C" int solattn_abi_version(void) { return (2 << 16) | 1; }
+extern "C" int solattn_abi_version(void) { return (2 << 16) | 2; }
 
 extern "C" int solattn_morton_perm(int64_t frames, int64_t height, int64_t width, int curve,
                                    int64_t roll, int64_t* perm, int64_t* inverse) {
@@ -392,4 +392,35 @@ extern "C" int solattn_sol_attn_int8_qblock(SOLATTN_INT8_CALL_PARAMS) {
   return sol_attn_int8_call(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H,
                             D, block, scale, tau, sink_kv_lo, sink_kv_hi, sink_q_lo, sink_q_hi,
                             int8_pv, workspace, workspace_bytes, o, so_b, so_t, so_h, stream, 1);
+}
+
+extern "C" int solattn_preprocess_int8(
+    const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k, int64_t sk_b,
+    int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b, int64_t sv_t, int64_t sv_h, int64_t B,
+    int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau, int64_t sink_kv_lo,
+    int64_t sink_kv_hi, int64_t sink_q_lo, int64_t sink_q_hi, int qk_block, uint16_t* kc, uint16_t* vc,
+    int64_t npad, float* qbar, float* kc_mean, float* kc_var, float* vamax_part, float* vscale,
+    float* thr, int32_t* counts, uint32_t* mask, int8_t* qi, float* qs, int8_t* ki, float* ks,
+    int8_t* vi, solattn_stream_t stream) {
+  clear_error();
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  SOLATTN_REQUIRE(D == kKernelD, SOLATTN_EUNSUPPORTED, "preprocess_int8: head_dim %lld != 128", (long long)D);
+  SOLATTN_REQUIRE(block == 64 || block == 128, SOLATTN_EUNSUPPORTED,
+                  "preprocess_int8: block %lld not in {64, 128}", (long long)block);
+  SOLATTN_REQUIRE(T > 0 && qi && qs && ki && ks && (!vscale || (vamax_part && vi)), SOLATTN_EINVAL,
+                  "preprocess_int8: empty sequence or null output");
+  SOLATTN_REQUIRE(npad >= cdiv(T, block) && npad < (1ll << 31), SOLATTN_EINVAL, "preprocess_int8: npad %lld",
+                  (long long)npad);
+  int rc = pool_checked(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H, D, block,
+                        kc, vc, npad, qbar, vscale ? vamax_part : nullptr, qk_block ? nullptr : qi,
+                        qk_block ? nullptr : qs, T, s, static_cast<int>(npad));
+  if (rc) return rc;
+  const int64_t NT = cdiv(T, block);
+  rc = moments(kc, npad, B, NT, H, D, 1, kc_mean, kc_var, vscale ? vamax_part : nullptr, vscale, s);
+  if (rc) return rc;
+  rc = route(qbar, kc, npad, nullptr, kc_var, B, T, H, D, block, scale, tau, 1, sink_kv_lo, sink_kv_hi,
+             sink_q_lo, sink_q_hi, thr, counts, mask, s);
+  if (rc) return rc;
+  return quant_qkv(qk_block ? q : nullptr, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T,
+                   H, D, kc_mean, vscale, qi, qs, ki, ks, vi, T, s, qk_block, /*ks_head_major=*/0);
 }

@@ -105,12 +105,13 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // The stages of the one-call pipelines for head dims 128 and (BF16 only) 64;
 // arguments are validated as in the public entry points, which take 128 alone.
 // pool_checked: the pooling pass (prep.hip) with, when qi != null, the per-token
-// INT8 of q (codes qi [B, TP, H, 128], scales qs [B, TP, H]) in the same read.
+// INT8 of q (codes qi [B, TP, H, 128], scales qs [B, TP, H]) in the same read;
+// rows [NT, zero_to) of kc and vc are zeroed.
 int pool_checked(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const uint16_t* k,
                  int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b,
                  int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t D,
                  int64_t block, uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar,
-                 float* vamax_part, int8_t* qi, float* qs, int64_t TP, hipStream_t s);
+                 float* vamax_part, int8_t* qi, float* qs, int64_t TP, hipStream_t s, int zero_to = 0);
 int moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H, int64_t D, int centre,
             float* kc_mean, float* kc_var, const float* vamax_part, float* vscale, hipStream_t s);
 int route(const float* qbar, const uint16_t* kc, int64_t npad, const float* kc_mean, const float* kc_var,

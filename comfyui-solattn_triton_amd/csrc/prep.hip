@@ -185,7 +185,7 @@ pool_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t 
             const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_t, int64_t sv_h, int64_t T,
             int H, int NT, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int64_t npad,
             float* __restrict__ qbar, float* __restrict__ vamax_part, int8_t* __restrict__ qi,
-            float* __restrict__ qs, int64_t TP) {
+            float* __restrict__ qs, int64_t TP, int zero_to) {
   constexpr int NB = kSpan / BLK;
   __shared__ __align__(16) float part[NB * kSlots * kHeadDim];
   __shared__ __align__(16) float amx[AMAX ? NB * kSlots * kHeadDim : 4];
@@ -243,6 +243,10 @@ pool_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t 
     __syncthreads();
     pool_q();
   }
+  // the padding rows of kc and vc, by the head's last workgroup
+  if (zero_to > NT && blockIdx.y == gridDim.y - 1 && h < H)
+    for (int r = NT + blk; r < zero_to; r += kPoolThreads / kHeadDim)
+      kc[((b * npad + r) * H + h) * HD + ch] = vc[((b * npad + r) * H + h) * HD + ch] = 0;
 }
 
 // --------------------------------------------------------------- moments --
@@ -937,7 +941,7 @@ int launch_pool(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, con
                 int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b,
                 int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t D, int64_t block,
                 uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar, float* vamax_part,
-                int8_t* qi, float* qs, int64_t TP, hipStream_t s) {
+                int8_t* qi, float* qs, int64_t TP, int zero_to, hipStream_t s) {
   const int64_t NT = cdiv(T, block);
   const int64_t spans = cdiv(T, kSpan);
   SOLATTN_REQUIRE(spans <= 65535 && B <= 65535 && H <= 65535, SOLATTN_EUNSUPPORTED,
@@ -963,7 +967,7 @@ int launch_pool(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, con
                 : (amax ? pool_kernel<128, false, true> : pool_kernel<128, false, false>));
   hipLaunchKernelGGL(kern, grid, dim3(kPoolThreads), 0, s, q, sq_b, sq_t, sq_h, k, sk_b, sk_t,
                      sk_h, v, sv_b, sv_t, sv_h, T, static_cast<int>(H), static_cast<int>(NT), kc,
-                     vc, npad, qbar, vamax_part, qi, qs, TP);
+                     vc, npad, qbar, vamax_part, qi, qs, TP, zero_to);
   return check_launch("pool");
 }
 
@@ -975,7 +979,7 @@ int pool_checked(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, co
                  int64_t sk_b, int64_t sk_t, int64_t sk_h, const uint16_t* v, int64_t sv_b,
                  int64_t sv_t, int64_t sv_h, int64_t B, int64_t T, int64_t H, int64_t D,
                  int64_t block, uint16_t* kc, uint16_t* vc, int64_t npad, float* qbar,
-                 float* vamax_part, int8_t* qi, float* qs, int64_t TP, hipStream_t s) {
+                 float* vamax_part, int8_t* qi, float* qs, int64_t TP, hipStream_t s, int zero_to) {
   SOLATTN_REQUIRE(D == kHeadDim || D == 64, SOLATTN_EUNSUPPORTED, "pool: head_dim %lld", (long long)D);
   SOLATTN_REQUIRE(block == 64 || block == 128, SOLATTN_EUNSUPPORTED, "pool: block %lld not in {64, 128}",
                   (long long)block);
@@ -989,7 +993,7 @@ int pool_checked(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, co
   if (int rc = check_bthd(k, sk_b, sk_t, sk_h, "pool k")) return rc;
   if (int rc = check_bthd(v, sv_b, sv_t, sv_h, "pool v")) return rc;
   return launch_pool(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H, D,
-                     block, kc, vc, npad, qbar, vamax_part, qi, qs, TP, s);
+                     block, kc, vc, npad, qbar, vamax_part, qi, qs, TP, zero_to, s);
 }
 
 }  // namespace solattn

@@ -182,6 +182,25 @@ int solattn_quant_v(const uint16_t* v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
                     int64_t T, int64_t H, int64_t D, const float* vscale, int8_t* vi,
                     int64_t TP, solattn_stream_t stream);
 
+/* ------------------------------------------------------ INT8 preparation --
+ * Everything the INT8 forward reads, in four launches: pool with the per-token
+ * Q codes from the same read, moments (centre = 1), route (mode 1), then the
+ * smoothed K codes and (vscale != NULL, which also needs vamax_part and vi) the
+ * V codes in one launch. The outputs and layouts are those of solattn_pool,
+ * solattn_moments, solattn_route, solattn_quant_rows and solattn_quant_v with
+ * TP = T, bit for bit; rows [NT, npad) of kc and vc are zeroed. qk_block != 0: Q
+ * and K codes as solattn_quant_rows_blocked (Q is then read twice).
+ * Replaces: fused_preprocess, /root/reference/_fused_prep.py:62-98. */
+int solattn_preprocess_int8(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
+                            const uint16_t* k, int64_t sk_b, int64_t sk_t, int64_t sk_h,
+                            const uint16_t* v, int64_t sv_b, int64_t sv_t, int64_t sv_h, int64_t B,
+                            int64_t T, int64_t H, int64_t D, int64_t block, float scale, float tau,
+                            int64_t sink_kv_lo, int64_t sink_kv_hi, int64_t sink_q_lo,
+                            int64_t sink_q_hi, int qk_block, uint16_t* kc, uint16_t* vc, int64_t npad,
+                            float* qbar, float* kc_mean, float* kc_var, float* vamax_part,
+                            float* vscale, float* thr, int32_t* counts, uint32_t* mask, int8_t* qi,
+                            float* qs, int8_t* ki, float* ks, int8_t* vi, solattn_stream_t stream);
+
 /* ------------------------------------------------------- single-read INT8 --
  * The INT8 path's preparation with one read of q, k and v: pooled keys and
  * values, query centroids, centred kc and its moments (solattn_moments with

@@ -592,3 +592,31 @@ def test_one_call_equals_its_stages(pkg, dev, NT, mode):
         r, *codes = fp.fused_preprocess_routing(q, k, v, scale=128 ** -0.5, int8_pv=pv, **kw)
         two = i8.forward_int8(q, v, r, *codes, int8_pv=pv)
     assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("T,block,H,quant_block", [(1, 64, 1, None), (64 * 64, 64, 2, None), (64 * 63 + 9, 64, 3, 128),
+                                                   (128 * 65 + 1, 128, 2, None), (777, 128, 3, 128)])
+@pytest.mark.parametrize("int8_pv", [True, False])
+def test_preprocess_one_call(pkg, dev, T, block, H, quant_block, int8_pv):
+    """The INT8 preparation's one call against the oracle, bit for bit, with the
+    padding rows of kc and vc zeroed in memory that held something else."""
+    fp = _mods(pkg)[3]
+    B = 2
+    q, k, v = (randn_bf16((B, T, H, 128), s) for s in (31, 32, 33))
+    junk = torch.full((64 << 20,), 7, dtype=torch.uint8, device=dev)  # recycled by the outputs
+    del junk
+    print(f"[preprocess] T={T} block={block} H={H} quant_block={quant_block} pv={int8_pv}", flush=True)
+    r, qi, qs, ki, ks, vi = fp.fused_preprocess_routing(q.to(dev), k.to(dev), v.to(dev), tau=0.8,
+                                                        scale=128 ** -0.5, block=block, int8_pv=int8_pv,
+                                                        quant_block=quant_block)
+    ref = oracle.prepare(bits(q), bits(k), bits(v), block=block, tau=0.8, int8=True, int8_pv=int8_pv,
+                         **({"quant_block": 128} if quant_block else {}))
+    NT = ref["NT"]
+    for name, t in (("kc", r.kc), ("vc", r.vc)):
+        assert np.array_equal(bits(t)[:, :NT], ref[name][:, :NT]) and not bits(t)[:, NT:].any()
+    f32 = lambda t: t.cpu().numpy().view(np.uint32)  # noqa: E731
+    assert np.array_equal(f32(r.threshold), ref["thr"].view(np.uint32))
+    assert np.array_equal(u32(r.mask), ref["mask"]) and np.array_equal(r.counts.cpu().numpy(), ref["counts"])
+    for name, t in (("qi", qi), ("ki", ki)) + ((("vi", vi),) if int8_pv else ()):
+        assert np.array_equal(t.cpu().numpy(), ref[name]), name
+    assert np.array_equal(f32(qs), ref["qs"].view(np.uint32)) and np.array_equal(f32(ks), ref["ks"].view(np.uint32))

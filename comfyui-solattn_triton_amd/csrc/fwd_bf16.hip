@@ -104,13 +104,17 @@ __device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
     const float m_new = new_max(st.m, xhalf_max(mx) * c, alpha);
-    if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
+    // A first half tile without a single unmasked pooled key (its 32 blocks all
+    // exact) leaves the max at -inf: its P are 0, not exp2(-inf + inf).
+    const bool none = POOLED && m_new == -INFINITY;
+    if (__any(m_new != st.m || none)) {  // lanes whose max stays recompute the same P
       st.m = m_new;
       psum = 0.f;
       if constexpr (POOLED) {
+        const float neg_new = none ? 0.f : -m_new;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r], c, -m_new));
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r], c, neg_new));
           pn[r >> 3][r & 7] = static_cast<__bf16>(p);
           psum += p;
         }

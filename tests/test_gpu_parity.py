@@ -515,21 +515,13 @@ def test_head_dim_64(pkg, dev, mode, case):
         assert err < BF16_MAXABS and cos >= BF16_COS
 
 
-@pytest.mark.parametrize("block,T", [(64, 64 * 70 + 17), (64, 64 * 64), (128, 128 * 66 + 64), (128, 128 * 65 + 90)])
-def test_fwd_bf16_hand_set_masks(pkg, dev, block, T):
-    """Tile orders the router never gives: rows with no exact block (pooled tiles
-    only, a partial chunk and a short last block among them), with the last block
-    alone, with the first alone, with every second block. Against float64: P and
-    the outputs are rounded to bf16 (2^-9 each) under values of order 1, far
-    inside BF16_MAXABS."""
+def _check_hand_set_masks(pkg, dev, block, T, exact_rows):
+    """The BF16 forward under hand-set exact blocks against float64 over the same pooled rows."""
     prep, tri = _mods(pkg)[0], _mods(pkg)[1]
     q, k, v = (randn_bf16((1, T, 1, 128), s) for s in (90, 91, 92))
     r = prep.route(q.to(dev), k.to(dev), v.to(dev), scale=128 ** -0.5, tau=0.9, block=block)
     NT = r.counts.shape[-1]
-    exact = torch.zeros(4, NT, dtype=torch.bool)
-    exact[1, NT - 1] = exact[2, 0] = True
-    exact[3, ::2] = True
-    rows = exact[torch.arange(NT) % 4]  # [query block, key block]
+    rows = exact_rows(NT)  # [query block, key block]
     j = torch.arange(NT)
     words = torch.zeros(NT, r.mask.shape[-1], dtype=torch.int64)
     words.index_add_(1, j >> 5, rows.long() << (j & 31))
@@ -548,6 +540,35 @@ def test_fwd_bf16_hand_set_masks(pkg, dev, block, T):
     ref = (s @ vd + p @ vc) / (s.sum(1) + p @ lens)[:, None]
     assert float((out - ref).abs().max()) < BF16_MAXABS
     assert cosine(out.numpy(), ref.numpy()) >= BF16_COS
+
+
+@pytest.mark.parametrize("block,T", [(64, 64 * 70 + 17), (64, 64 * 64), (128, 128 * 66 + 64), (128, 128 * 65 + 90)])
+def test_fwd_bf16_hand_set_masks(pkg, dev, block, T):
+    """Tile orders the router never gives: rows with no exact block (pooled tiles
+    only, a partial chunk and a short last block among them), with the last block
+    alone, with the first alone, with every second block. Against float64: P and
+    the outputs are rounded to bf16 (2^-9 each) under values of order 1, far
+    inside BF16_MAXABS."""
+    def exact_rows(NT):
+        exact = torch.zeros(4, NT, dtype=torch.bool)
+        exact[1, NT - 1] = exact[2, 0] = True
+        exact[3, ::2] = True
+        return exact[torch.arange(NT) % 4]
+
+    _check_hand_set_masks(pkg, dev, block, T, exact_rows)
+
+
+@pytest.mark.parametrize("block,T", [(64, 64 * 70), (128, 128 * 66)])
+def test_fwd_bf16_half_chunk_exact(pkg, dev, block, T):
+    """The first half tile of pooled keys without a pooled key (its 32 blocks all
+    exact, as behind a sink of 32 blocks), alone and with the next one; lengths of
+    whole blocks, so that no plain tile comes before it."""
+    def exact_rows(NT):
+        exact = torch.zeros(3, NT, dtype=torch.bool)
+        exact[0, :32] = exact[1, :63] = exact[2, 32:64] = True
+        return exact[torch.arange(NT) % 3]
+
+    _check_hand_set_masks(pkg, dev, block, T, exact_rows)
 
 
 @pytest.mark.parametrize("D", [8, 40, 64])

@@ -6,6 +6,8 @@ the oracle's restatement of the reference loop within max-abs 2e-2 and cosine
 >= 0.9995 (BF16) / cosine >= 0.999 (INT8).
 """
 
+import importlib
+
 import numpy as np
 import pytest
 import torch
@@ -161,6 +163,28 @@ def test_reorder_matches_index_select(pkg, dev):
     s = randn_bf16((500, 256), 8).to(dev)
     idx = torch.randperm(500, generator=torch.Generator().manual_seed(1)).to(dev)
     assert torch.equal(mort.reorder_tokens(s, idx, dim=0), s[idx])
+
+
+@pytest.mark.parametrize("chunks", [1, 39, 40, 41, 63, 64, 65, 128, 129, 449, 511, 512, 513, 1025])
+def test_reorder_row_lengths(pkg, dev, chunks):
+    """Rows around the lengths where the copy changes form (40 chunks of 16 bytes,
+    one more load per lane, one more pass of 512), strided source rows, a row count that leaves waves idle,
+    and an index outside the source (its row is zeroed)."""
+    mod, capi = _mods(pkg)[5], importlib.import_module(f"{pkg.__name__}._capi")
+    print(f"[reorder rows] chunks={chunks}", flush=True)
+    g = torch.Generator().manual_seed(chunks)
+    wide = torch.randn(2, 37, chunks * 8 + 8, generator=g).to(torch.bfloat16).to(dev)
+    x = wide[..., : chunks * 8]
+    idx = torch.randint(0, 37, (41,), generator=g).to(dev)
+    assert torch.equal(mod.reorder_tokens(x.contiguous(), idx, dim=1), x[:, idx])
+    out = torch.full((2, 41, chunks * 8), 7.0, dtype=torch.bfloat16, device=dev)
+    bad = idx.clone()
+    bad[3], bad[40] = -1, 37
+    capi.call("solattn_reorder_rows", capi.ptr(x), 37, x.stride(0) * 2, x.stride(1) * 2, capi.ptr(out),
+              out.stride(0) * 2, out.stride(1) * 2, 2, 41, chunks * 16, capi.ptr(bad), capi.stream(dev))
+    want = x[:, idx].clone()
+    want[:, [3, 40]] = 0
+    assert torch.equal(out, want)
 
 
 FWD_CASES = [  # (B, T, H, block, tau, sink_kv, sink_q)

@@ -200,7 +200,7 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     if (t >= npool) {
       if (kv == 0) issue_k_at(first_of(t), hh); else issue_v_at(first_of(t), hh);
     } else {
-      issue_generic_half<NTHREADS, D>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, t, NT), hh, src);
+      issue_pooled_half<NTHREADS, D>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, t, NT), hh, src);
     }
   };
   const auto issue_start = [&] {  // what the first half steps need

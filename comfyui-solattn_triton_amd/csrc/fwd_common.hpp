@@ -344,22 +344,29 @@ __device__ __forceinline__ void issue_full(uint32_t dst, const uint16_t* base, i
   }
 }
 
-// The same for half a tile (32 keys): rows [32 hh, 32 hh + 32) of the tile `td`
-// (issue_generic_half) or a base at the half's first row (issue_half).
+// Copies of half a bf16 tile (32 keys) into the half buffer at LDS byte address
+// dst: rows [32 hh, 32 hh + 32) of the pooled tile `td` (issue_pooled_half; rows past
+// nvalid re-read its last one, finite data that the softmax masks out), or the rows
+// from `base` on, `stride` elements apart (issue_half).
 template <int NTHREADS, int D>
-__device__ __forceinline__ void issue_generic_half(uint32_t dst, int kv, const TileDesc& td, int hh,
-                                                   const KVSource& src) {
+__device__ __forceinline__ void issue_pooled_half(uint32_t dst, int kv, const TileDesc& td, int hh,
+                                                  const KVSource& src) {
   constexpr int C = D / 8, U = CopyOffsets<NTHREADS, D>::U / 2;
   const uint32_t l0 = dst + wave_id() * 64 * 16;
-  const uint16_t* b = kv == 0 ? (td.pooled ? src.kc : src.k) : (td.pooled ? src.vc : src.v);
-  const int64_t stride = td.pooled ? src.skc : (kv == 0 ? src.sk : src.sv);
+  const uint16_t* b = (kv == 0 ? src.kc : src.vc) +
+                      static_cast<int64_t>(__builtin_amdgcn_readfirstlane(td.first)) * src.skc;
+  // (the row stride fits 32 bits, as 128 rows of kc and vc fit the memory; 63 of them need not)
+  const uint32_t stride = static_cast<uint32_t>(src.skc * 2), top = static_cast<uint32_t>(td.nvalid - 1);
+  // The addresses are made at each copy, not held through the pipeline: 4-18
+  // registers fewer, and the BF16 call of 32760 tokens at block 64 2728 -> 2710 us.
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int e = threadIdx.x + NTHREADS * u;
-    const int row = 32 * hh + e / C, pc = e % C;
-    const int srow = td.first + (row < td.nvalid ? row : 0);
+    const uint32_t e = tid + NTHREADS * u, row = 32 * hh + e / C, pc = e % C;
     const int chunk = kv == 0 ? swz_k<D>(row, pc) : swz_v<D>(row, pc);
-    g2l16(b + static_cast<int64_t>(srow) * stride + chunk * 8, l0 + NTHREADS * u * 16);
+    g2l16(reinterpret_cast<const char*>(b) + (static_cast<uint64_t>(min(row, top)) * stride + chunk * 16),
+          l0 + NTHREADS * u * 16);
   }
 }
 template <int NTHREADS, int D>

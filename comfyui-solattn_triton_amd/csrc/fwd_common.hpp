@@ -277,14 +277,6 @@ __device__ __forceinline__ void g2l4_s(const void* base, uint32_t off, uint32_t 
 
 __device__ __forceinline__ void wait_tile_copies() { __builtin_amdgcn_s_waitcnt(0); }
 
-// s_waitcnt vmcnt(N): all but the N newest copies have landed (vmcnt is bits
-// [3:0] and [15:14]; expcnt and lgkmcnt stay at their maxima).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
-}
-
 // Copy the K (kv == 0) or V (kv == 1) rows of the bf16 tile `td` into an LDS
 // tile, each lane computing its own source rows: rows past nvalid re-read row
 // 0 of the tile (finite data that the softmax masks out). U copies per lane.
@@ -328,21 +320,6 @@ struct CopyOffsets {
     }
   }
 };
-
-// Copies of a full bf16 tile whose first row is at `base` (row stride
-// `stride` elements) into the LDS tile at byte address dst.
-template <int NTHREADS>
-__device__ __forceinline__ void issue_full(uint32_t dst, const uint16_t* base, int64_t stride,
-                                           const uint32_t (&off)[CopyOffsets<NTHREADS>::P]) {
-  using CO = CopyOffsets<NTHREADS>;
-  const uint32_t l0 = dst + wave_id() * 64 * 16;
-  const char* b = reinterpret_cast<const char*>(base);
-#pragma unroll
-  for (int u = 0; u < CO::U; ++u) {
-    const char* row_base = b + static_cast<int64_t>(u / CO::P) * CO::kStep * stride * 2;
-    g2l16_s(row_base, off[u % CO::P], l0 + NTHREADS * u * 16);
-  }
-}
 
 // Copies of half a bf16 tile (32 keys) into the half buffer at LDS byte address
 // dst: rows [32 hh, 32 hh + 32) of the pooled tile `td` (issue_pooled_half; rows past

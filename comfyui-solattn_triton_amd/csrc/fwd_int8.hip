@@ -9,15 +9,16 @@
 //     block is one 64-key tile (fwd_int8_kernel). Block 128:
 //     fwd_int8_b128_kernel works on whole 128-key blocks; the tiles of a
 //     ragged last block are quantised per 64-key tile.
-//   otherwise: P.V in bf16 against the bf16 V, as in the BF16 forward.
+//   otherwise: P.V in bf16 against the bf16 V, as in the BF16 forward
+//     (fwd_int8_bf16pv_kernel).
 // Pooled tiles run last in bf16 on the centred kc and vc. The online softmax
 // is exact under any tile order, up to fp32 rounding.
 //
 // Tile order: the ragged exact tile (if any) through a plain path, the full
-// exact tiles through a pipeline (step n: copies of K(n+2) and V(n+1); the i8
-// MFMAs of S(n+1) interleaved with the softmax of tile n; P(n).V(n), then the
-// conversion of S(n+1) to fp32 scores while tile n+1's ks are in LDS), then
-// the pooled tiles. Tiles are copied global -> LDS directly: int8 K and V rows
+// exact tiles through a pipeline (int8 P.V, step n: copies of K(n+2) and V(n+1);
+// the i8 MFMAs of S(n+1) interleaved with the softmax of tile n; P(n).V(n), then
+// the conversion of S(n+1) to fp32 scores while tile n+1's ks are in LDS; bf16
+// P.V: the BF16 forward's pipeline of half tiles), then the pooled tiles. Tiles are copied global -> LDS directly: int8 K and V rows
 // of 128 bytes with XOR-swizzled 16-byte chunks, ks behind the K rows;
 // ds_read_b64_tr_b8 delivers int8 V transposed as the MFMA A operand.
 #include "common.hpp"
@@ -28,6 +29,8 @@ namespace int8fwd {
 
 constexpr int kI8Row = kD;                  // bytes per int8 K / V row
 constexpr int kKsOffset = kKeys * kI8Row;   // ks[64] after the int8 K rows (bytes)
+constexpr int kHalfKs = 32 * kI8Row;        // ks[32] after the 32 int8 rows of a half tile
+constexpr int kHalfKStride = kHalfKs + 256;  // bytes of a half tile of K and its ks
 
 // 16 lanes per cycle read one 16-byte chunk of 16 consecutive rows; two 128-byte
 // rows share a bank sweep, so rows of equal parity need distinct chunks.
@@ -282,12 +285,6 @@ __device__ __forceinline__ void exact_softmax_pv(SoftmaxState& st, f32x16 (&s)[2
   }
 }
 
-// Pipelined step over full exact tile n (scaled scores in sc, factor qsl):
-// the i8 MFMAs of S(n+1) from the K tile kn are interleaved with the softmax
-// of tile n; then P(n).V(n) and the conversion of S(n+1) into sn (ks of tile
-// n+1 from kn).
-// mid(): called before P(n).V(n) reads the V tile (a single-buffered V tile
-// is waited for there).
 // asm i8 MFMAs of the hand-ordered step (hazards as for the bf16 ones in
 // fwd_common.hpp).
 __device__ __forceinline__ void mfma_i8_v0(i32x16& d, const i32x4& a, const i32x4& b) {
@@ -297,215 +294,93 @@ __device__ __forceinline__ void mfma_i8_v(i32x16& d, const i32x4& a, const i32x4
   asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
 }
 
-// bf16 P.V form of the pipelined step, hand-ordered like the BF16 forward's
-// steps: each of the 8 i8 score MFMAs of S(n+1) is followed by the exps of two
-// P(n) words; after mid(), each of the 16 P.V MFMAs by the conversion of two
-// int32 scores of S(n+1) to fp32 (times their ks). The K and V operands are
-// read two MFMAs ahead, the ks one group (four scores) ahead; the lazy tile
-// max is the BF16 forward's. (Spreading the exps over both phases, with the
-// tile max taken every step so that the P.V MFMAs could start on the first P
-// words, measured 7% slower.)
-template <bool UKS, typename Mid>
-__device__ __forceinline__ void fast_step_bf16pv(SoftmaxState& st, const f32x16 (&sc)[2],
-                                                 f32x16 (&sn)[2], const char* kn, const void* vt,
-                                                 const i32x4 (&qi)[4], float qsl, int lane,
-                                                 Mid&& mid) {
-  const int col = lane & 31, half = lane >> 5;
-  i32x16 si[2];
-  i32x4 ka[3];
-  bf16x8 va[3], pb[4];
-  uint32_t pw[4][4];
-  float psum = 0.f;
-  const float neg = -st.m;
-  const uint16_t* vtile = static_cast<const uint16_t*>(vt);
-  ka[0] = ki_op(kn, 0, 0, col, half);
-  ka[1] = ki_op(kn, 1, 0, col, half);
-  asm volatile("" ::: "memory");
-  const auto unit = [&](int u) {
-    const int ks = u >> 2, w = u & 3;
-    const int r = 8 * (ks & 1) + 2 * w;
-    pw[ks][w] = exp_pair(sc[ks >> 1][r], sc[ks >> 1][r + 1], qsl, neg, psum);
-  };
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if (i + 2 < 8) {
-      ka[(i + 2) % 3] = ki_op(kn, (i + 2) & 1, (i + 2) >> 1, col, half);
-      asm volatile("" ::: "memory");
-    }
-    if (i < 2)
-      mfma_i8_v0(si[i & 1], ka[i % 3], qi[i >> 1]);
-    else
-      mfma_i8_v(si[i & 1], ka[i % 3], qi[i >> 1]);
-    unit(2 * i);
-    unit(2 * i + 1);
-  }
-  // the int32 scores are read after this point: 16 VALU instructions (the
-  // last two exp pairs) follow the last score MFMA
-  asm volatile("" : "+v"(si[0]), "+v"(si[1]));
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    pb[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
-  float alpha = 1.f;
-  if (__any(!(psum <= 255.f))) {  // (also catches inf / NaN)
-    float mx = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
-    const float m_new = new_max(st.m, xhalf_max(mx) * qsl, alpha);
-    if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
-      st.m = m_new;
-      psum = 0.f;
-      psum = exp8<0>(sc[0], qsl, -m_new, pb[0], psum);
-      psum = exp8<8>(sc[0], qsl, -m_new, pb[1], psum);
-      psum = exp8<0>(sc[1], qsl, -m_new, pb[2], psum);
-      psum = exp8<8>(sc[1], qsl, -m_new, pb[3], psum);
-      mfma_fence(st.acc);  // the rescale reads O
-      rescale(st, alpha);
-    }
-  }
-  st.l = fmaf(st.l, alpha, psum);
-  mid();
-  // ks of score group g (elements 4(g%4) .. +3 of tile g/4): read one group
-  // ahead of its two slots
-  const float* ksl = reinterpret_cast<const float*>(kn + kKsOffset);
-  const auto ks_group = [&](int g) {
-    return *reinterpret_cast<const float4*>(ksl + 32 * (g >> 2) + 8 * (g & 3) + 4 * half);
-  };
-  float4 kq[2];
-  if constexpr (!UKS) kq[0] = ks_group(0);
-  const uint32_t vl = v_lane(lds_addr(vtile), lane);
-  va[0] = v_op_x(vl, 0, 0);
-  va[1] = v_op_x(vl, 0, 1);
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + 2 < 16) {
-      va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
-      if (!UKS && (i & 1) == 0 && (i >> 1) + 1 < 8) kq[((i >> 1) + 1) & 1] = ks_group((i >> 1) + 1);
-      asm volatile("" ::: "memory");
-    }
-    if (i == 0)
-      mfma_v_first(st.acc[0], va[0], pb[0]);
-    else
-      mfma_v(st.acc[i & 3], va[i % 3], pb[i >> 2]);
-    // scores 2i, 2i + 1 of S(n+1): element e of tile m (group i/2)
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int e2 = 2 * i + t, m = e2 >> 4, e = e2 & 15;
-      const float f = static_cast<float>(si[m][e]);
-      if constexpr (UKS) {
-        sn[m][e] = f;
-      } else {
-        const float4 kk = kq[(i >> 1) & 1];
-        const float kv = (e & 3) == 0 ? kk.x : (e & 3) == 1 ? kk.y : (e & 3) == 2 ? kk.z : kk.w;
-        sn[m][e] = f * kv;
-      }
-    }
-    asm volatile("" : "+v"(sn[i >> 3]));
-  }
-  mfma_fence(st.acc);  // O is read by plain code after the pipeline
+// Address of this lane's K operands in a 128-byte-aligned int8 K tile (or half
+// tile): operand cc of its first 32 keys sits at k ^ (cc << 5), as the swizzle
+// flips only chunk bits that cc shares with bits 5-6 of the address. The half
+// buffers are whole offsets behind it, so both share the operand addresses.
+__device__ __forceinline__ uint32_t ki_lane(uint32_t tile, int col, int half) {
+  return tile + col * kI8Row + 16 * swz_ki(col, half);
+}
+__device__ __forceinline__ i32x4 ki_op_x(uint32_t kl, int cc, int offset) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) i32x4*>(
+      static_cast<uintptr_t>((kl ^ static_cast<uint32_t>(cc << 5)) + offset));
+}
+__device__ __forceinline__ f32x4 ks_quad(uint32_t a) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(static_cast<uintptr_t>(a));
 }
 
-// Three-stage bf16 P.V step (block 128): S(n+1) = Ki(n+1) Qi^T (8 i8 MFMAs),
-// O += P(n-1) V(n-1) (16 bf16 MFMAs) and the softmax of S(n) in one
-// hand-ordered stream: slot i (16) issues score MFMA i (i < 8), the exps of P
-// word i, then P.V MFMA i; slots 8-15 also convert four int32 scores of S(n+1)
-// to fp32 times their ks (read two slots ahead, while tile n+1's ks are in
-// LDS). The last score MFMA is followed by two exp pairs and a P.V MFMA before
-// the int32 scores are read. QK = false: the last tile (no scores to make);
-// PV = false: the first. Lazy tile max, hazards and the final O rescale as
-// in the BF16 forward's half_step. qc: the factor of sc's scores.
-template <bool QK, bool PV, bool UKS>
-__device__ __forceinline__ void step3_i8(SoftmaxState& st, const f32x16 (&sc)[2], float qc,
-                                         f32x16 (&sn)[2], const bf16x8 (&pp)[4], bf16x8 (&pn)[4],
-                                         const char* kn, uint32_t vl, const i32x4 (&qi)[4],
-                                         int lane) {
-  const int col = lane & 31, half = lane >> 5;
-  i32x16 si[2];
+// bf16 P.V step over half tiles of 32 keys, the BF16 forward's half_step with
+// int8 scores: S(n+1) = Ki(n+1) Qi^T (4 i8 MFMAs), O += P(n-1) V(n-1) (8 bf16
+// MFMAs) and the softmax of S(n) in one hand-ordered stream: slot i issues score
+// MFMA i (i < 4), the exps of P(n) word i, then P.V MFMA i; slots 4-7 also
+// convert four int32 scores of S(n+1) to fp32 times their ks (read a slot
+// ahead). Two exp pairs and a P.V MFMA follow the last score MFMA before its
+// int32 scores are read. PV = false: the first half tile. Lazy tile max, hazards
+// and the O rescale as in half_step. qc: the factor of sc's scores; K(n+1), its
+// ks and V(n-1) are in half buffer HH, kl, ksl and vl this lane's operand addresses
+// in half buffer 0.
+template <int HH, bool PV, bool UKS>
+__device__ __forceinline__ void half_step_i8(SoftmaxState& st, const f32x16& sc, float qc, f32x16& sn,
+                                             const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
+                                             uint32_t ksl, uint32_t vl, const i32x4 (&qi)[4]) {
+  i32x16 si;
   i32x4 ka[3];
   bf16x8 va[3];
-  float4 kq[3];
-  uint32_t pw[4][4];
+  f32x4 kq[2];
+  uint32_t pw[2][4];
   float psum = 0.f;
   const float neg = -st.m;
-  const float* ksl = QK ? reinterpret_cast<const float*>(kn + kKsOffset) : nullptr;
-  const auto ks_group = [&](int g) {
-    return *reinterpret_cast<const float4*>(ksl + 32 * (g >> 2) + 8 * (g & 3) + 4 * half);
-  };
-  if constexpr (QK) {
-    ka[0] = ki_op(kn, 0, 0, col, half);
-    ka[1] = ki_op(kn, 1, 0, col, half);
-  }
+  ka[0] = ki_op_x(kl, 0, HH * kHalfKStride);
+  ka[1] = ki_op_x(kl, 1, HH * kHalfKStride);
   if constexpr (PV) {
-    va[0] = v_op_x(vl, 0, 0);
-    va[1] = v_op_x(vl, 0, 1);
+    va[0] = v_op_x(vl, 2 * HH, 0);
+    va[1] = v_op_x(vl, 2 * HH, 1);
   }
   asm volatile("" ::: "memory");
-  const auto unit = [&](int u) {
-    const int ks = u >> 2, w = u & 3;
-    const int r = 8 * (ks & 1) + 2 * w;
-    pw[ks][w] = exp_pair(sc[ks >> 1][r], sc[ks >> 1][r + 1], qc, neg, psum);
-  };
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if constexpr (QK) {
-      if (i + 2 < 8) ka[(i + 2) % 3] = ki_op(kn, (i + 2) & 1, (i + 2) >> 1, col, half);
-      if (!UKS && i >= 6 && i <= 13) kq[(i - 6) % 3] = ks_group(i - 6);
-    }
+  for (int i = 0; i < 8; ++i) {
+    if (i + 2 < 4) ka[(i + 2) % 3] = ki_op_x(kl, i + 2, HH * kHalfKStride);
+    if (!UKS && i >= 3 && i < 7) kq[(i - 3) & 1] = ks_quad(ksl + HH * kHalfKStride + 32 * (i - 3));
     if constexpr (PV) {
-      if (i + 2 < 16) va[(i + 2) % 3] = v_op_x(vl, (i + 2) >> 2, (i + 2) & 3);
+      if (i + 2 < 8) va[(i + 2) % 3] = v_op_x(vl, 2 * HH + ((i + 2) >> 2), (i + 2) & 3);
     }
     asm volatile("" ::: "memory");
-    if constexpr (QK) {
-      if (i < 2)
-        mfma_i8_v0(si[i & 1], ka[i % 3], qi[i >> 1]);
-      else if (i < 8)
-        mfma_i8_v(si[i & 1], ka[i % 3], qi[i >> 1]);
-    }
-    unit(i);
+    if (i == 0)
+      mfma_i8_v0(si, ka[0], qi[0]);
+    else if (i < 4)
+      mfma_i8_v(si, ka[i % 3], qi[i]);
+    pw[i >> 2][i & 3] = exp_pair(sc[2 * i], sc[2 * i + 1], qc, neg, psum);
     if constexpr (PV) {
       if (i == 0)
         mfma_v_first(st.acc[0], va[0], pp[0]);
       else
         mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
     }
-    if constexpr (QK) {
-      if (i == 8) asm volatile("" : "+v"(si[0]), "+v"(si[1]));  // the int32 scores are read after this
-      if (i >= 8) {
-        const int g = i - 8, m = g >> 2, e0 = 4 * (g & 3);
-        const float4 kk = kq[g % 3];
+    if (i == 4) asm volatile("" : "+v"(si));  // the int32 scores are read after this
+    if (i >= 4) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const float f = static_cast<float>(si[m][e0 + t]);
-          if constexpr (UKS) {
-            sn[m][e0 + t] = f;
-          } else {
-            const float kv = t == 0 ? kk.x : t == 1 ? kk.y : t == 2 ? kk.z : kk.w;
-            sn[m][e0 + t] = f * kv;
-          }
-        }
-        asm volatile("" : "+v"(sn[m]));
+      for (int e = 4 * (i - 4); e < 4 * (i - 3); ++e) {
+        const float f = static_cast<float>(si[e]);
+        sn[e] = UKS ? f : f * kq[(i - 4) & 1][e & 3];
       }
+      asm volatile("" : "+v"(sn));
     }
     if (i == 0) __builtin_amdgcn_s_setprio(1);
   }
   __builtin_amdgcn_s_setprio(0);
-  if constexpr (!QK) mfma_fence(st.acc);  // the plain path's builtin MFMAs follow
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
+  for (int ks = 0; ks < 2; ++ks)
     pn[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
   float alpha = 1.f;
   if (__any(!(psum <= 255.f))) {  // (also catches inf / NaN)
     float mx = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
     const float m_new = new_max(st.m, xhalf_max(mx) * qc, alpha);
     if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
       st.m = m_new;
-      psum = 0.f;
-      psum = exp8<0>(sc[0], qc, -m_new, pn[0], psum);
-      psum = exp8<8>(sc[0], qc, -m_new, pn[1], psum);
-      psum = exp8<0>(sc[1], qc, -m_new, pn[2], psum);
-      psum = exp8<8>(sc[1], qc, -m_new, pn[3], psum);
+      psum = exp8<0>(sc, qc, -m_new, pn[0], 0.f);
+      psum = exp8<8>(sc, qc, -m_new, pn[1], psum);
       if constexpr (PV) mfma_fence(st.acc);  // the rescale reads O
       rescale(st, alpha);
     }
@@ -513,26 +388,22 @@ __device__ __forceinline__ void step3_i8(SoftmaxState& st, const f32x16 (&sc)[2]
   st.l = fmaf(st.l, alpha, psum);
 }
 
-template <bool INT8_PV, bool UKS, bool RUN, typename Mid>
+// Pipelined step over full exact tile n (scaled scores in sc, factor qsl):
+// the i8 MFMAs of S(n+1) from the K tile kn are interleaved with the softmax
+// of tile n; then P(n).V(n) and the conversion of S(n+1) into sn (ks of tile
+// n+1 from kn).
+template <bool UKS, bool RUN>
 __device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32x16 (&sn)[2],
-                                          const char* kn, const void* vt, const i32x4 (&qi)[4],
-                                          float qsl, int lane, Mid&& mid) {
-  if constexpr (!INT8_PV) {
-    fast_step_bf16pv<UKS>(st, sc, sn, kn, vt, qi, qsl, lane, mid);
-    return;
-  }
+                                          const char* kn, const char* vt, const i32x4 (&qi)[4],
+                                          float qsl, int lane) {
   const int col = lane & 31, half = lane >> 5;
   const i32x16 zero = {};
   i32x16 si[2];
   i32x4 ka[4][2];
-  // bf16 P.V: lazy tile max, as in the BF16 forward's steps (the exps use the
-  // running max as it stands; the tile max is taken only when a lane's row
-  // sum exceeds 255, or is inf on a first tile with the running max -inf), so
-  // the running max evolves as if taken every tile. int8 P.V needs the block
-  // max itself: its P codes are relative to it (RUN: to the running max).
-  float mx = -INFINITY, alpha = 1.f, bmax = 0.f, neg = INT8_PV ? 0.f : -st.m, psum = 0.f;
+  // The P codes are relative to the block's own max (RUN: to the running max),
+  // so the max is taken before them.
+  float mx = -INFINITY, alpha = 1.f, bmax = 0.f;
   uint32_t csum = 0u;
-  bf16x8 pb[4];
   i32x4 pi[2];
   ka[0][0] = ki_op(kn, 0, 0, col, half);
   ka[0][1] = ki_op(kn, 1, 0, col, half);
@@ -544,7 +415,7 @@ __device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32
     }
     si[0] = mfma_i8(ka[cc][0], qi[cc], cc == 0 ? zero : si[0]);
     si[1] = mfma_i8(ka[cc][1], qi[cc], cc == 0 ? zero : si[1]);
-    if (cc == 0 && INT8_PV) {
+    if (cc == 0) {
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
@@ -556,56 +427,20 @@ __device__ __forceinline__ void fast_step(SoftmaxState& st, f32x16 (&sc)[2], f32
       } else {
         st.m = new_max(st.m, bmax, alpha);
       }
-      neg = -st.m;
-    } else if (cc == 1) {
-      if constexpr (INT8_PV) {
-        csum = probs_i8(sc[0], qsl, kLog2_127 - bmax, pi[0], csum);
-      } else {
-        psum = exp8<0>(sc[0], qsl, neg, pb[0], psum);
-        psum = exp8<8>(sc[0], qsl, neg, pb[1], psum);
-      }
-    } else if (cc == 2) {
-      if constexpr (INT8_PV) {
-        csum = probs_i8(sc[1], qsl, kLog2_127 - bmax, pi[1], csum);
-      } else {
-        psum = exp8<0>(sc[1], qsl, neg, pb[2], psum);
-        psum = exp8<8>(sc[1], qsl, neg, pb[3], psum);
-        if (__any(!(psum <= 255.f))) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
-          const float m_new = new_max(st.m, xhalf_max(mx) * qsl, alpha);
-          if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
-            st.m = m_new;
-            neg = -m_new;
-            psum = 0.f;
-            psum = exp8<0>(sc[0], qsl, neg, pb[0], psum);
-            psum = exp8<8>(sc[0], qsl, neg, pb[1], psum);
-            psum = exp8<0>(sc[1], qsl, neg, pb[2], psum);
-            psum = exp8<8>(sc[1], qsl, neg, pb[3], psum);
-          }
-        }
-      }
+    } else if (cc < 3) {
+      csum = probs_i8(sc[cc - 1], qsl, kLog2_127 - bmax, pi[cc - 1], csum);
     }
   }
   float beta = 1.f;
-  if constexpr (INT8_PV && RUN) {
+  if constexpr (RUN) {
     st.l += static_cast<float>(csum);
-  } else if constexpr (INT8_PV) {
+  } else {
     beta = __builtin_amdgcn_exp2f(bmax - st.m);
     st.l = fmaf(st.l, alpha, beta * (1.f / 127.f) * static_cast<float>(csum));
-  } else {
-    st.l = fmaf(st.l, alpha, psum);
+    rescale(st, alpha);
   }
-  if constexpr (!RUN) rescale(st, alpha);
-  if constexpr (INT8_PV) {
-    scale_scores<UKS>(kn, si, half, sn);  // frees the int32 scores before the P.V accumulators
-    mid();
-    pv_i8<RUN>(static_cast<const char*>(vt), pi, beta * (1.f / 127.f), lane, st.acc);
-  } else {
-    mid();
-    pv_tile(static_cast<const uint16_t*>(vt), pb, lane, st.acc);
-    scale_scores<UKS>(kn, si, half, sn);
-  }
+  scale_scores<UKS>(kn, si, half, sn);  // frees the int32 scores before the P.V accumulators
+  pv_i8<RUN>(vt, pi, beta * (1.f / 127.f), lane, st.acc);
 }
 
 // ------------------------------------------------------------------ copies
@@ -673,51 +508,252 @@ __device__ __forceinline__ void issue_i8(uint32_t dst, const int8_t* rows, const
   }
 }
 
-// K and V tiles double buffered. Block 128: 68 KB of LDS, two workgroups per
-// CU, two waves per SIMD. Block 64: packed int8 K tiles, double buffered; with
-// int8 P.V packed int8 V too, double buffered (37 KB, four workgroups per CU),
-// with bf16 P.V one bf16 V tile (VSINGLE: 36 KB, four workgroups per CU, two
-// waves on every SIMD), copied after the step's P.V and waited for before the
-// next one's.
-template <int BLK, bool INT8_PV, bool UKS, bool RUN>
-__global__ void __launch_bounds__(BLK * 2)
+// K rows [first, first + 32) of ki and their ks into an LDS half tile (the waves
+// copy 32 / nwaves ks each).
+template <int NTHREADS>
+__device__ __forceinline__ void issue_ki_half(uint32_t dst, const I8Source& is, int first, uint32_t off) {
+  const int wave = wave_id();
+#pragma unroll
+  for (int u = 0; u < 256 / NTHREADS; ++u)
+    g2l16_s(reinterpret_cast<const char*>(is.ki) + static_cast<int64_t>(first + u * (NTHREADS / 8)) * is.srow,
+            off, dst + (wave * 64 + NTHREADS * u) * 16);
+  // the lane index is made here: held through the pipeline, its offset was spilled,
+  // and the reload waited for the copies above
+  constexpr uint32_t kpw = 32 * 64 / NTHREADS;
+  uint32_t lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  if (lane < kpw)
+    g2l4_s(is.ks + static_cast<int64_t>(first + kpw * wave) * is.kst, lane * static_cast<uint32_t>(is.kst * 4),
+           dst + kHalfKs + 4 * kpw * wave);
+}
+
+// The forward with bf16 P.V. Tile order: the ragged exact tile (plain, masked),
+// the full exact tiles through a pipeline of half tiles (32 keys), the pooled
+// tiles (plain). On entry to half step n: S(n) and P(n-1) in registers, K(n+1)
+// and V(n-1) in LDS; the step copies K(n+2) over K(n) and V(n) over V(n-2), so
+// every copy has a whole step to land. Two waves per SIMD (four workgroups per
+// CU at block 64, two at block 128).
+//
+// Bound: the VALU. A wave's half step takes about 650 cycles of it (16 exps at a
+// quarter of the rate, 16 fma, 32 conversions and scalings, the packing and row
+// sums) against 384 of its MFMAs, and two waves share a SIMD. Against a two-stage
+// step with a single-buffered V tile at block 64 and a three-stage step over whole
+// tiles at block 128: 15990 tokens 825 -> 818 and 747 -> 741 us, 7280 tokens 189 ->
+// 186 and 181 -> 177, 32760 tokens 2757 -> 2748 and 2350 -> 2346, 2040 tokens 68.4
+// -> 67.4 and 72.0 -> 72.1. All exps in the four slots with a score MFMA: 0.9%
+// faster at block 64, 0.8% slower at block 128.
+template <int BLK, bool UKS>
+__global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))
+fwd_int8_bf16pv_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
+                       const int8_t* __restrict__ qi, const float* __restrict__ qs,
+                       const int8_t* __restrict__ ki, const float* __restrict__ ks,
+                       const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
+                       int64_t TP, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+                       int64_t npad, const int32_t* __restrict__ counts,
+                       const uint32_t* __restrict__ mask, int T, int H, int NT, int W, float c,
+                       uint16_t* __restrict__ o, int64_t so_b, int64_t so_t, int64_t so_h, int kst,
+                       int64_t ksh) {
+  constexpr int NTHREADS = BLK * 2;
+  // LDS: K(i) and V(i), i < 2, half tiles; a whole tile spans the two (the ragged
+  // tile: 64 int8 rows and their ks). Pooled tiles: whole bf16 K and V tiles,
+  // double buffered at block 128.
+  constexpr uint32_t kVHalf = kTileBytes / 2, kVBase = 2 * kHalfKStride;
+  constexpr int PNBUF = BLK == 128 ? 2 : 1;
+  static_assert(kVBase + 2 * kVHalf <= 2 * kTileBytes && kKsOffset + 256 <= static_cast<int>(kVBase),
+                "exact tiles must fit");
+  static_assert(kVBase % 256 == 0, "V tiles are addressed by XOR");
+  __shared__ __align__(256) char arena[PNBUF * 2 * kTileBytes];
+  __shared__ TileList tl;
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  int bh, qb;
+  tile_coords_lpt<kLptTokens / BLK>(counts, NT, bh, qb);
+  const int b = bh / H, h = bh % H;
+  const int64_t row = static_cast<int64_t>(bh) * NT + qb;
+
+  const int ntiles = build_tile_list<BLK>(tl, mask, row, NT, W, T);
+  if (ntiles == 0) return;  // cannot happen for routed masks: the diagonal is exact
+  const int nrag = ragged_tiles(tl, NT, T);
+  const int nfast = tl.nexact - nrag;  // list tiles [0, nfast); the ragged one is the last exact one
+  const int npool = ntiles - tl.nexact;
+
+  const int64_t bhD = (static_cast<int64_t>(b) * npad * H + h) * kD;
+  const KVSource src{nullptr, 0, v + b * sv_b + h * sv_h, sv_t, kc + bhD,
+                     static_cast<int64_t>(H) * kD, vc + bhD};
+  const I8Source is{ki + (static_cast<int64_t>(b) * TP * H + h) * kD,
+                    ks + static_cast<int64_t>(b) * TP * H + h * ksh, nullptr,
+                    static_cast<int64_t>(H) * kD, kst};
+  // this lane's chunk of an int8 half tile, and its bf16 V chunks
+  const uint32_t k_off = static_cast<uint32_t>((threadIdx.x >> 3) * is.srow +
+                                               swz_ki(threadIdx.x >> 3, threadIdx.x & 7) * 16);
+  CopyOffsets<NTHREADS> off;
+  off.init(0, sv_t);
+  const uint32_t kb = lds_addr(arena), vb = kb + kVBase;  // LDS byte addresses
+  const auto first_of = [&](int e) { return exact_first<BLK>(tl, e); };
+  const auto issue_k = [&](int first, int hh) {
+    issue_ki_half<NTHREADS>(kb + hh * kHalfKStride, is, first + 32 * hh, k_off);
+  };
+  const auto issue_v = [&](int first, int hh) {
+    issue_half<NTHREADS, kD>(vb + hh * kVHalf, src.v + static_cast<int64_t>(first + 32 * hh) * src.sv,
+                             src.sv, off.v);
+  };
+  const auto issue_start = [&] {  // what the first half steps need
+    const int first = first_of(0);
+    issue_k(first, 0);
+    issue_k(first, 1);
+    issue_v(first, 0);
+  };
+  const auto issue_pooled = [&](int p) {
+    const TileDesc td = pooled_desc(tl, p, NT);
+    const uint32_t d = kb + (PNBUF == 2 ? p & 1 : 0) * 2 * kTileBytes;
+    issue_generic<NTHREADS>(d, 0, td, src);
+    issue_generic<NTHREADS>(d + kTileBytes, 1, td, src);
+  };
+  if (nrag) {
+    const TileDesc td = exact_desc<BLK>(tl, nfast, T, NT);
+    issue_i8<NTHREADS, false, true>(kb, is.ki, is, td.first, td.nvalid, 0, 0, false);
+    issue_generic<NTHREADS>(vb, 1, td, src);
+  } else if (nfast > 0) {
+    issue_start();
+  }
+
+  const int qrow = qb * BLK + wave * 32 + col;
+  const int qread = min(qrow, T - 1);  // rows past T repeat row T - 1 and are not stored
+  SoftmaxState st;
+  st.init();
+  const auto land = [] {
+    wait_tile_copies();
+    __syncthreads();
+  };
+
+  // ---- exact tiles (int8 Q: 16 VGPRs)
+  if (nrag + nfast > 0) {
+    i32x4 qireg[4];
+    const int64_t qoff = (static_cast<int64_t>(b) * TP + qread) * H + h;
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc)
+      qireg[cc] = __builtin_bit_cast(i32x4, *reinterpret_cast<const uint4*>(qi + qoff * kD + half * 16 + cc * 32));
+    const float qsl = qs[qoff] * c;
+    if (nrag) {
+      land();
+      const TileDesc td = exact_desc<BLK>(tl, nfast, T, NT);
+      i32x16 si[2];
+      f32x16 s[2];
+      qk_i8_tile(arena, qireg, col, half, si);
+      scale_scores<UKS>(arena, si, half, s);
+      mask_scores(s, td.amask);
+      exact_softmax_pv<false>(st, s, arena + kVBase, tile_qsl<UKS>(arena, kKsOffset, qsl), lane);
+      __syncthreads();  // every wave is done with K and V
+      if (nfast > 0) issue_start();
+    }
+    if (nfast > 0) {
+      // lane addresses of the K, ks and V operands in half buffer 0
+      const uint32_t kl = ki_lane(kb, col, half), ksl = kb + kHalfKs + 16 * half, vl = v_lane(vb, lane);
+      // the factor of half buffer hh's scores
+      const auto factor = [&](int hh) { return tile_qsl<UKS>(arena + hh * kHalfKStride, kHalfKs, qsl); };
+      f32x16 sa, sb;
+      bf16x8 pa[2], pb[2];
+      land();
+      {
+        const i32x16 zero = {};
+        i32x16 si;
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) si = mfma_i8(ki_op_x(kl, cc, 0), qireg[cc], cc == 0 ? zero : si);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float f = static_cast<float>(si[e]);
+          sa[e] = UKS ? f : f * ks_quad(ksl + 32 * (e >> 2))[e & 3];
+        }
+      }
+      float fa = factor(0), fb;
+      __syncthreads();  // every wave is done with K(0)
+      const int last = nfast - 1;
+      // The first token rows of tiles t and t + 1 are read from the LDS list an
+      // iteration ahead. K of the tile past the last is clamped to it: a redundant
+      // copy into a buffer that nothing reads afterwards.
+      int f0 = first_of(0), f1 = first_of(min(1, last));
+      issue_k(f1, 0);
+      half_step_i8<1, false, UKS>(st, sa, fa, sb, pb, pa, kl, ksl, vl, qireg);
+      fb = factor(1);
+      land();
+      issue_k(f1, 1);
+      issue_v(f0, 1);
+      half_step_i8<0, true, UKS>(st, sb, fb, sa, pa, pb, kl, ksl, vl, qireg);
+      fa = factor(0);
+      f0 = f1;
+      f1 = first_of(min(2, last));
+      land();
+      for (int t = 1; t < nfast; ++t) {
+        issue_k(f1, 0);
+        issue_v(f0, 0);
+        half_step_i8<1, true, UKS>(st, sa, fa, sb, pb, pa, kl, ksl, vl, qireg);
+        fb = factor(1);
+        asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
+        const int f2 = first_of(min(t + 2, last));
+        land();
+        issue_k(f1, 1);
+        issue_v(f0, 1);
+        half_step_i8<0, true, UKS>(st, sb, fb, sa, pa, pb, kl, ksl, vl, qireg);
+        fa = factor(0);
+        land();
+        f0 = f1;
+        f1 = f2;
+      }
+      mfma_fence(st.acc);  // P.V of the last half tile
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        st.acc[i & 3] = mfma_bf16(v_op_x(vl, 2 + (i >> 2), i & 3), pb[i >> 2], st.acc[i & 3]);
+      __syncthreads();
+    }
+  }
+
+  // ---- pooled tiles (bf16 Q: 32 VGPRs)
+  if (npool > 0) {
+    bf16x8 qreg[8];
+    const uint16_t* qp = q + b * sq_b + static_cast<int64_t>(qread) * sq_t + h * sq_h + half * 8;
+#pragma unroll
+    for (int cc = 0; cc < 8; ++cc)
+      qreg[cc] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + cc * 16));
+    issue_pooled(0);  // every earlier copy has landed and been read
+    for (int p = 0; p < npool; ++p) {
+      land();  // pooled tile p: the only copies in flight
+      if (PNBUF == 2 && p + 1 < npool) issue_pooled(p + 1);
+      const uint32_t kt = kb + (PNBUF == 2 ? p & 1 : 0) * 2 * kTileBytes;
+      f32x16 s[2];
+      qk_tile<kD>(k_lane(kt, col, half), qreg, s);
+      finish_tile<BLK>(st, s, v_lane(kt + kTileBytes, lane), pooled_desc(tl, p, NT), c, lane, NT, T);
+      __syncthreads();
+      if (PNBUF == 1 && p + 1 < npool) issue_pooled(p + 1);
+    }
+  }
+  wait_tile_copies();
+  store_rows(st, o + b * so_b + h * so_h, so_t, qrow, T, half);
+}
+
+// Block 64, int8 P.V: K and V tiles packed and double buffered (33 KB, four
+// workgroups per CU, two waves on every SIMD).
+template <bool UKS, bool RUN>
+__global__ void __launch_bounds__(128)
 __attribute__((amdgpu_waves_per_eu(2)))
 fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
                 const int8_t* __restrict__ qi, const float* __restrict__ qs,
                 const int8_t* __restrict__ ki, const float* __restrict__ ks,
                 const int8_t* __restrict__ vi, const float* __restrict__ vscale,
-                const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_t, int64_t sv_h,
                 int64_t TP, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
                 int64_t npad, const int32_t* __restrict__ counts, const uint32_t* __restrict__ mask, int T, int H, int NT, int W, float c,
                 uint16_t* __restrict__ o, int64_t so_b, int64_t so_t, int64_t so_h, int kst,
                 int64_t ksh) {
-  constexpr int NTHREADS = BLK * 2;
-  // LDS: exact-tile buffers K(i), V(i), i < 2. COMPACT (block 64): the int8
-  // tiles are packed (K + its ks: 8448 B; int8 V: 8192 B), so with int8 P.V two
-  // of each take 33 KB and four workgroups fit a CU, with bf16 P.V (16 KB V
-  // tiles) 49 KB and three; a bf16 pooled tile then spans K(0)-K(1) (and, with
-  // int8 P.V, V(0)-V(1)) and the pooled tiles are single buffered.
-  constexpr int NBUF = 2;
-  constexpr bool COMPACT = BLK == 64;
-  constexpr bool VSINGLE = COMPACT && !INT8_PV;  // one bf16 V tile buffer
-  constexpr int NVBUF = VSINGLE ? 1 : NBUF;
-  constexpr int KSTRIDE = COMPACT ? kKsOffset + 256 : static_cast<int>(kTileBytes);
-  constexpr int VSTRIDE = COMPACT && INT8_PV ? kKeys * kD : static_cast<int>(kTileBytes);
-  constexpr int VBASE = NBUF * KSTRIDE;
-  constexpr int PNBUF = COMPACT ? 1 : NBUF;  // buffers for pooled tiles
-  static_assert(!COMPACT || (2 * KSTRIDE >= static_cast<int>(kTileBytes) &&
-                             NVBUF * VSTRIDE >= static_cast<int>(kTileBytes)), "pooled tile must fit");
-  // copies per wave of one K tile (rows and ks): VSINGLE waits for the V tile
-  // issued before them with these still in flight
-  constexpr int kKCopies = I8Offsets<NTHREADS>::U + 1;
-  __shared__ __align__(256) char arena[VBASE + NVBUF * VSTRIDE];
+  constexpr int BLK = 64, NTHREADS = 128;
+  // LDS: exact-tile buffers K(i) with its ks (8448 B) and V(i) (8192 B), i < 2; a
+  // bf16 pooled tile spans K(0)-K(1) and V(0)-V(1), single buffered.
+  constexpr int KSTRIDE = kKsOffset + 256, VSTRIDE = kKeys * kD, VBASE = 2 * KSTRIDE;
+  static_assert(2 * KSTRIDE >= static_cast<int>(kTileBytes) && 2 * VSTRIDE >= static_cast<int>(kTileBytes),
+                "pooled tile must fit");
+  __shared__ __align__(256) char arena[VBASE + 2 * VSTRIDE];
   __shared__ TileList tl;
-  const auto Kp = [&](int i) { return reinterpret_cast<uint16_t*>(arena + i * KSTRIDE); };
-  const auto Vp = [&](int i) {
-    return reinterpret_cast<uint16_t*>(arena + VBASE + (VSINGLE ? 0 : i) * VSTRIDE);
-  };
-  const auto bi = [](int n) { return n & 1; };                      // buffer of exact tile n
-  const auto bp = [](int n) { return PNBUF == 2 ? (n & 1) : 0; };   // buffer of pooled tile n
+  const auto Kp = [&](int i) { return arena + i * KSTRIDE; };
+  const auto Vp = [&](int i) { return arena + VBASE + i * VSTRIDE; };
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 31, half = lane >> 5;
@@ -733,16 +769,13 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
   const int nfast = nexact - nrag;    // tiles [nexact, ntiles): pooled
 
   const int64_t bhD = (static_cast<int64_t>(b) * npad * H + h) * kD;
-  const KVSource src{nullptr, 0, v + b * sv_b + h * sv_h, sv_t, kc + bhD,
-                     static_cast<int64_t>(H) * kD, vc + bhD};
+  const KVSource src{nullptr, 0, nullptr, 0, kc + bhD, static_cast<int64_t>(H) * kD, vc + bhD};
   const I8Source is{ki + (static_cast<int64_t>(b) * TP * H + h) * kD,
                     ks + static_cast<int64_t>(b) * TP * H + h * ksh,
                     vi + (static_cast<int64_t>(b) * TP * H + h) * kD,
                     static_cast<int64_t>(H) * kD, kst};
   I8Offsets<NTHREADS> ioff;
   ioff.init(is.srow, kst);
-  CopyOffsets<NTHREADS> boff;
-  boff.init(0, sv_t);
 
   // Exact tile n of this kernel's order: n < nrag is the ragged one (list
   // tile nexact - 1), then list tiles 0 .. nfast-1.
@@ -751,16 +784,11 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
   };
   const uint32_t kb = lds_addr(arena), vb = kb + VBASE;  // LDS byte addresses
   const auto kbuf_at = [&](int buf) { return kb + buf * KSTRIDE; };
-  const auto vbuf_at = [&](int buf) { return vb + (VSINGLE ? 0 : buf) * VSTRIDE; };
+  const auto vbuf_at = [&](int buf) { return vb + buf * VSTRIDE; };
   const auto issue_exact_full = [&](int n, uint32_t kd, uint32_t vd, bool with_k, bool with_v) {
     const int first = exact_first<BLK>(tl, n - nrag);
     if (with_k) issue_i8<NTHREADS, true, true>(kd, is.ki, is, first, kKeys, ioff.k, ioff.ks, false);
-    if (with_v) {
-      if constexpr (INT8_PV)
-        issue_i8<NTHREADS, true, false>(vd, is.vi, is, first, kKeys, ioff.v, 0, true);
-      else
-        issue_full<NTHREADS>(vd, src.v + static_cast<int64_t>(first) * src.sv, src.sv, boff.v);
-    }
+    if (with_v) issue_i8<NTHREADS, true, false>(vd, is.vi, is, first, kKeys, ioff.v, 0, true);
   };
   const auto issue_tile = [&](int n, int buf) {
     const uint32_t kd = kbuf_at(buf), vd = vbuf_at(buf);
@@ -773,10 +801,7 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     } else {
       const TileDesc td = exact_tile(n);
       issue_i8<NTHREADS, false, true>(kd, is.ki, is, td.first, td.nvalid, 0, 0, false);
-      if constexpr (INT8_PV)
-        issue_i8<NTHREADS, false, false>(vd, is.vi, is, td.first, td.nvalid, 0, 0, true);
-      else
-        issue_generic<NTHREADS>(vd, 1, td, src);
+      issue_i8<NTHREADS, false, false>(vd, is.vi, is, td.first, td.nvalid, 0, 0, true);
     }
   };
   issue_tile(0, 0);
@@ -805,18 +830,12 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
     if (nrag) {
       wait_tile_copies();
       __syncthreads();
-      // a pooled tile 1 does not fit buffer 1 when COMPACT: the pooled phase
-      // issues it; VSINGLE: tile 1's V follows the ragged tile's P.V
-      if (1 < ntiles && (!COMPACT || 1 < nexact)) {
-        if constexpr (VSINGLE)
-          issue_exact_full(1, kbuf_at(1), 0u, true, false);
-        else
-          issue_tile(1, 1);
-      }
+      // (a pooled tile 1 does not fit buffer 1: the pooled phase issues it)
+      if (1 < nexact) issue_tile(1, 1);
       const TileDesc td = exact_tile(0);
       i32x16 si[2];
       f32x16 s[2];
-      const char* kt = reinterpret_cast<const char*>(Kp(0));
+      const char* kt = Kp(0);
       qk_i8_tile(kt, qireg, col, half, si);
       scale_scores<UKS>(kt, si, half, s);
 #pragma unroll
@@ -826,11 +845,8 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
         for (int r = 0; r < 16; ++r)
           s[m][r] = ((bits >> (8 * (r >> 2) + (r & 3))) & 1u) ? s[m][r] : -INFINITY;
       }
-      exact_softmax_pv<INT8_PV, RUN>(st, s, Vp(0), tile_qsl<UKS>(kt, kKsOffset, qsl), lane);
+      exact_softmax_pv<true, RUN>(st, s, Vp(0), tile_qsl<UKS>(kt, kKsOffset, qsl), lane);
       __syncthreads();
-      if constexpr (VSINGLE) {
-        if (1 < nexact) issue_exact_full(1, 0u, vbuf_at(0), false, true);
-      }
     }
     // full exact tiles, pipelined (tile F = nrag was issued into buffers bi(F));
     // fa, fb: the score factors of sa, sb
@@ -839,9 +855,8 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
       const int E = nexact;  // one past the last full exact tile
       f32x16 sa[2], sb[2];
       float fa, fb;
-      const auto qk_scaled = [&](const uint16_t* kb, f32x16 (&s)[2]) {
+      const auto qk_scaled = [&](const char* kt, f32x16 (&s)[2]) {
         i32x16 si[2];
-        const char* kt = reinterpret_cast<const char*>(kb);
         qk_i8_tile(kt, qireg, col, half, si);
         scale_scores<UKS>(kt, si, half, s);
         return tile_qsl<UKS>(kt, kKsOffset, qsl);
@@ -853,115 +868,42 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
       wait_tile_copies();
       __syncthreads();  // K(F & 1) is refilled (K of tile F+2) by the first step
       int n = F;
-      if constexpr (!INT8_PV && !VSINGLE) {
-        // Three-stage pipeline (step3_i8). On entry to step n (F < n < E-1):
-        // S(n) and P(n-1) in registers, K(n+1) and V(n-1) in LDS; the step
-        // copies K(n+2) over K(n) and V(n) over V(n-2) (V(F) came with tile F).
-        const uint32_t vl0 = v_lane(vbuf_at(0), lane);
-        if (F + 1 < E) {
-          bf16x8 pa[4], pb[4];
-          issue_exact_full(min(F + 2, E - 1), kbuf_at(F & 1), 0u, true, false);
-          {
-            const char* kn = reinterpret_cast<const char*>(Kp((F + 1) & 1));
-            step3_i8<true, false, UKS>(st, sa, fa, sb, pb, pa, kn, 0u, qireg, lane);
-            fb = tile_qsl<UKS>(kn, kKsOffset, qsl);
-          }
-          wait_tile_copies();
-          __syncthreads();
-          n = F + 1;  // S(n) in sb (factor fb), P(n-1) in pa
-          const auto gstep = [&](const f32x16 (&sc)[2], float fc, f32x16 (&sn)[2], float& fnext,
-                                 const bf16x8 (&pp)[4], bf16x8 (&pn)[4]) {
-            issue_exact_full(min(n + 2, E - 1), kbuf_at(n & 1), 0u, true, false);
-            issue_exact_full(n, 0u, vbuf_at(n & 1), false, true);
-            const char* kn = reinterpret_cast<const char*>(Kp((n + 1) & 1));
-            step3_i8<true, true, UKS>(st, sc, fc, sn, pp, pn, kn, vl0 + ((n - 1) & 1) * VSTRIDE,
-                                      qireg, lane);
-            fnext = tile_qsl<UKS>(kn, kKsOffset, qsl);
-            wait_tile_copies();
-            __syncthreads();
-            ++n;
-          };
-          const auto last = [&](const f32x16 (&sc)[2], float fc, f32x16 (&dummy)[2],
-                                const bf16x8 (&pp)[4], bf16x8 (&pn)[4]) {
-            issue_exact_full(n, 0u, vbuf_at(n & 1), false, true);  // V(E-1)
-            step3_i8<false, true, UKS>(st, sc, fc, dummy, pp, pn, nullptr,
-                                       vl0 + ((n - 1) & 1) * VSTRIDE, qireg, lane);
-            wait_tile_copies();
-            __syncthreads();
-            pv_tile(reinterpret_cast<const uint16_t*>(Vp(n & 1)), pn, lane, st.acc);
-          };
-          while (n + 2 < E) {
-            gstep(sb, fb, sa, fa, pa, pb);
-            gstep(sa, fa, sb, fb, pb, pa);
-          }
-          if (n + 1 < E) {
-            gstep(sb, fb, sa, fa, pa, pb);
-            last(sa, fa, sb, pb, pa);
-          } else {
-            last(sb, fb, sa, pa, pb);
-          }
-        } else {
-          exact_softmax_pv<INT8_PV, RUN>(st, sa, Vp(bi(n)), fa, lane);
-        }
-        __syncthreads();
-      } else {
       // Step n needs n + 1 < E. K(n+2) of the last step is clamped to the
       // last full tile: a redundant copy into a buffer nothing reads afterwards.
-      // VSINGLE: V(n) was copied at the end of step n-1, before this step's
-      // K(n+2); it is waited for before P(n).V(n), and V(n+1) is copied once
-      // every wave is past P(n).V(n).
       const auto step = [&](f32x16 (&sc)[2], float qc, f32x16 (&sn)[2], float& qn) {
         issue_exact_full(min(n + 2, E - 1), kbuf_at(n & 1), 0u, true, false);
-        if constexpr (!VSINGLE) issue_exact_full(n + 1, 0u, vbuf_at((n + 1) & 1), false, true);
-        const char* kn = reinterpret_cast<const char*>(Kp((n + 1) & 1));
-        fast_step<INT8_PV, UKS, RUN>(st, sc, sn, kn, Vp(n & 1), qireg, qc, lane, [&] {
-          if constexpr (VSINGLE) {
-            wait_vmcnt<kKCopies>();
-            __syncthreads();
-          }
-        });
+        issue_exact_full(n + 1, 0u, vbuf_at((n + 1) & 1), false, true);
+        const char* kn = Kp((n + 1) & 1);
+        fast_step<UKS, RUN>(st, sc, sn, kn, Vp(n & 1), qireg, qc, lane);
         qn = tile_qsl<UKS>(kn, kKsOffset, qsl);
         wait_tile_copies();
         __syncthreads();
-        if constexpr (VSINGLE) issue_exact_full(n + 1, 0u, vbuf_at(0), false, true);
         ++n;
       };
       while (n + 2 < E) {
         step(sa, fa, sb, fb);
         step(sb, fb, sa, fa);
       }
-      if constexpr (VSINGLE) {
-        const bool odd = n + 1 < E;  // one more step, the last tile's scores in sb
-        if (odd) step(sa, fa, sb, fb);
-        wait_tile_copies();  // V of the last tile
-        __syncthreads();
-        if (odd)
-          exact_softmax_pv<INT8_PV, RUN>(st, sb, Vp(bi(n)), fb, lane);
-        else
-          exact_softmax_pv<INT8_PV, RUN>(st, sa, Vp(bi(n)), fa, lane);
-      } else if (n + 1 < E) {
+      if (n + 1 < E) {
         step(sa, fa, sb, fb);
-        exact_softmax_pv<INT8_PV, RUN>(st, sb, Vp(bi(n)), fb, lane);
+        exact_softmax_pv<true, RUN>(st, sb, Vp(n & 1), fb, lane);
       } else {
-        exact_softmax_pv<INT8_PV, RUN>(st, sa, Vp(bi(n)), fa, lane);
+        exact_softmax_pv<true, RUN>(st, sa, Vp(n & 1), fa, lane);
       }
       __syncthreads();
-      }
     }
-    if constexpr (INT8_PV) {
-      // The per-channel V scale, common to every exact tile. The empty asm
-      // keeps its 64 loads here: hoisted above the exact tiles they would
-      // hold 64 VGPRs through the whole pipeline.
-      const float* vsc = vscale + static_cast<int64_t>(bh) * kD;
-      asm volatile("" : "+s"(vsc));
-      if constexpr (RUN) {
-        run_finish(st, vsc, half);
-      } else {
+    // The per-channel V scale, common to every exact tile. The empty asm
+    // keeps its 64 loads here: hoisted above the exact tiles they would
+    // hold 64 VGPRs through the whole pipeline.
+    const float* vsc = vscale + static_cast<int64_t>(bh) * kD;
+    asm volatile("" : "+s"(vsc));
+    if constexpr (RUN) {
+      run_finish(st, vsc, half);
+    } else {
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+      for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) st.acc[dt][r] *= vsc[32 * dt + 8 * (r >> 2) + 4 * half + (r & 3)];
-      }
+        for (int r = 0; r < 16; ++r) st.acc[dt][r] *= vsc[32 * dt + 8 * (r >> 2) + 4 * half + (r & 3)];
     }
   }
 
@@ -975,20 +917,16 @@ fwd_int8_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
       if (qvalid) r = *reinterpret_cast<const uint4*>(qp + cc * 16);
       qreg[cc] = __builtin_bit_cast(bf16x8, r);
     }
-    if (nexact > 0) issue_tile(nexact, bp(nexact));  // every earlier copy has landed
+    if (nexact > 0) issue_tile(nexact, 0);  // every earlier copy has landed
     for (int n = nexact; n < ntiles; ++n) {
       wait_tile_copies();  // tile n: the only copies in flight
       __syncthreads();
-      if constexpr (PNBUF == 2) {
-        if (n + 1 < ntiles) issue_tile(n + 1, (n + 1) & 1);
-      }
       f32x16 s[2];
-      qk_tile(Kp(bp(n)), qreg, col, half, s);
-      finish_tile<BLK>(st, s, Vp(bp(n)), pooled_desc(tl, n - nexact, NT), c, lane, NT, T);
+      qk_tile(reinterpret_cast<const uint16_t*>(Kp(0)), qreg, col, half, s);
+      finish_tile<BLK>(st, s, reinterpret_cast<const uint16_t*>(Vp(0)), pooled_desc(tl, n - nexact, NT), c,
+                       lane, NT, T);
       __syncthreads();
-      if constexpr (PNBUF == 1) {
-        if (n + 1 < ntiles) issue_tile(n + 1, 0);
-      }
+      if (n + 1 < ntiles) issue_tile(n + 1, 0);
     }
   }
   wait_tile_copies();
@@ -1343,31 +1281,6 @@ fwd_int8_b128_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t,
   store_rows(st, o + b * so_b + h * so_h, so_t, qrow, T, half);
 }
 
-template <int BLK, bool PV, bool UKS, bool RUN>
-void launch_i8(uint32_t grid, hipStream_t s, const uint16_t* q, int64_t sq_b, int64_t sq_t,
-               int64_t sq_h, const int8_t* qi, const float* qs, const int8_t* ki, const float* ks,
-               const int8_t* vi, const float* vscale, const uint16_t* v, int64_t sv_b,
-               int64_t sv_t, int64_t sv_h, int64_t TP, const uint16_t* kc, const uint16_t* vc,
-               int64_t npad, const int32_t* counts, const uint32_t* mask,
-               int T, int H, int NT, int W, float c, uint16_t* o, int64_t so_b, int64_t so_t,
-               int64_t so_h, int kst, int64_t ksh) {
-  hipLaunchKernelGGL((fwd_int8_kernel<BLK, PV, UKS, RUN>), dim3(grid), dim3(BLK * 2), blist_lds_bytes(NT), s, q, sq_b, sq_t,
-                     sq_h, qi, qs, ki, ks, vi, vscale, v, sv_b, sv_t, sv_h, TP, kc, vc, npad,
-                     counts, mask, T, H, NT, W, c, o, so_b, so_t, so_h, kst, ksh);
-}
-
-template <int BLK, bool PV, bool RUN = false>
-void launch_i8_ks(bool uks, uint32_t grid, hipStream_t s, const uint16_t* q, int64_t sq_b,
-                  int64_t sq_t, int64_t sq_h, const int8_t* qi, const float* qs, const int8_t* ki,
-                  const float* ks, const int8_t* vi, const float* vscale, const uint16_t* v,
-                  int64_t sv_b, int64_t sv_t, int64_t sv_h, int64_t TP, const uint16_t* kc,
-                  const uint16_t* vc, int64_t npad, const int32_t* counts, const uint32_t* mask, int T, int H, int NT, int W, float c, uint16_t* o,
-                  int64_t so_b, int64_t so_t, int64_t so_h, int kst, int64_t ksh) {
-  (uks ? launch_i8<BLK, PV, true, RUN> : launch_i8<BLK, PV, false, RUN>)(
-      grid, s, q, sq_b, sq_t, sq_h, qi, qs, ki, ks, vi, vscale, v, sv_b, sv_t, sv_h, TP, kc, vc,
-      npad, counts, mask, T, H, NT, W, c, o, so_b, so_t, so_h, kst, ksh);
-}
-
 }  // namespace int8fwd
 
 int fwd_int8(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const int8_t* qi,
@@ -1407,30 +1320,26 @@ int fwd_int8(const uint16_t* q, int64_t sq_b, int64_t sq_t, int64_t sq_h, const 
   // ks: token-major [B, TP, H] (the reference's) or head-major [B, H, TP]
   const int kst = ks_head_major ? 1 : static_cast<int>(H);
   const int64_t ksh = ks_head_major ? TP : 1;
-#define SOLATTN_I8_ARGS                                                                          \
-  grid, s, q, sq_b, sq_t, sq_h, qi, qs, ki, ks, vi, vscale, v, sv_b, sv_t, sv_h, TP, kc, vc, npad, \
-      counts, mask, static_cast<int>(T), static_cast<int>(H), static_cast<int>(NT), W, c, o, \
-      so_b, so_t, so_h, kst, ksh
-  const bool run = int8_pv == SOLATTN_PV_INT8_RUNNING;
-  if (block == 128) {
-    if (int8_pv) {
-      const auto kern = uniform_ks ? (run ? int8fwd::fwd_int8_b128_kernel<true, true>
-                                          : int8fwd::fwd_int8_b128_kernel<true, false>)
-                                   : (run ? int8fwd::fwd_int8_b128_kernel<false, true>
-                                          : int8fwd::fwd_int8_b128_kernel<false, false>);
-      hipLaunchKernelGGL(kern, dim3(grid), dim3(256), blist_lds_bytes(NT), s, q, sq_b, sq_t, sq_h,
-                         qi, qs, ki, ks, vi, vscale, TP, kc, vc, npad, counts, mask,
-                         static_cast<int>(T), static_cast<int>(H), static_cast<int>(NT), W, c, o,
-                         so_b, so_t, so_h, kst, ksh);
-    } else {
-      int8fwd::launch_i8_ks<128, false>(uniform_ks, SOLATTN_I8_ARGS);
-    }
+  const int t32 = static_cast<int>(T), h32 = static_cast<int>(H), n32 = static_cast<int>(NT);
+  const dim3 threads(static_cast<uint32_t>(block) * 2);
+  if (int8_pv) {
+    using namespace int8fwd;
+    const bool run = int8_pv == SOLATTN_PV_INT8_RUNNING;
+    const auto kern = block == 128 ? (uniform_ks ? (run ? fwd_int8_b128_kernel<true, true> : fwd_int8_b128_kernel<true, false>)
+                                                 : (run ? fwd_int8_b128_kernel<false, true> : fwd_int8_b128_kernel<false, false>))
+                                   : (uniform_ks ? (run ? fwd_int8_kernel<true, true> : fwd_int8_kernel<true, false>)
+                                                 : (run ? fwd_int8_kernel<false, true> : fwd_int8_kernel<false, false>));
+    hipLaunchKernelGGL(kern, dim3(grid), threads, blist_lds_bytes(NT), s, q, sq_b, sq_t, sq_h, qi, qs,
+                       ki, ks, vi, vscale, TP, kc, vc, npad, counts, mask, t32, h32, n32, W, c, o, so_b,
+                       so_t, so_h, kst, ksh);
   } else {
-    if (run) int8fwd::launch_i8_ks<64, true, true>(uniform_ks, SOLATTN_I8_ARGS);
-    else if (int8_pv) int8fwd::launch_i8_ks<64, true>(uniform_ks, SOLATTN_I8_ARGS);
-    else int8fwd::launch_i8_ks<64, false>(uniform_ks, SOLATTN_I8_ARGS);
+    using namespace int8fwd;
+    const auto kern = block == 128 ? (uniform_ks ? fwd_int8_bf16pv_kernel<128, true> : fwd_int8_bf16pv_kernel<128, false>)
+                                   : (uniform_ks ? fwd_int8_bf16pv_kernel<64, true> : fwd_int8_bf16pv_kernel<64, false>);
+    hipLaunchKernelGGL(kern, dim3(grid), threads, blist_lds_bytes(NT), s, q, sq_b, sq_t, sq_h, qi, qs,
+                       ki, ks, v, sv_b, sv_t, sv_h, TP, kc, vc, npad, counts, mask, t32, h32, n32, W, c, o,
+                       so_b, so_t, so_h, kst, ksh);
   }
-#undef SOLATTN_I8_ARGS
   return check_launch("fwd_int8");
 }
 

@@ -595,6 +595,42 @@ def test_fwd_bf16_half_chunk_exact(pkg, dev, block, T):
     _check_hand_set_masks(pkg, dev, block, T, exact_rows)
 
 
+@pytest.mark.parametrize("block,T", [(64, 64 * 67 + 17), (64, 64 * 66), (128, 128 * 66 + 90), (128, 128 * 65 + 64),
+                                     (128, 128 * 65 + 17)])
+def test_fwd_int8_bf16pv_hand_set_masks(pkg, dev, block, T):
+    """The INT8 forward with bf16 P.V where its pipeline is empty or a tile or two long:
+    no exact block, the last alone, the first alone, both, every second block. Against
+    float64 over the same codes and scales: P and the outputs are rounded to bf16 (2^-9
+    each) under values of order 1, far inside BF16_MAXABS."""
+    i8, fp = _mods(pkg)[2:4]
+    q, k, v = (randn_bf16((1, T, 1, 128), s) for s in (93, 94, 95))
+    r, qi, qs, ki, ks, _ = fp.fused_preprocess_routing(q.to(dev), k.to(dev), v.to(dev), tau=0.9, scale=128 ** -0.5,
+                                                       block=block, int8_pv=False)
+    NT = r.counts.shape[-1]
+    exact = torch.zeros(5, NT, dtype=torch.bool)
+    exact[1, NT - 1] = exact[2, 0] = exact[3, 0] = exact[3, NT - 1] = True
+    exact[4, ::2] = True
+    rows = exact[torch.arange(NT) % 5]  # [query block, key block]
+    j = torch.arange(NT)
+    words = torch.zeros(NT, r.mask.shape[-1], dtype=torch.int64)
+    words.index_add_(1, j >> 5, rows.long() << (j & 31))
+    mask = torch.where(words >= 2 ** 31, words - 2 ** 32, words).to(torch.int32).to(dev)
+    r = r._replace(mask=mask.reshape(r.mask.shape).contiguous(),
+                   counts=rows.sum(-1).to(torch.int32).to(dev).reshape(r.counts.shape))
+    print(f"[int8 bf16pv hand masks] block={block} T={T}", flush=True)
+    out = i8.forward_int8(q.to(dev), v.to(dev), r, qi, qs, ki, ks, None, int8_pv=False).float().cpu()[0, :, 0]
+    lens = torch.full((NT,), float(block), dtype=torch.float64)
+    lens[-1] = T - (NT - 1) * block
+    qc, kcode = (c[0, :T, 0].double().cpu() * s[0, :T, 0, None].double().cpu() for c, s in ((qi, qs), (ki, ks)))
+    kc, vc = (t[0, :NT, 0].double().cpu() for t in (r.kc, r.vc))
+    on = rows[torch.arange(T) // block]
+    s = (qc @ kcode.t() * 128 ** -0.5).masked_fill(~on[:, torch.arange(T) // block], -torch.inf).exp()
+    p = (q[0, :, 0].double() @ kc.t() * 128 ** -0.5).masked_fill(on, -torch.inf).exp()
+    ref = (s @ v[0, :, 0].double() + p @ vc) / (s.sum(1) + p @ lens)[:, None]
+    assert float((out - ref).abs().max()) < BF16_MAXABS
+    assert cosine(out.numpy(), ref.numpy()) >= BF16_COS
+
+
 @pytest.mark.parametrize("D", [8, 40, 64])
 @pytest.mark.parametrize("shape,block", [((2, 333, 3), 64), ((1, 777, 5), 128), ((1, 64, 1), 64),
                                          ((1, 64 * 65 + 7, 3), 64), ((1, 128 * 20 + 64, 2), 128)])

@@ -8,12 +8,11 @@
 //                 (/root/reference/_tri_fwd.py:288-308);
 //   exact tiles   64 tokens of an exact block (/root/reference/_tri_fwd.py:310-340).
 // All tiles feed one online softmax per query row, which is exact under any
-// tile order (up to fp32 rounding). The pooled and the full exact tiles run
-// through a software pipeline of half tiles (32 keys): step n computes S(n+1) =
-// K(n+1) Q^T, O += P(n-1) V(n-1) and the softmax of S(n) in one instruction
-// stream, hand-ordered from inline-asm MFMAs and softmax exp pairs
-// (fwd_common.hpp), which the compiler's own schedule did not give. The tile of
-// a short last block goes through a plain path first.
+// tile order (up to fp32 rounding), through a software pipeline of half tiles
+// (32 keys): step n computes S(n+1) = K(n+1) Q^T, O += P(n-1) V(n-1) and the
+// softmax of S(n) in one instruction stream, hand-ordered from inline-asm MFMAs
+// and softmax exp pairs (fwd_common.hpp), which the compiler's own schedule did
+// not give.
 //
 // MFMA dataflow (v_mfma_f32_32x32x16_bf16): S^T = K . Q^T puts one query row
 // per lane column, so row max / sum need one cross-lane step (lanes 32 apart,
@@ -32,38 +31,36 @@ namespace bf16fwd {
 // hand-ordered stream: slot i issues score MFMA i, the exps of P(n) word i, then
 // P.V MFMA i; the K and V operands of slot i + 2 are read at the top of slot i
 // (the empty asm with a memory clobber keeps the reads there). O is rescaled to
-// the new running max after the P(n-1) V(n-1) products. PV = false: the first
-// half tile, which has no value product to add. POOLED: the keys of n are
-// pooled keys of whole blocks (masked scores -inf), each weighing BLK in the row
-// sum, which adds the fp32 p. kl, vl: this lane's operand addresses in K(n+1)
-// and V(n-1).
+// the new running max after the P(n-1) V(n-1) products. HH: the half of its tile
+// that n is. psum: this lane's sum of the tile's P, started by half 0 and carried
+// on by half 1 (POOLED, the keys of n are pooled keys: of the fp32 p). kl, vl:
+// this lane's operand addresses in K(n+1) and V(n-1). Returns the factor that the
+// row sum so far takes with a new running max.
 // Lazy tile max: the exps use the running max as it stands, and the tile's max
 // is taken only when a lane's row sum exceeds 255. No sum above 255 means every
 // p <= 255, i.e. every score is below the running max + log2(255.5) <
 // kMaxSlack, so the tile would not have moved the max: the running max evolves
-// as with the max taken every step. The first tile of a workgroup (running max
-// -inf, p = inf or NaN) always takes that path.
+// as with the max taken every step.
 // Raised wave priority for the step's stream: the issue arbiter then prefers a
 // wave inside its MFMAs over one at its copies or barrier (without it, 6%
 // slower at block 64 and 32760 tokens).
 // 64 channels halve the MFMAs: one of each product per two slots.
-template <int BLK, int D, bool POOLED, bool PV>
-__device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x16& sc, f32x16& sn,
+template <int D, bool POOLED, int HH>
+__device__ __forceinline__ float half_step(SoftmaxStateOf<D / 32>& st, const f32x16& sc, f32x16& sn,
                                           const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
-                                          uint32_t vl, const bf16x8 (&q)[D / 16], float c) {
+                                          uint32_t vl, const bf16x8 (&q)[D / 16], float c, float& psum) {
   static_assert(kMaxSlack >= 8.f, "the lazy test relies on 255 < 2^kMaxSlack");
   constexpr int ND = D / 32, NM = D / 16;  // MFMAs of each product
   constexpr int SLOTS = 8 / NM;            // slots per MFMA of each
   bf16x8 ka[3], va[3];
   uint32_t pw[2][4];
-  float psum = 0.f;
+  const float before = HH == 0 ? 0.f : psum;
+  if constexpr (HH == 0) psum = 0.f;
   const float neg = -st.m;
   ka[0] = k_op_x<D>(kl, 0, 0);
   ka[1] = k_op_x<D>(kl, 0, 1);
-  if constexpr (PV) {
-    va[0] = v_op_x<D>(vl, 0, 0);
-    va[1] = v_op_x<D>(vl, 0, 1);
-  }
+  va[0] = v_op_x<D>(vl, 0, 0);
+  va[1] = v_op_x<D>(vl, 0, 1);
   asm volatile("" ::: "memory");
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -71,7 +68,7 @@ __device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x
     if (i % SLOTS == 0) {
       if (j + 2 < NM) {
         ka[(j + 2) % 3] = k_op_x<D>(kl, 0, j + 2);
-        if constexpr (PV) va[(j + 2) % 3] = v_op_x<D>(vl, (j + 2) / ND, (j + 2) % ND);
+        va[(j + 2) % 3] = v_op_x<D>(vl, (j + 2) / ND, (j + 2) % ND);
         asm volatile("" ::: "memory");
       }
       if (j == 0)
@@ -81,20 +78,17 @@ __device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x
     }
     pw[i >> 2][i & 3] = POOLED ? exp_pair_f32sum(sc[2 * i], sc[2 * i + 1], c, neg, psum)
                                : exp_pair(sc[2 * i], sc[2 * i + 1], c, neg, psum);
-    if constexpr (PV) {
-      if (i % SLOTS == SLOTS - 1) {
-        if (j == 0)
-          mfma_v_first(st.acc[0], va[0], pp[0]);
-        else if (j == NM - 1)
-          mfma_v_tie(st.acc[ND - 1], va[j % 3], pp[1], sn);
-        else
-          mfma_v(st.acc[j % ND], va[j % 3], pp[j / ND]);
-      }
+    if (i % SLOTS == SLOTS - 1) {
+      if (j == 0)
+        mfma_v_first(st.acc[0], va[0], pp[0]);
+      else if (j == NM - 1)
+        mfma_v_tie(st.acc[ND - 1], va[j % 3], pp[1], sn);
+      else
+        mfma_v(st.acc[j % ND], va[j % 3], pp[j / ND]);
     }
     if (i == 0) __builtin_amdgcn_s_setprio(1);
   }
   __builtin_amdgcn_s_setprio(0);
-  if constexpr (!PV) mfma_fence(sn);
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks)
     pn[ks] = __builtin_bit_cast(bf16x8, make_uint4(pw[ks][0], pw[ks][1], pw[ks][2], pw[ks][3]));
@@ -104,17 +98,13 @@ __device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[r]);
     const float m_new = new_max(st.m, xhalf_max(mx) * c, alpha);
-    // A first half tile without a single unmasked pooled key (its 32 blocks all
-    // exact) leaves the max at -inf: its P are 0, not exp2(-inf + inf).
-    const bool none = POOLED && m_new == -INFINITY;
-    if (__any(m_new != st.m || none)) {  // lanes whose max stays recompute the same P
+    if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
       st.m = m_new;
-      psum = 0.f;
+      psum = before * alpha;
       if constexpr (POOLED) {
-        const float neg_new = none ? 0.f : -m_new;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r], c, neg_new));
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[r], c, -m_new));
           pn[r >> 3][r & 7] = static_cast<__bf16>(p);
           psum += p;
         }
@@ -122,19 +112,27 @@ __device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x
         psum = exp8<0>(sc, c, -m_new, pn[0], psum);
         psum = exp8<8>(sc, c, -m_new, pn[1], psum);
       }
-      if constexpr (PV) mfma_fence(st.acc);  // the rescale reads O
+      mfma_fence(st.acc);  // the rescale reads O
       rescale(st, alpha);
     }
   }
-  st.l = fmaf(st.l, alpha, POOLED ? psum * static_cast<float>(BLK) : psum);
+  return alpha;
+}
+
+// The score of key `key` (of the 32 of s) in the lanes that hold it, -inf elsewhere.
+__device__ __forceinline__ float score_of_key(const f32x16& s, int key, int half) {
+  float x = -INFINITY;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) x = 8 * (r >> 2) + 4 * half + (r & 3) == key ? s[r] : x;
+  return x;
 }
 
 // The forward. Workgroups of 2 waves at block 64 (four per CU), 4 at block 128
 // (two per CU): two waves per SIMD. K and V hold two half tiles of 32 keys each
-// (32 KiB). Tile order: the tile of a short last block, if any, through the
-// plain path (as a ragged exact tile, or inside its pooled tile, where it weighs
-// its own length); then the pooled and the full exact tiles through the
-// pipeline, two half steps a tile.
+// (32 KiB). Every tile takes two half steps of the pipeline, in the order pooled,
+// ragged exact (the short last block's, its rows past T masked), full exact at
+// block 64, and full exact, ragged exact, pooled at block 128. The pooled key of
+// a short last block weighs its own length.
 //
 // Bound: at 32760 tokens the MFMAs at the power-limited clock and the tile
 // copies (block 64: without them, results wrong by construction, the two-stage
@@ -148,6 +146,11 @@ __device__ __forceinline__ void half_step(SoftmaxStateOf<D / 32>& st, const f32x
 // three-stage step over whole tiles, double buffered in 64 KiB, with plain
 // pooled tiles: 32760 tokens 2370 -> 2325 us, 75600 tokens 21.2 -> 21.0 ms; four
 // half buffers with copies two steps ahead were slower (2400 us).
+// The order of the tiles, the max of the whole first tile and the row sums of whole
+// tiles are those of that whole-tile step, and so are the results, but for rows whose
+// max a later tile moves. Against a max of 32 keys and the short last block's tile
+// first, on a plain path: 32760 tokens 2744 -> 2742 us at block 64 and 2379 -> 2384
+// at block 128, 4096 tokens 81.9 -> 82.0, 1000 tokens 29.35 -> 29.8.
 template <int BLK, int D>
 __global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2)))
 fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t sq_h,
@@ -171,12 +174,15 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
 
   const int ntiles = build_tile_list<BLK>(tl, mask, row, NT, W, T);
   if (ntiles == 0) return;  // cannot happen for routed masks: the diagonal is exact
-  // The plain tile: a ragged exact one, or the pooled tile of a short last block.
-  const bool rag = ragged_tiles(tl, NT, T) != 0;
-  const bool tail = T % BLK != 0 && tl.last != NT - 1;
-  const int nplain = rag || tail ? 1 : 0;
-  const int npool = tl.npool - (tail ? 1 : 0);  // pipelined pooled tiles, first in order
-  const int npipe = ntiles - nplain;
+  // (the lists' sizes made scalar: the loops and branches over tiles are uniform)
+  const int npool = __builtin_amdgcn_readfirstlane(tl.npool);
+  const int nrag = __builtin_amdgcn_readfirstlane(ragged_tiles(tl, NT, T));
+  const int nfull = __builtin_amdgcn_readfirstlane(tl.nexact) - nrag;
+  // the order: tile t is pooled from pool0 on, ragged at rag0 (if there is one),
+  // full exact from full0 on
+  constexpr bool kPoolFirst = BLK == 64;
+  const int pool0 = kPoolFirst ? 0 : nfull + nrag, rag0 = kPoolFirst ? npool : nfull;
+  const int full0 = kPoolFirst ? npool + nrag : 0, last = npool + nrag + nfull - 1;
 
   const KVSource src{k + b * sk_b + h * sk_h, sk_t, v + b * sv_b + h * sv_h, sv_t,
                      kc + (static_cast<int64_t>(b) * npad * H + h) * D,
@@ -185,38 +191,41 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
   off.init(sk_t, sv_t);
   const uint32_t kb = lds_addr(kbuf), vb = lds_addr(vbuf);  // LDS byte addresses
   const uint32_t kl = k_lane<D>(kb, col, half), vl = v_lane<D>(vb, lane);  // this lane's operands
-  // Half hh of pipelined tile t (pooled tiles, then the full exact tiles) into
-  // K or V half buffer hh.
-  const auto first_of = [&](int t) { return exact_first<BLK>(tl, max(t - npool, 0)); };
-  const auto issue_k_at = [&](int first, int hh) {
+  // Half hh of a tile into K or V half buffer hh. (The lambdas are always_inline: one
+  // that is called in several places would take its captures through memory.)
+  const auto full_first = [&](int e) __attribute__((always_inline)) { return exact_first<BLK>(tl, e); };
+  const auto issue_k_at = [&](int first, int hh) __attribute__((always_inline)) {
     issue_half<NTHREADS, D>(kb + hh * kHalfBytes, src.k + static_cast<int64_t>(first + 32 * hh) * src.sk,
                          src.sk, off.k);
   };
-  const auto issue_v_at = [&](int first, int hh) {
+  const auto issue_v_at = [&](int first, int hh) __attribute__((always_inline)) {
     issue_half<NTHREADS, D>(vb + hh * kHalfBytes, src.v + static_cast<int64_t>(first + 32 * hh) * src.sv,
                          src.sv, off.v);
   };
-  const auto issue_any = [&](int t, int kv, int hh) {
-    if (t >= npool) {
-      if (kv == 0) issue_k_at(first_of(t), hh); else issue_v_at(first_of(t), hh);
-    } else {
-      issue_pooled_half<NTHREADS, D>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, t, NT), hh, src);
-    }
+  const auto issue_pooled = [&](int p, int kv, int hh) __attribute__((always_inline)) {
+    issue_clamped_half<NTHREADS, D>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv, pooled_desc(tl, p, NT), hh, src);
   };
-  const auto issue_start = [&] {  // what the first half steps need
-    issue_any(0, 0, 0);
-    issue_any(0, 0, 1);
-    issue_any(0, 1, 0);
+  const auto issue_ragged = [&](int kv, int hh) __attribute__((always_inline)) {
+    issue_clamped_half<NTHREADS, D>((kv == 0 ? kb : vb) + hh * kHalfBytes, kv,
+                                    exact_desc<BLK>(tl, tl.nexact - 1, T, NT), hh, src);
   };
-  const auto plain_desc = [&] {
-    return rag ? exact_desc<BLK>(tl, tl.nexact - 1, T, NT) : pooled_desc(tl, tl.npool - 1, NT);
+  const auto issue_any_k = [&](int t, int hh) __attribute__((always_inline)) {
+    if (nrag && t == rag0)
+      issue_ragged(0, hh);
+    else if (t >= pool0 && t < pool0 + npool)
+      issue_pooled(t - pool0, 0, hh);
+    else
+      issue_k_at(full_first(t - full0), hh);
   };
-  if (nplain) {
-    issue_generic<NTHREADS, D>(kb, 0, plain_desc(), src);
-    issue_generic<NTHREADS, D>(vb, 1, plain_desc(), src);
-  } else {
-    issue_start();
-  }
+  const bool first_pooled = npool && pool0 == 0, first_ragged = nrag && rag0 == 0;
+  issue_any_k(0, 0);
+  issue_any_k(0, 1);
+  if (first_pooled)
+    issue_pooled(0, 1, 0);
+  else if (first_ragged)
+    issue_ragged(1, 0);
+  else
+    issue_v_at(full_first(0), 0);
 
   // This wave's 32 query rows as the B operand of S^T = K Q^T (rows past T
   // repeat row T - 1 and are not stored).
@@ -232,101 +241,184 @@ fwd_bf16_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int6
   SoftmaxStateOf<D / 32> st;
   st.init();
 
-  // ---- the short last block's tile
-  if (nplain) {
+  // The tiles by half tiles n = 2t, 2t + 1. On entry to step n: S(n) and P(n-1)
+  // in registers, K(n+1) and V(n-1) in LDS; the step copies K(n+2) over K(n) and
+  // V(n) over V(n-2), so a copy has a whole step to land. K of the tile past the
+  // last is clamped to it: a redundant copy that nothing reads.
+  f32x16 sa, sb;  // scores of the halves 0 and 1
+  bf16x8 pa[2], pb[2];
+  float psum = 0.f;
+  const uint32_t kl1 = kl + kHalfBytes, vl1 = vl + kHalfBytes;
+  const auto land = [&]() __attribute__((always_inline)) {
     wait_tile_copies();
     __syncthreads();
-    f32x16 s[2];
-    qk_tile<D>(kl, qreg, s);
-    finish_tile<BLK>(st, s, vl, plain_desc(), c, lane, NT, T);
-    __syncthreads();  // every wave is done with K and V
-    if (npipe > 0) issue_start();
-  }
+  };
+  // The pooled tile with a short last block's key, that key's score (-inf in the
+  // lanes without it), and the weight it lacks of BLK.
+  const int klast = npool ? NT - 1 - tl.pchunk[npool - 1] * kKeys : kKeys;
+  const int pshort = T % BLK != 0 && klast < kKeys ? npool - 1 : -1;
+  float slast = -INFINITY;
 
-  // ---- pooled and full exact tiles, pipelined by half tiles n = 2t, 2t + 1. On
-  // entry to step n: S(n) and P(n-1) in registers, K(n+1) and V(n-1) in LDS; the
-  // step copies K(n+2) over K(n) and V(n) over V(n-2), so a copy has a whole step
-  // to land. K of the tile past the last is clamped to it: a redundant copy that
-  // nothing reads.
-  if (npipe > 0) {
-    f32x16 sa, sb;
-    bf16x8 pa[2], pb[2];
-    wait_tile_copies();
-    __syncthreads();
-    {
-      const f32x16 zero = {};
+  // Step 0, without a stream: the running max comes from the whole first tile, so
+  // both halves' scores come first. (P is rounded relative to that max, and the
+  // keys at it round to nothing: with a max over the first 32 keys the result was
+  // 0.02-0.45% further from the exact one at block 64.)
+  land();
+  {
+    const uint64_t keep = first_pooled ? tl.pmask[0] : first_ragged ? exact_desc<BLK>(tl, tl.nexact - 1, T, NT).amask : ~0ull;
+    f32x16 s[2];
+    const f32x16 zero = {};
 #pragma unroll
-      for (int cc = 0; cc < D / 16; ++cc) sa = mfma_bf16(k_op_x<D>(kl, 0, cc), qreg[cc], cc == 0 ? zero : sa);
-    }
-    mfma_fence(sa);   // the steps read the scores through asm
+    for (int cc = 0; cc < D / 16; ++cc) s[0] = mfma_bf16(k_op_x<D>(kl, 0, cc), qreg[cc], cc == 0 ? zero : s[0]);
     __syncthreads();  // every wave is done with K(0)
-    const uint32_t kl1 = kl + kHalfBytes, vl1 = vl + kHalfBytes;
-    const int last = npipe - 1;
-    int t = 0;
-    const auto land = [&] {
-      wait_tile_copies();
-      __syncthreads();
-    };
-    // half steps 0 (its V came with the first copies) and 1
-    if (npool > 0) {
-      issue_any(min(1, last), 0, 0);
-      mask_scores(sa, static_cast<uint32_t>(tl.pmask[0]));
-      half_step<BLK, D, true, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
-      land();
-      issue_any(min(1, last), 0, 1);
-      issue_any(0, 1, 1);
-      mask_scores(sb, static_cast<uint32_t>(tl.pmask[0] >> 32));
-      half_step<BLK, D, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
-      land();
-      for (t = 1; t < npool; ++t) {
-        issue_any(min(t + 1, last), 0, 0);
-        issue_any(t, 1, 0);
-        mask_scores(sa, static_cast<uint32_t>(tl.pmask[t]));
-        half_step<BLK, D, true, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
-        land();
-        issue_any(min(t + 1, last), 0, 1);
-        issue_any(t, 1, 1);
-        mask_scores(sb, static_cast<uint32_t>(tl.pmask[t] >> 32));
-        half_step<BLK, D, true, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
-        land();
-      }
-    }
-    // The first token rows of tiles t and t + 1 are read from the LDS list an
-    // iteration ahead, so no copy waits on an LDS read.
-    int f0 = first_of(min(t, last)), f1 = first_of(min(t + 1, last));
-    if (npool == 0) {
-      issue_k_at(f1, 0);
-      half_step<BLK, D, false, false>(st, sa, sb, pb, pa, kl1, 0u, qreg, c);
-      land();
-      issue_k_at(f1, 1);
-      issue_v_at(f0, 1);
-      half_step<BLK, D, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
-      f0 = f1;
-      f1 = first_of(min(2, last));
-      land();
-      t = 1;
-    }
-    for (; t < npipe; ++t) {
-      issue_k_at(f1, 0);
-      issue_v_at(f0, 0);
-      half_step<BLK, D, false, true>(st, sa, sb, pb, pa, kl1, vl1, qreg, c);
-      asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
-      const int f2 = first_of(min(t + 2, last));
-      land();
-      issue_k_at(f1, 1);
-      issue_v_at(f0, 1);
-      half_step<BLK, D, false, true>(st, sb, sa, pa, pb, kl, vl, qreg, c);
-      land();
-      f0 = f1;
-      f1 = f2;
-    }
-    // P.V of the last half tile
-    mfma_fence(st.acc);
+    issue_any_k(min(1, last), 0);
 #pragma unroll
-    for (int i = 0; i < D / 16; ++i) {
-      const int ks = i / (D / 32), dt = i % (D / 32);
-      st.acc[dt] = mfma_bf16(v_op_x<D>(vl1, ks, dt), pb[ks], st.acc[dt]);
+    for (int cc = 0; cc < D / 16; ++cc) s[1] = mfma_bf16(k_op_x<D>(kl1, 0, cc), qreg[cc], cc == 0 ? zero : s[1]);
+    mask_scores(s, keep);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[m][r]);
+    st.m = xhalf_max(mx) * c;
+    if (first_pooled) {
+      if (pshort == 0) slast = score_of_key(s[0], klast, half);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[0][r], c, -st.m));
+        pa[r >> 3][r & 7] = static_cast<__bf16>(p);
+        psum += p;
+      }
+    } else {
+      psum = exp8<0>(s[0], c, -st.m, pa[0], psum);
+      psum = exp8<8>(s[0], c, -st.m, pa[1], psum);
     }
+    sb = s[1];
+  }
+  mfma_fence(st.acc);  // O's zeros are in their registers before the asm MFMAs that add to them
+  land();
+
+  // The half steps of the three kinds of tiles.
+  const auto pooled_next_k = [&](int p, int hh) __attribute__((always_inline)) {
+    if (!kPoolFirst || p + 1 < npool)
+      issue_pooled(min(p + 1, npool - 1), 0, hh);
+    else
+      issue_any_k(min(npool, last), hh);
+  };
+  const auto pooled_half0 = [&](int p) __attribute__((always_inline)) {
+    pooled_next_k(p, 0);
+    issue_pooled(p, 1, 0);
+    mask_scores(sa, static_cast<uint32_t>(tl.pmask[p]));
+    if (p == pshort) slast = score_of_key(sa, klast, half);
+    st.l *= half_step<D, true, 0>(st, sa, sb, pb, pa, kl1, vl1, qreg, c, psum);
+    land();
+  };
+  const auto pooled_half1 = [&](int p) __attribute__((always_inline)) {
+    pooled_next_k(p, 1);
+    issue_pooled(p, 1, 1);
+    mask_scores(sb, static_cast<uint32_t>(tl.pmask[p] >> 32));
+    if (p == pshort) slast = fmaxf(slast, score_of_key(sb, klast - 32, half));
+    const float alpha = half_step<D, true, 1>(st, sb, sa, pa, pb, kl, vl, qreg, c, psum);
+    psum *= static_cast<float>(BLK);
+    if (p == pshort)
+      psum = fmaf(__builtin_amdgcn_exp2f(fmaf(slast, c, -st.m)), static_cast<float>(T - NT * BLK), psum);
+    st.l = fmaf(st.l, alpha, psum);
+    land();
+  };
+  const auto ragged_half0 = [&]() __attribute__((always_inline)) {
+    issue_any_k(min(rag0 + 1, last), 0);
+    issue_ragged(1, 0);
+    mask_scores(sa, static_cast<uint32_t>(exact_desc<BLK>(tl, tl.nexact - 1, T, NT).amask));
+    st.l *= half_step<D, false, 0>(st, sa, sb, pb, pa, kl1, vl1, qreg, c, psum);
+    land();
+  };
+  const auto ragged_half1 = [&]() __attribute__((always_inline)) {
+    issue_any_k(min(rag0 + 1, last), 1);
+    issue_ragged(1, 1);
+    mask_scores(sb, static_cast<uint32_t>(exact_desc<BLK>(tl, tl.nexact - 1, T, NT).amask >> 32));
+    const float alpha = half_step<D, false, 1>(st, sb, sa, pa, pb, kl, vl, qreg, c, psum);
+    st.l = fmaf(st.l, alpha, psum);
+    land();
+  };
+  // f0, f1: the first token rows of full tiles e and e + 1, read from the LDS list
+  // an iteration ahead, so no copy waits on an LDS read
+  int f0 = 0, f1 = 0;
+  // (behind: K of the tile behind the last full one comes next)
+  const auto full_next_k = [&](int hh, bool behind) __attribute__((always_inline)) {
+    if (behind)
+      issue_any_k(min(nfull, last), hh);
+    else
+      issue_k_at(f1, hh);
+  };
+  const auto full_half0 = [&](bool behind) __attribute__((always_inline)) {
+    full_next_k(0, behind);
+    issue_v_at(f0, 0);
+    st.l *= half_step<D, false, 0>(st, sa, sb, pb, pa, kl1, vl1, qreg, c, psum);
+    land();
+  };
+  const auto full_half1 = [&](int e, bool behind) __attribute__((always_inline)) {
+    full_next_k(1, behind);
+    issue_v_at(f0, 1);
+    const float alpha = half_step<D, false, 1>(st, sb, sa, pa, pb, kl, vl, qreg, c, psum);
+    st.l = fmaf(st.l, alpha, psum);
+    asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
+    f0 = f1;
+    f1 = full_first(min(e + 2, nfull - 1));
+    land();
+  };
+
+  // The tiles in order; half 0 of the first one is step 0.
+  const auto pooled_tiles = [&]() __attribute__((always_inline)) {
+    if (npool == 0) return;
+    int p = 0;
+    if constexpr (kPoolFirst) pooled_half1(p++);
+    for (; p < npool; ++p) {
+      if (kPoolFirst || pool0 + p > 0) pooled_half0(p);
+      pooled_half1(p);
+    }
+  };
+  const auto ragged_tile = [&]() __attribute__((always_inline)) {
+    if (nrag == 0) return;
+    if (rag0 > 0) ragged_half0();
+    ragged_half1();
+  };
+  const auto full_tiles = [&]() __attribute__((always_inline)) {
+    if (nfull == 0) return;
+    f0 = full_first(0);
+    f1 = full_first(min(1, nfull - 1));
+    if constexpr (kPoolFirst) {
+      for (int e = 0; e < nfull; ++e) {
+        if (full0 + e > 0) full_half0(false);
+        full_half1(e, false);
+      }
+    } else {
+      int e = 0;
+      if (nfull > 1) {
+        full_half1(e++, false);
+        for (; e < nfull - 1; ++e) {
+          full_half0(false);
+          full_half1(e, false);
+        }
+        full_half0(true);
+      }
+      full_half1(e, true);
+    }
+  };
+  if constexpr (kPoolFirst) {
+    pooled_tiles();
+    ragged_tile();
+    full_tiles();
+  } else {
+    full_tiles();
+    ragged_tile();
+    pooled_tiles();
+  }
+  // P.V of the last half tile
+  mfma_fence(st.acc);
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) {
+    const int ks = i / (D / 32), dt = i % (D / 32);
+    st.acc[dt] = mfma_bf16(v_op_x<D>(vl1, ks, dt), pb[ks], st.acc[dt]);
   }
   wait_tile_copies();
 

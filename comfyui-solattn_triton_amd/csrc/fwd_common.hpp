@@ -322,18 +322,20 @@ struct CopyOffsets {
 };
 
 // Copies of half a bf16 tile (32 keys) into the half buffer at LDS byte address
-// dst: rows [32 hh, 32 hh + 32) of the pooled tile `td` (issue_pooled_half; rows past
-// nvalid re-read its last one, finite data that the softmax masks out), or the rows
-// from `base` on, `stride` elements apart (issue_half).
+// dst: rows [32 hh, 32 hh + 32) of the pooled or exact tile `td` (issue_clamped_half;
+// rows past nvalid re-read its last one, finite data that the softmax masks out), or
+// the rows from `base` on, `stride` elements apart (issue_half).
 template <int NTHREADS, int D>
-__device__ __forceinline__ void issue_pooled_half(uint32_t dst, int kv, const TileDesc& td, int hh,
-                                                  const KVSource& src) {
+__device__ __forceinline__ void issue_clamped_half(uint32_t dst, int kv, const TileDesc& td, int hh,
+                                                   const KVSource& src) {
   constexpr int C = D / 8, U = CopyOffsets<NTHREADS, D>::U / 2;
   const uint32_t l0 = dst + wave_id() * 64 * 16;
-  const uint16_t* b = (kv == 0 ? src.kc : src.vc) +
-                      static_cast<int64_t>(__builtin_amdgcn_readfirstlane(td.first)) * src.skc;
-  // (the row stride fits 32 bits, as 128 rows of kc and vc fit the memory; 63 of them need not)
-  const uint32_t stride = static_cast<uint32_t>(src.skc * 2), top = static_cast<uint32_t>(td.nvalid - 1);
+  const int64_t st = td.pooled ? src.skc : (kv == 0 ? src.sk : src.sv);
+  const uint16_t* b = (kv == 0 ? (td.pooled ? src.kc : src.k) : (td.pooled ? src.vc : src.v)) +
+                      static_cast<int64_t>(__builtin_amdgcn_readfirstlane(td.first)) * st;
+  // (the row stride fits 32 bits: 128 rows of kc and vc fit the memory, and token strides
+  // are below 2^24 elements; 63 rows need not)
+  const uint32_t stride = static_cast<uint32_t>(st * 2), top = static_cast<uint32_t>(td.nvalid - 1);
   // The addresses are made at each copy, not held through the pipeline: 4-18
   // registers fewer, and the BF16 call of 32760 tokens at block 64 2728 -> 2710 us.
   uint32_t tid = threadIdx.x;
@@ -488,7 +490,9 @@ __device__ __forceinline__ void pv_tile(uint32_t vl, const bf16x8 (&pb)[4], int 
 // hazards it would cover with wait states are covered here:
 //   VALU write -> MFMA read of that VGPR: 2 wait states, the s_nop 2 in front
 //     of the first P.V MFMA of a step (P and the rescaled O are written by
-//     VALU code before it);
+//     VALU code before it). O's first values are held in place by an mfma_fence
+//     before the first step: the compiler may otherwise write them right in front
+//     of the MFMA that adds to them;
 //   MFMA write -> VALU read of the result: at most NumPasses + 4 = 12 wait
 //     states for these 8-pass MFMAs; scores reach the softmax only through
 //     mfma_fence (16 wait states) or the in-out operands of the last MFMA
@@ -647,8 +651,8 @@ __device__ __forceinline__ void mask_scores(f32x16 (&s)[2], uint64_t amask) {
   mask_scores(s[1], static_cast<uint32_t>(amask >> 32));
 }
 
-// Softmax and P.V of one bf16 tile whose scores are in s (the plain path:
-// pooled, ragged and last tiles). Masked keys get -inf; pooled keys weigh
+// Softmax and P.V of one bf16 tile whose scores are in s (the INT8 forwards'
+// pooled tiles). Masked keys get -inf; pooled keys weigh
 // len_j in the row sum (/root/reference/_tri_fwd.py:302-307); P is rounded to
 // bf16 for the MFMA and, for exact tiles, summed as rounded (as on the
 // pipelined path).

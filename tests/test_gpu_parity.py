@@ -595,6 +595,69 @@ def test_fwd_bf16_half_chunk_exact(pkg, dev, block, T):
     _check_hand_set_masks(pkg, dev, block, T, exact_rows)
 
 
+def _rounded_p_model(q, qx, kx, vx, kc, vc, on, lens, first, block):
+    """The forward's arithmetic for one head with P rounded to bf16 against the running
+    max that its first tile gives (`first`: its keys, exact tokens [T] behind pooled blocks
+    [NT] in one row per query block), in float64 otherwise. q scores the pooled keys, qx the exact ones. Rows whose max a later tile
+    moves (by more than 8 in log2) are left out: [rows kept, model]."""
+    T, D = q.shape
+    tok = torch.arange(T, device=q.device) // block
+    c = D ** -0.5 * 1.4426950408889634
+    s = torch.cat([(q @ kc.t()).masked_fill(on[tok], -torch.inf),
+                   (qx @ kx.t()).masked_fill(~on[tok][:, tok], -torch.inf)], 1) * c
+    m = s.masked_fill(~first[tok], -torch.inf).amax(1, keepdim=True)
+    keep = s.amax(1) <= m[:, 0] + 8
+    p = torch.exp2(s - m)
+    pr = p.float().to(torch.bfloat16).double()
+    NT = kc.shape[0]
+    total = (p[:, :NT] * lens).sum(1) + pr[:, NT:].sum(1)  # pooled keys: the fp32 p, exact keys: the packed ones
+    return keep, (pr @ torch.cat([vc, vx])) / total[:, None]
+
+
+@pytest.mark.parametrize("block,T", [(64, 64 * 64), (64, 64 * 70 + 17), (128, 128 * 40), (128, 128 * 33 + 90)])
+@pytest.mark.parametrize("path", ["bf16"])
+def test_running_max_of_whole_first_tile(pkg, dev, path, block, T):
+    """P is rounded against the max of the whole first 64-key tile: pooled keys (block 64)
+    or tokens (block 128, INT8) first, as the order of the tiles is. The bound: fp32 scores
+    put one P in some 10^3 on the other side of a bf16 step and leave 1e-5 of the output,
+    which puts one output in 10^2 on the other side of its own (2^-9 each): 2e-4 in all
+    (measured 6e-5 to 1.1e-4). With the max of 32 keys every P rounds anew: 2e-3 to 3e-3."""
+    prep, tri, i8, fp = _mods(pkg)[:4]
+    q, k, v = (randn_bf16((1, T, 1, 128), s).to(dev) for s in (101, 102, 103))
+    kw = dict(tau=0.9, block=block, scale=128 ** -0.5)
+    print(f"[whole first tile] {path} block={block} T={T}", flush=True)
+    if path == "bf16":
+        r = prep.route(q, k, v, **kw)
+        out = tri.forward_bf16(q, k, v, r)
+        qx, kx = q[0, :, 0].double(), k[0, :, 0].double()
+    else:
+        r, qi, qs, ki, ks, _ = fp.fused_preprocess_routing(q, k, v, int8_pv=False, **kw)
+        out = i8.forward_int8(q, v, r, qi, qs, ki, ks, None, int8_pv=False)
+        qx, kx = (c[0, :, 0].double() * s[0, :, 0, None].double() for c, s in ((qi, qs), (ki, ks)))
+    NT = r.counts.shape[-1]
+    on = torch.from_numpy(mask_bits(u32(r.mask), NT)[0, 0]).to(dev)
+    j = torch.arange(NT, device=dev)
+    if block == 64 and path == "bf16":  # the first chunk of pooled keys
+        first = torch.cat([(~on) & (j < 64), torch.zeros(NT, T, dtype=torch.bool, device=dev)], 1)
+    else:  # the first exact block's first 64 tokens; INT8: the ragged last block's last tile before it
+        blk = on.int().argmax(1)
+        start = blk * block
+        if path != "bf16" and T % 64:
+            start = torch.where(on[:, NT - 1], T // 64 * 64, start)
+        t = torch.arange(T, device=dev)
+        inside = (t >= start[:, None]) & (t < start[:, None] + 64)
+        first = torch.cat([torch.zeros(NT, NT, dtype=torch.bool, device=dev), inside], 1)
+    lens = torch.full((NT,), float(block), dtype=torch.float64, device=dev)
+    lens[-1] = T - (NT - 1) * block
+    kc, vc = (t[0, :NT, 0].double() for t in (r.kc, r.vc))
+    keep, ref = _rounded_p_model(q[0, :, 0].double(), qx, kx, v[0, :, 0].double(), kc, vc, on, lens, first, block)
+    assert keep.float().mean() > 0.9
+    ref = ref.to(torch.bfloat16).double()[keep]
+    rel = float((out[0, :, 0].double()[keep] - ref).norm() / ref.norm())
+    print(f"    rel {rel:.2e}", flush=True)
+    assert rel < 4e-4
+
+
 @pytest.mark.parametrize("block,T", [(64, 64 * 67 + 17), (64, 64 * 66), (128, 128 * 66 + 90), (128, 128 * 65 + 64),
                                      (128, 128 * 65 + 17)])
 def test_fwd_int8_bf16pv_hand_set_masks(pkg, dev, block, T):

@@ -315,47 +315,43 @@ __device__ __forceinline__ f32x4 ks_quad(uint32_t a) {
 // MFMA i (i < 4), the exps of P(n) word i, then P.V MFMA i; slots 4-7 also
 // convert four int32 scores of S(n+1) to fp32 times their ks (read a slot
 // ahead). Two exp pairs and a P.V MFMA follow the last score MFMA before its
-// int32 scores are read. PV = false: the first half tile. Lazy tile max, hazards
-// and the O rescale as in half_step. qc: the factor of sc's scores; K(n+1), its
-// ks and V(n-1) are in half buffer HH, kl, ksl and vl this lane's operand addresses
-// in half buffer 0.
-template <int HH, bool PV, bool UKS>
-__device__ __forceinline__ void half_step_i8(SoftmaxState& st, const f32x16& sc, float qc, f32x16& sn,
-                                             const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
-                                             uint32_t ksl, uint32_t vl, const i32x4 (&qi)[4]) {
+// int32 scores are read. HH: the half of its tile that n is. Lazy tile max, psum,
+// hazards, the O rescale and the result as in half_step. qc: the factor of sc's
+// scores; kl, ksl and vl: this lane's operand addresses in half buffer 0 (K(n+1),
+// its ks and V(n-1) are in the other half's buffer).
+template <int HH, bool UKS>
+__device__ __forceinline__ float half_step_i8(SoftmaxState& st, const f32x16& sc, float qc, f32x16& sn,
+                                              const bf16x8 (&pp)[2], bf16x8 (&pn)[2], uint32_t kl,
+                                              uint32_t ksl, uint32_t vl, const i32x4 (&qi)[4], float& psum) {
+  constexpr int BUF = 1 - HH, KOFF = BUF * kHalfKStride;
   i32x16 si;
   i32x4 ka[3];
   bf16x8 va[3];
   f32x4 kq[2];
   uint32_t pw[2][4];
-  float psum = 0.f;
+  const float before = HH == 0 ? 0.f : psum;
+  if constexpr (HH == 0) psum = 0.f;
   const float neg = -st.m;
-  ka[0] = ki_op_x(kl, 0, HH * kHalfKStride);
-  ka[1] = ki_op_x(kl, 1, HH * kHalfKStride);
-  if constexpr (PV) {
-    va[0] = v_op_x(vl, 2 * HH, 0);
-    va[1] = v_op_x(vl, 2 * HH, 1);
-  }
+  ka[0] = ki_op_x(kl, 0, KOFF);
+  ka[1] = ki_op_x(kl, 1, KOFF);
+  va[0] = v_op_x(vl, 2 * BUF, 0);
+  va[1] = v_op_x(vl, 2 * BUF, 1);
   asm volatile("" ::: "memory");
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    if (i + 2 < 4) ka[(i + 2) % 3] = ki_op_x(kl, i + 2, HH * kHalfKStride);
-    if (!UKS && i >= 3 && i < 7) kq[(i - 3) & 1] = ks_quad(ksl + HH * kHalfKStride + 32 * (i - 3));
-    if constexpr (PV) {
-      if (i + 2 < 8) va[(i + 2) % 3] = v_op_x(vl, 2 * HH + ((i + 2) >> 2), (i + 2) & 3);
-    }
+    if (i + 2 < 4) ka[(i + 2) % 3] = ki_op_x(kl, i + 2, KOFF);
+    if (!UKS && i >= 3 && i < 7) kq[(i - 3) & 1] = ks_quad(ksl + KOFF + 32 * (i - 3));
+    if (i + 2 < 8) va[(i + 2) % 3] = v_op_x(vl, 2 * BUF + ((i + 2) >> 2), (i + 2) & 3);
     asm volatile("" ::: "memory");
     if (i == 0)
       mfma_i8_v0(si, ka[0], qi[0]);
     else if (i < 4)
       mfma_i8_v(si, ka[i % 3], qi[i]);
     pw[i >> 2][i & 3] = exp_pair(sc[2 * i], sc[2 * i + 1], qc, neg, psum);
-    if constexpr (PV) {
-      if (i == 0)
-        mfma_v_first(st.acc[0], va[0], pp[0]);
-      else
-        mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
-    }
+    if (i == 0)
+      mfma_v_first(st.acc[0], va[0], pp[0]);
+    else
+      mfma_v(st.acc[i & 3], va[i % 3], pp[i >> 2]);
     if (i == 4) asm volatile("" : "+v"(si));  // the int32 scores are read after this
     if (i >= 4) {
 #pragma unroll
@@ -379,13 +375,13 @@ __device__ __forceinline__ void half_step_i8(SoftmaxState& st, const f32x16& sc,
     const float m_new = new_max(st.m, xhalf_max(mx) * qc, alpha);
     if (__any(m_new != st.m)) {  // lanes whose max stays recompute the same P
       st.m = m_new;
-      psum = exp8<0>(sc, qc, -m_new, pn[0], 0.f);
+      psum = exp8<0>(sc, qc, -m_new, pn[0], before * alpha);
       psum = exp8<8>(sc, qc, -m_new, pn[1], psum);
-      if constexpr (PV) mfma_fence(st.acc);  // the rescale reads O
+      mfma_fence(st.acc);  // the rescale reads O
       rescale(st, alpha);
     }
   }
-  st.l = fmaf(st.l, alpha, psum);
+  return alpha;
 }
 
 // Pipelined step over full exact tile n (scaled scores in sc, factor qsl):
@@ -652,51 +648,67 @@ fwd_int8_bf16pv_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_
       const uint32_t kl = ki_lane(kb, col, half), ksl = kb + kHalfKs + 16 * half, vl = v_lane(vb, lane);
       // the factor of half buffer hh's scores
       const auto factor = [&](int hh) { return tile_qsl<UKS>(arena + hh * kHalfKStride, kHalfKs, qsl); };
-      f32x16 sa, sb;
+      f32x16 sa, sb;  // scores of the halves 0 and 1
       bf16x8 pa[2], pb[2];
-      land();
-      {
-        const i32x16 zero = {};
-        i32x16 si;
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) si = mfma_i8(ki_op_x(kl, cc, 0), qireg[cc], cc == 0 ? zero : si);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float f = static_cast<float>(si[e]);
-          sa[e] = UKS ? f : f * ks_quad(ksl + 32 * (e >> 2))[e & 3];
-        }
-      }
-      float fa = factor(0), fb;
-      __syncthreads();  // every wave is done with K(0)
       const int last = nfast - 1;
       // The first token rows of tiles t and t + 1 are read from the LDS list an
       // iteration ahead. K of the tile past the last is clamped to it: a redundant
       // copy into a buffer that nothing reads afterwards.
       int f0 = first_of(0), f1 = first_of(min(1, last));
-      issue_k(f1, 0);
-      half_step_i8<1, false, UKS>(st, sa, fa, sb, pb, pa, kl, ksl, vl, qireg);
-      fb = factor(1);
+      const auto half_scores = [&](int hh, f32x16& s) {
+        const i32x16 zero = {};
+        i32x16 si;
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc)
+          si = mfma_i8(ki_op_x(kl, cc, hh * kHalfKStride), qireg[cc], cc == 0 ? zero : si);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float f = static_cast<float>(si[e]);
+          s[e] = UKS ? f : f * ks_quad(ksl + hh * kHalfKStride + 32 * (e >> 2))[e & 3];
+        }
+      };
+      // Step 0 without a stream, as in the BF16 forward: the running max comes from
+      // the whole first tile.
       land();
-      issue_k(f1, 1);
-      issue_v(f0, 1);
-      half_step_i8<0, true, UKS>(st, sb, fb, sa, pa, pb, kl, ksl, vl, qireg);
-      fa = factor(0);
+      half_scores(0, sa);
+      float fa = factor(0), fb;
+      __syncthreads();  // every wave is done with K(0)
+      issue_k(f1, 0);
+      half_scores(1, sb);
+      fb = factor(1);
+      float psum;
+      {
+        float mx = -INFINITY, alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaxf(sa[r], sb[r]));
+        st.m = new_max(st.m, xhalf_max(mx) * fa, alpha);  // (both halves of a tile have one factor)
+        psum = exp8<0>(sa, fa, -st.m, pa[0], 0.f);
+        psum = exp8<8>(sa, fa, -st.m, pa[1], psum);
+        st.l *= alpha;
+        rescale(st, alpha);
+      }
+      mfma_fence(st.acc);  // O is in its registers before the asm MFMAs that add to it
+      land();
+      const auto half1 = [&]() __attribute__((always_inline)) {
+        issue_k(f1, 1);
+        issue_v(f0, 1);
+        const float alpha = half_step_i8<1, UKS>(st, sb, fb, sa, pa, pb, kl, ksl, vl, qireg, psum);
+        st.l = fmaf(st.l, alpha, psum);
+        fa = factor(0);
+        land();
+      };
+      half1();
       f0 = f1;
       f1 = first_of(min(2, last));
-      land();
       for (int t = 1; t < nfast; ++t) {
         issue_k(f1, 0);
         issue_v(f0, 0);
-        half_step_i8<1, true, UKS>(st, sa, fa, sb, pb, pa, kl, ksl, vl, qireg);
+        st.l *= half_step_i8<0, UKS>(st, sa, fa, sb, pb, pa, kl, ksl, vl, qireg, psum);
         fb = factor(1);
         asm volatile("" ::: "memory");  // the list read stays behind the MFMA stream
         const int f2 = first_of(min(t + 2, last));
         land();
-        issue_k(f1, 1);
-        issue_v(f0, 1);
-        half_step_i8<0, true, UKS>(st, sb, fb, sa, pa, pb, kl, ksl, vl, qireg);
-        fa = factor(0);
-        land();
+        half1();
         f0 = f1;
         f1 = f2;
       }

@@ -615,7 +615,7 @@ def _rounded_p_model(q, qx, kx, vx, kc, vc, on, lens, first, block):
 
 
 @pytest.mark.parametrize("block,T", [(64, 64 * 64), (64, 64 * 70 + 17), (128, 128 * 40), (128, 128 * 33 + 90)])
-@pytest.mark.parametrize("path", ["bf16"])
+@pytest.mark.parametrize("path", ["bf16", "int8_bf16pv"])
 def test_running_max_of_whole_first_tile(pkg, dev, path, block, T):
     """P is rounded against the max of the whole first 64-key tile: pooled keys (block 64)
     or tokens (block 128, INT8) first, as the order of the tiles is. The bound: fp32 scores

@@ -154,7 +154,9 @@ extern "C" int solattn_reorder_rows(const void* src, int64_t src_rows, int64_t s
   SOLATTN_REQUIRE(rows < (1ll << 31) && row_bytes / 16 < (1ll << 24) && batch <= 65535,
                   SOLATTN_EUNSUPPORTED, "reorder: sizes beyond the 32-bit index range");
   const uint32_t cpr = static_cast<uint32_t>(row_bytes / 16);
-  if (cpr >= kWaveRowChunks) {
+  // A launch covers fewer than 2^32 threads in x, and drops the rest without an error:
+  // more rows than that take the flat form.
+  if (cpr >= kWaveRowChunks && cdiv(rows, kRowWaves) * kReorderThreads < (1ll << 32)) {
     using Kern = decltype(&reorder_rows_wave_kernel<1>);
     constexpr Kern kerns[8] = {reorder_rows_wave_kernel<1>, reorder_rows_wave_kernel<2>,
                                reorder_rows_wave_kernel<3>, reorder_rows_wave_kernel<4>,

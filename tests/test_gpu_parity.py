@@ -187,6 +187,20 @@ def test_reorder_row_lengths(pkg, dev, chunks):
     assert torch.equal(out, want)
 
 
+def test_reorder_rows_past_one_launch(pkg, dev):
+    """2^26 rows and more, a wave each, are 2^32 threads: more than a launch covers in x.
+    Every row is written (rows of 40 chunks of one value, 16 bytes apart in the output)."""
+    capi = importlib.import_module(f"{pkg.__name__}._capi")
+    rows = (1 << 26) + 5
+    print(f"[reorder rows] {rows}", flush=True)
+    src = torch.full((320,), 7.0, dtype=torch.bfloat16, device=dev)
+    out = torch.zeros(rows * 8 + 312, dtype=torch.bfloat16, device=dev)
+    idx = torch.zeros(rows, dtype=torch.int64, device=dev)
+    capi.call("solattn_reorder_rows", capi.ptr(src), 1, 0, 0, capi.ptr(out), 0, 16, 1, rows, 640, capi.ptr(idx),
+              capi.stream(dev))
+    assert bool((out == 7.0).all())
+
+
 FWD_CASES = [  # (B, T, H, block, tau, sink_kv, sink_q)
     (1, 1000, 2, 64, 0.9, (0, 0), (0, 0)),      # ragged last tile
     (1, 2500, 2, 128, 0.9, (0, 0), (0, 0)),     # block 128: 64-row full tile + 4-row ragged tile

@@ -1,7 +1,7 @@
 // Row gather for the Morton token permutation and its inverse:
 //   dst[b, t, :] = src[b, index[t], :]
-// HBM-bound copy in 16-byte lanes: a wave per row, or, for short rows, a run of
-// whole rows per workgroup taken as one sequence of chunks. Replaces the
+// HBM-bound copy in 16-byte lanes: a wave per row (per 8 KiB of a longer one), or,
+// for short rows, a run of whole rows per workgroup taken as one sequence of chunks. Replaces the
 // torch index_select calls of /root/reference/_morton.py:113,128,148 and
 // /root/reference/_morton_h3.py:193,217.
 #include <algorithm>
@@ -50,44 +50,47 @@ reorder_rows_kernel(const char* __restrict__ src, int64_t src_stride_b, int64_t 
   }
 }
 
-// Rows of at least kWaveRowChunks chunks: one wave per row. The row's index is wave-uniform
-// (a scalar load), so a chunk needs no division and no index of its own, and all U
-// loads of a pass go out before the first store; lanes past the row's end re-read
-// its last chunk and store nothing. A pass covers 64 U chunks, U chosen so that a
-// row's passes are even. An index outside the source rows yields a zero row.
+// Rows of at least kWaveRowChunks chunks: one wave per piece of 64 U chunks of a row,
+// U chosen so that a row's pieces are even; rows of up to 512 chunks are one piece.
+// The row's index is wave-uniform (a scalar load), so a chunk needs no division and no
+// index of its own, and all U loads go out before the first store; lanes past the
+// row's end re-read its last chunk and store nothing. An index outside the source rows
+// yields a zero row. (One wave for all pieces of a row left the chip idle where rows
+// are few and long: 16 rows of 1 MiB 115 us, against 85 us in the flat form.)
 // Bound: HBM and the infinity cache. 134 MB of random rows, against the flat form:
 // 32 chunks a row 56 vs 53 us (lanes idle), 40 50 vs 56, 64 43 vs 53, 384 44 vs 50;
-// hence the line. 32760 rows of 6 KiB, there and back: 164.1 -> 147.6 us (5.45 TB/s).
+// hence the line. Pieces of a row in neighbouring workgroups: 75600 rows of 10 KiB 300
+// us, 307 with all first pieces before the second ones. 32760 rows of 6 KiB, there and back: 164.1 -> 147.6 us (5.45 TB/s).
 constexpr uint32_t kWaveRowChunks = 40;
 constexpr int kRowWaves = kReorderThreads / 64;
-template <int U>
+template <int U, bool WHOLE>  // WHOLE: rows are one piece
 __global__ void __launch_bounds__(kReorderThreads)
 reorder_rows_wave_kernel(const char* __restrict__ src, int64_t src_stride_b, int64_t src_stride_row,
                          char* __restrict__ dst, int64_t dst_stride_b, int64_t dst_stride_row,
                          const int64_t* __restrict__ index, int64_t src_rows, uint32_t rows,
-                         uint32_t chunks_per_row) {
+                         uint32_t chunks_per_row, uint32_t pieces) {
+  const uint32_t group = WHOLE ? blockIdx.x : blockIdx.x / pieces;
   const uint32_t r = static_cast<uint32_t>(
-      __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kRowWaves + (threadIdx.x >> 6))));
+      __builtin_amdgcn_readfirstlane(static_cast<int>(group * kRowWaves + (threadIdx.x >> 6))));
   if (r >= rows) return;
   const int64_t srow = index[r];
   const bool valid = srow >= 0 && srow < src_rows;
   const uint32_t lane = threadIdx.x & 63;
   const char* s = src + static_cast<int64_t>(blockIdx.y) * src_stride_b + (valid ? srow : 0) * src_stride_row;
   char* d = dst + static_cast<int64_t>(blockIdx.y) * dst_stride_b + static_cast<int64_t>(r) * dst_stride_row;
-  for (uint32_t c0 = 0; c0 < chunks_per_row; c0 += 64 * U) {
-    uint4 v[U];
+  const uint32_t c0 = WHOLE ? 0 : (blockIdx.x - group * pieces) * 64 * U;
+  uint4 v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      v[u] = *reinterpret_cast<const uint4*>(s + min(c0 + 64 * u + lane, chunks_per_row - 1) * 16ull);
-    if (!valid) {
+  for (int u = 0; u < U; ++u)
+    v[u] = *reinterpret_cast<const uint4*>(s + min(c0 + 64 * u + lane, chunks_per_row - 1) * 16ull);
+  if (!valid) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = make_uint4(0u, 0u, 0u, 0u);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c0 + 64 * u + lane < chunks_per_row)
-        *reinterpret_cast<uint4*>(d + (c0 + 64 * u + lane) * 16ull) = v[u];
+    for (int u = 0; u < U; ++u) v[u] = make_uint4(0u, 0u, 0u, 0u);
   }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (c0 + 64 * u + lane < chunks_per_row)
+      *reinterpret_cast<uint4*>(d + (c0 + 64 * u + lane) * 16ull) = v[u];
 }
 
 // ------------------------------------------------------------- head padding
@@ -156,19 +159,23 @@ extern "C" int solattn_reorder_rows(const void* src, int64_t src_rows, int64_t s
   const uint32_t cpr = static_cast<uint32_t>(row_bytes / 16);
   // A launch covers fewer than 2^32 threads in x, and drops the rest without an error:
   // more rows than that take the flat form.
-  if (cpr >= kWaveRowChunks && cdiv(rows, kRowWaves) * kReorderThreads < (1ll << 32)) {
-    using Kern = decltype(&reorder_rows_wave_kernel<1>);
-    constexpr Kern kerns[8] = {reorder_rows_wave_kernel<1>, reorder_rows_wave_kernel<2>,
-                               reorder_rows_wave_kernel<3>, reorder_rows_wave_kernel<4>,
-                               reorder_rows_wave_kernel<5>, reorder_rows_wave_kernel<6>,
-                               reorder_rows_wave_kernel<7>, reorder_rows_wave_kernel<8>};
-    const int64_t waves = cdiv(cpr, 64), passes = cdiv(waves, 8);
-    hipLaunchKernelGGL(kerns[cdiv(waves, passes) - 1],
-                       dim3(static_cast<uint32_t>(cdiv(rows, kRowWaves)), static_cast<uint32_t>(batch)),
+  const int64_t waves = cdiv(cpr, 64), pieces = cdiv(waves, 8), groups = cdiv(rows, kRowWaves) * pieces;
+  if (cpr >= kWaveRowChunks && groups * kReorderThreads < (1ll << 32)) {
+    using Kern = decltype(&reorder_rows_wave_kernel<1, true>);
+    constexpr Kern whole[8] = {reorder_rows_wave_kernel<1, true>, reorder_rows_wave_kernel<2, true>,
+                               reorder_rows_wave_kernel<3, true>, reorder_rows_wave_kernel<4, true>,
+                               reorder_rows_wave_kernel<5, true>, reorder_rows_wave_kernel<6, true>,
+                               reorder_rows_wave_kernel<7, true>, reorder_rows_wave_kernel<8, true>};
+    // (the pieces of a longer row have at least 5 chunks a lane: 9 or more, in two)
+    constexpr Kern split[4] = {reorder_rows_wave_kernel<5, false>, reorder_rows_wave_kernel<6, false>,
+                               reorder_rows_wave_kernel<7, false>, reorder_rows_wave_kernel<8, false>};
+    const int64_t U = cdiv(waves, pieces);
+    hipLaunchKernelGGL(pieces == 1 ? whole[U - 1] : split[U - 5],
+                       dim3(static_cast<uint32_t>(groups), static_cast<uint32_t>(batch)),
                        dim3(kReorderThreads), 0, reinterpret_cast<hipStream_t>(stream),
                        static_cast<const char*>(src), src_stride_b_bytes, src_stride_row_bytes,
                        static_cast<char*>(dst), dst_stride_b_bytes, dst_stride_row_bytes, index, src_rows,
-                       static_cast<uint32_t>(rows), cpr);
+                       static_cast<uint32_t>(rows), cpr, static_cast<uint32_t>(pieces));
     return check_launch("reorder_rows");
   }
   // About 4096 chunks (64 KiB) per workgroup, at least one row.

@@ -165,10 +165,10 @@ def test_reorder_matches_index_select(pkg, dev):
     assert torch.equal(mort.reorder_tokens(s, idx, dim=0), s[idx])
 
 
-@pytest.mark.parametrize("chunks", [1, 39, 40, 41, 63, 64, 65, 128, 129, 449, 511, 512, 513, 1025])
+@pytest.mark.parametrize("chunks", [1, 39, 40, 41, 63, 64, 65, 128, 129, 449, 511, 512, 513, 800, 1000, 1025, 5003])
 def test_reorder_row_lengths(pkg, dev, chunks):
     """Rows around the lengths where the copy changes form (40 chunks of 16 bytes,
-    one more load per lane, one more pass of 512), strided source rows, a row count that leaves waves idle,
+    one more load per lane, one more piece of 512), strided source rows, a row count that leaves waves idle,
     and an index outside the source (its row is zeroed)."""
     mod, capi = _mods(pkg)[5], importlib.import_module(f"{pkg.__name__}._capi")
     print(f"[reorder rows] chunks={chunks}", flush=True)

@@ -369,6 +369,8 @@ int sol_attn_int8_call(SOLATTN_INT8_CALL_PARAMS, int qk_block) {
   if (int rc = check_pipeline(B, T, H, D, block, "sol_attn_int8")) return rc;
   SOLATTN_REQUIRE(int8_pv >= SOLATTN_PV_BF16 && int8_pv <= SOLATTN_PV_INT8_RUNNING, SOLATTN_EINVAL,
                   "sol_attn_int8: int8_pv %d is not a SOLATTN_PV_* mode", int8_pv);
+  SOLATTN_REQUIRE(!int8_pv || H < kMaxVScaleHeads, SOLATTN_EUNSUPPORTED,
+                  "sol_attn_int8: %lld heads with int8 P.V (at most %d)", (long long)H, kMaxVScaleHeads - 1);
   const Layout L(B, T, H, D, block, true);
   SOLATTN_REQUIRE(workspace && workspace_bytes >= L.total, SOLATTN_ESIZE,
                   "sol_attn_int8: workspace %lld < %lld bytes", (long long)workspace_bytes,

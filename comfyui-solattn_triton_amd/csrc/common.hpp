@@ -102,6 +102,9 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// moments_kernel's 32-bit offsets into the |v| maxima: heads that a V scale can have.
+constexpr int kMaxVScaleHeads = 32768;
+
 // The stages of the one-call pipelines for head dims 128 and (BF16 only) 64;
 // arguments are validated as in the public entry points, which take 128 alone.
 // pool_checked: the pooling pass (prep.hip) with, when qi != null, the per-token

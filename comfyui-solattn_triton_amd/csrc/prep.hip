@@ -1022,8 +1022,8 @@ int moments(uint16_t* kc, int64_t npad, int64_t B, int64_t NT, int64_t H, int64_
                   SOLATTN_EINVAL, "moments: bad sizes");
   SOLATTN_REQUIRE(kc && kc_mean && kc_var, SOLATTN_EINVAL, "moments: null pointer");
   SOLATTN_REQUIRE(!vamax_part || vscale, SOLATTN_EINVAL, "moments: vamax_part needs vscale");
-  SOLATTN_REQUIRE(!vamax_part || H < 32768, SOLATTN_EUNSUPPORTED,
-                  "moments: %lld heads with vamax_part (at most 32767)", (long long)H);
+  SOLATTN_REQUIRE(!vamax_part || H < kMaxVScaleHeads, SOLATTN_EUNSUPPORTED,
+                  "moments: %lld heads with vamax_part (at most %d)", (long long)H, kMaxVScaleHeads - 1);
   SOLATTN_REQUIRE(reinterpret_cast<uintptr_t>(kc) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(vamax_part) % 16 == 0,
                   SOLATTN_EINVAL, "moments: kc and vamax_part must be 16-byte aligned");

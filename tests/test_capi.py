@@ -132,6 +132,18 @@ def test_int8_pv_modes(capi, pkg):
         i8._pv_mode(True, "tile")
 
 
+def test_int8_call_head_limit(capi):
+    """32768 heads and more with int8 P.V are refused at every length, also where the
+    moments run inside the routing launch (no device work: stand-in addresses)."""
+    L = capi.LIB
+    a = 1 << 20
+    for T in (1, 64 * 128, 64 * 129):
+        for H, rc_want, text in ((32768, -2, b"heads"), (32767, -4, b"workspace")):
+            rc = L.solattn_sol_attn_int8(*([a, 0, 128, 0] * 3), 1, T, H, 128, 64, 0.1, 1.0, 0, 0, 0, 0, 1, a, 1,
+                                         a, 0, 128, 0, None)
+            assert rc == rc_want and text in L.solattn_last_error()
+
+
 def test_noalloc_rejects_oversize_before_device_work(capi):
     """The allocation-free pipeline refuses shapes whose intermediates exceed
     its fixed scratch, with SOLATTN_ESIZE, before it touches a device."""

@@ -409,10 +409,20 @@ extern "C" int solattn_preprocess_int8(
   SOLATTN_REQUIRE(D == kKernelD, SOLATTN_EUNSUPPORTED, "preprocess_int8: head_dim %lld != 128", (long long)D);
   SOLATTN_REQUIRE(block == 64 || block == 128, SOLATTN_EUNSUPPORTED,
                   "preprocess_int8: block %lld not in {64, 128}", (long long)block);
-  SOLATTN_REQUIRE(T > 0 && qi && qs && ki && ks && (!vscale || (vamax_part && vi)), SOLATTN_EINVAL,
-                  "preprocess_int8: empty sequence or null output");
+  // Everything that a stage behind the first would refuse is refused before it runs.
+  const auto aligned = [](const void* p, int n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
+  SOLATTN_REQUIRE(T > 0 && kc && vc && qbar && kc_mean && kc_var && thr && counts && mask && qi && qs && ki &&
+                      ks && (!vscale || (vamax_part && vi)),
+                  SOLATTN_EINVAL, "preprocess_int8: empty sequence or null output");
   SOLATTN_REQUIRE(npad >= cdiv(T, block) && npad < (1ll << 31), SOLATTN_EINVAL, "preprocess_int8: npad %lld",
                   (long long)npad);
+  SOLATTN_REQUIRE(cdiv(cdiv(T, block), 32) <= kMaxWords, SOLATTN_EUNSUPPORTED,
+                  "preprocess_int8: %lld blocks exceed %d", (long long)cdiv(T, block), kMaxWords * 32);
+  SOLATTN_REQUIRE(!vscale || H < kMaxVScaleHeads, SOLATTN_EUNSUPPORTED,
+                  "preprocess_int8: %lld heads with a V scale (at most %d)", (long long)H, kMaxVScaleHeads - 1);
+  SOLATTN_REQUIRE(aligned(kc, 16) && (!vscale || (aligned(vamax_part, 16) && aligned(vi, 8))) && aligned(qi, 8) &&
+                      aligned(ki, 8),
+                  SOLATTN_EINVAL, "preprocess_int8: kc and vamax_part must be 16-byte aligned, codes 8-byte");
   int rc = pool_checked(q, sq_b, sq_t, sq_h, k, sk_b, sk_t, sk_h, v, sv_b, sv_t, sv_h, B, T, H, D, block,
                         kc, vc, npad, qbar, vscale ? vamax_part : nullptr, qk_block ? nullptr : qi,
                         qk_block ? nullptr : qs, T, s, static_cast<int>(npad));

@@ -102,6 +102,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+constexpr int kMaxWords = 512;  // mask words of a query block: NT <= 16384 (the forwards' limit)
 // moments_kernel's 32-bit offsets into the |v| maxima: heads that a V scale can have.
 constexpr int kMaxVScaleHeads = 32768;
 

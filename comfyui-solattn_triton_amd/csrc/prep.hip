@@ -660,7 +660,6 @@ prep_int8_single_read_kernel(const PrepInt8Args a) {
 // One launch for two: 3.6 + 9.1 -> 8.2 us at NT 16, 4.5 + 9.2 -> 8.7 at NT 64,
 // 7.2 + 13.0 -> 18.0 at NT 81 with the INT8 outputs.
 constexpr int kRouteThreads = 256;
-constexpr int kMaxWords = 512;  // NT <= 16384 (the forwards' limit)
 enum RouteFuse { kNoFuse = 0, kMoments = 1, kCentred = 2 };
 
 struct RouteArgs {

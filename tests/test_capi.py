@@ -144,6 +144,33 @@ def test_int8_call_head_limit(capi):
             assert rc == rc_want and text in L.solattn_last_error()
 
 
+def test_preprocess_int8_rejects_before_any_launch(capi):
+    """solattn_preprocess_int8 refuses what any of its stages would (null or unaligned
+    outputs, too many blocks or heads) before the first of them runs: nothing here
+    reaches a launch, and every address is a stand-in."""
+    L = capi.LIB
+    a = 1 << 20
+    outs = ["kc", "vc", "npad", "qbar", "kc_mean", "kc_var", "vamax", "vscale", "thr", "counts", "mask", "qi", "qs",
+            "ki", "ks", "vi"]
+
+    def call(T=1000, H=2, block=64, **kw):
+        st = H * 128
+        vals = {n: a for n in outs}
+        vals["npad"] = -(-T // block) + 63
+        vals.update(kw)
+        return L.solattn_preprocess_int8(*([a, 0, st, 128] * 3), 1, T, H, 128, block, 0.1, 1.0, 0, 0, 0, 0, 0,
+                                         *(vals[n] for n in outs), None)
+
+    for name in outs:
+        if name not in ("npad", "vscale"):
+            assert call(**{name: None}) == -1 and b"null" in L.solattn_last_error(), name
+    for name, off in (("qi", 4), ("ki", 4), ("vi", 4), ("kc", 8), ("vamax", 8)):
+        assert call(**{name: a + off}) == -1 and b"aligned" in L.solattn_last_error(), name
+    assert call(T=64 * 16385) == -2 and b"exceed" in L.solattn_last_error()
+    assert call(H=32768) == -2 and b"heads" in L.solattn_last_error()
+    assert call(npad=3) == -1 and b"npad" in L.solattn_last_error()
+
+
 def test_noalloc_rejects_oversize_before_device_work(capi):
     """The allocation-free pipeline refuses shapes whose intermediates exceed
     its fixed scratch, with SOLATTN_ESIZE, before it touches a device."""

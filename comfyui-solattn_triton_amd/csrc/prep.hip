@@ -50,9 +50,9 @@ struct PoolLane {
         c8(static_cast<int>(threadIdx.x & 15) * 8) {}
 };
 
-// The lane's kSlotRows rows of one head (xh = x + b*sb + h*sh + c8, row stride
-// st) from span row r0; rows past T re-read row T-1 (unconditional loads, so
-// all are in flight together; the pooling adds 0.0f for them).
+// The lane's kSlotRows rows of one head (xh = x + b*sb + h*sh + c8, a per-lane
+// address; row stride st) from span row r0; rows past T re-read row T-1
+// (unconditional loads, so all are in flight together; the pooling adds 0.0f for them).
 __device__ __forceinline__ void load_span(const uint16_t* xh, int64_t st, int64_t r0, int64_t T,
                                           int g, uint4 (&raw)[kSlotRows]) {
 #pragma unroll
@@ -163,15 +163,6 @@ __device__ __forceinline__ void quant_span_rows_buf(const uint4 (&raw)[kSlotRows
   }
 }
 
-// load_span_buf for the lane's own head (64-channel heads): xl is a per-lane
-// address, rows past T re-read row T-1 (the pooling adds 0.0f for them).
-__device__ __forceinline__ void load_span_lane(const uint16_t* xl, int64_t st, int64_t r0, int64_t T,
-                                               int g, uint4 (&raw)[kSlotRows]) {
-#pragma unroll
-  for (int m = 0; m < kSlotRows; ++m)
-    raw[m] = *reinterpret_cast<const uint4*>(xl + min(r0 + g + 16 * m, T - 1) * st);
-}
-
 // QUANT: Q's rows come first and are quantised while K's and V's land, then
 // Q, K and V are pooled in that order; otherwise K, V, Q. AMAX: the per-block
 // |v| max (vamax_part). HD: the head dim, 128 or 64. At 64 a workgroup covers
@@ -199,7 +190,7 @@ pool_kernel(const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_t, int64_t 
     if constexpr (HD == kHeadDim)
       load_span_buf(x + b * sb + h0 * sh, st, r0, T, pl, raw);
     else
-      load_span_lane(x + b * sb + min(h0 + pl.c8 / HD, H - 1) * sh + pl.c8 % HD, st, r0, T, pl.g, raw);
+      load_span(x + b * sb + min(h0 + pl.c8 / HD, H - 1) * sh + pl.c8 % HD, st, r0, T, pl.g, raw);
   };
   if (QUANT) load(q, sq_b, sq_t, sq_h, rq);
   load(k, sk_b, sk_t, sk_h, rk);

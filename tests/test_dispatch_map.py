@@ -1,78 +1,25 @@
 """Host-side check of the forward kernels' workgroup -> query-block mapping.
 
-The forwards (``csrc/fwd_common.hpp``, ``tile_coords_lpt``) deal workgroups
-to XCDs round-robin, give each XCD a contiguous run of query blocks, and
-inside each window of 8192 query tokens (64 dispatches at block 128, 128 at
-block 64) take the query blocks longest first. The
-mapping must be a permutation of ``[0, grid)`` for every grid size and every
-count pattern, or a query block is computed twice and another never (or an
-index leaves the buffers). This restates the index arithmetic step by step
-(fill the window, rank it, pick rank r) for the workgroup sizes the kernels
-launch with and checks the permutation property, which the kernel's parity
-tests only see for the grid sizes they run.
+The forwards (``csrc/fwd_common.hpp``, ``tile_coords_lpt``) deal workgroups to
+XCDs round-robin and give each XCD a contiguous run of query blocks, total // 8
+of them and one more for the first total % 8 XCDs. Inside each window of 8192
+query tokens of a run (64 dispatches at block 128, 128 at block 64; the last
+window spans up to two of them) the query blocks are taken longest first, ties
+by index: the workgroup at place r selects the r-th largest key (exact-block
+count, then earlier index first), built bit by bit from ballots. The mapping
+must be a permutation of ``[0, grid)`` for every grid size and every count
+pattern, or a query block is computed twice and another never (or an index
+leaves the buffers). This restates the kernel's arithmetic and checks the
+permutation and the order, which the kernel's parity tests only see for the
+grid sizes they run.
 """
 import numpy as np
 import pytest
 
 
-def _mapping(counts, threads, WINDOW):
-    total = len(counts)
-    out = np.empty(total, dtype=np.int64)
-    for w in range(total):
-        if total % 8 == 0:
-            per, li = total // 8, w // 8
-            base = (w % 8) * per + (li & ~(WINDOW - 1))
-            r = li & (WINDOW - 1)
-            nwin = min(WINDOW, per - (li & ~(WINDOW - 1)))
-        else:
-            base = w & ~(WINDOW - 1)
-            r = w & (WINDOW - 1)
-            nwin = min(WINDOW, total - base)
-        s_cnt = [-1] * WINDOW
-        for t0 in range(threads):  # strided fill, as the kernel does
-            for t in range(t0, WINDOW, threads):
-                s_cnt[t] = counts[base + t] if t < nwin else -1
-        pick = None
-        for t0 in range(threads):
-            for t in range(t0, nwin, threads):
-                rank = sum((s_cnt[u] > s_cnt[t]) or (s_cnt[u] == s_cnt[t] and u < t)
-                           for u in range(nwin))
-                if rank == r:
-                    assert pick is None, "two slots share a rank"
-                    pick = t
-        assert pick is not None, f"no slot has rank {r} (w={w})"
-        out[w] = base + pick
-    return out
-
-
-@pytest.mark.parametrize("total", [1, 7, 8, 24, 63, 64, 65, 200, 512, 520, 1031, 2048 + 8])
-@pytest.mark.parametrize("threads,window", [(256, 64), (128, 128), (128, 64), (256, 128)])
-def test_dispatch_map_is_permutation(total, threads, window):
-    rng = np.random.default_rng(total * 7 + threads)
-    counts = rng.integers(0, 5, size=total).tolist()  # many ties
-    m = _mapping(counts, threads, window)
-    assert sorted(m.tolist()) == list(range(total))
-
-
-@pytest.mark.parametrize("threads,WINDOW", [(256, 64), (128, 128)])
-def test_dispatch_map_longest_first_within_window(threads, WINDOW):
-    total = 8 * 256
-    counts = list(range(total))  # strictly increasing: every window reverses
-    m = _mapping(counts, threads, WINDOW)
-    per = total // 8
-    for xcd in range(8):
-        for win in range(0, per, WINDOW):
-            ws = [m[(li * 8) + xcd] for li in range(win, win + WINDOW)]
-            got = [counts[i] for i in ws]
-            assert got == sorted(got, reverse=True)
-            assert sorted(ws) == list(range(xcd * per + win, xcd * per + win + WINDOW))
-
-
 def _select(counts, WINDOW, NT):
-    """The kernel's selection: XCD shares of total // 8 (+1 for the first
-    total % 8), windows of WINDOW dispatches with a last one of up to two,
-    unique keys (count clamped to [0, NT], earlier index first), the r-th
-    largest key built bit by bit."""
+    """The kernel's selection, one entry per workgroup: keys are unique (count
+    clamped to [0, NT], earlier index first)."""
     total, idx = len(counts), 2 * WINDOW
     bits = idx.bit_length() - 1
     out = np.empty(total, dtype=np.int64)
@@ -93,14 +40,43 @@ def _select(counts, WINDOW, NT):
     return out
 
 
-@pytest.mark.parametrize("total", [1, 7, 8, 9, 65, 513, 8 * 64, 8 * 128 + 8, 8 * 192, 2056, 3079])
+def _windows(per, WINDOW):
+    """The windows of a run of `per` query blocks, as (first, size): whole ones while
+    more than two windows' worth would be left, then what is left in one."""
+    first, out = 0, []
+    while per - first > 2 * WINDOW:
+        out.append((first, WINDOW))
+        first += WINDOW
+    return out + [(first, per - first)]
+
+
+TOTALS = [1, 7, 8, 9, 24, 65, 513, 8 * 64, 8 * 65 + 3, 8 * 128, 8 * 128 + 8, 8 * 129 + 5, 8 * 192, 2056, 3079]
+
+
+@pytest.mark.parametrize("total", TOTALS)
 @pytest.mark.parametrize("window", [64, 128])
-def test_window_selection(total, window):
-    """A permutation for any counts (negative and beyond NT too) and any grid;
-    for XCD shares of one window, the entry that ranking the window gives."""
+def test_dispatch_map_is_permutation(total, window):
+    """For any counts (ties, negative and beyond NT too) and any grid."""
     rng = np.random.default_rng(total + window)
-    counts = rng.integers(-2, 12, size=total).tolist()
-    assert sorted(_select(counts, window, 8).tolist()) == list(range(total))
-    if total % 8 == 0 and total // 8 <= window:
-        counts = rng.integers(0, 9, size=total).tolist()
-        assert np.array_equal(_select(counts, window, 8), _mapping(counts, 256, window))
+    for lo, hi in ((0, 5), (-2, 12)):
+        counts = rng.integers(lo, hi, size=total).tolist()
+        assert sorted(_select(counts, window, 8).tolist()) == list(range(total))
+
+
+@pytest.mark.parametrize("total", TOTALS)
+@pytest.mark.parametrize("window", [64, 128])
+def test_dispatch_map_longest_first_within_window(total, window):
+    """Counts descend, ties by index, along the dispatches of every window of every
+    XCD's run, the last one and runs of unequal length among them."""
+    rng = np.random.default_rng(3 * total + window)
+    counts = rng.integers(0, 9, size=total)
+    m = _select(counts.tolist(), window, 8)
+    start = 0
+    for xcd in range(min(8, total)):
+        run = m[xcd::8]
+        for first, size in _windows(len(run), window):
+            blocks = np.arange(start + first, start + first + size)
+            order = blocks[np.argsort(-counts[blocks], kind="stable")]
+            assert np.array_equal(run[first:first + size], order)
+        start += len(run)
+    assert start == total

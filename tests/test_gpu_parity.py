@@ -756,13 +756,12 @@ def test_one_call_equals_its_stages(pkg, dev, NT, mode):
                                                    (128 * 65 + 1, 128, 2, None), (777, 128, 3, 128)])
 @pytest.mark.parametrize("int8_pv", [True, False])
 def test_preprocess_one_call(pkg, dev, T, block, H, quant_block, int8_pv):
-    """The INT8 preparation's one call against the oracle, bit for bit, with the
-    padding rows of kc and vc zeroed in memory that held something else."""
-    fp = _mods(pkg)[3]
+    """The INT8 preparation's one call against the oracle, bit for bit; and straight into
+    buffers that hold something else, with padding rows behind every length: those of kc
+    and vc are zeroed, the other outputs are the same."""
+    fp, capi = _mods(pkg)[3], importlib.import_module(f"{pkg.__name__}._capi")
     B = 2
     q, k, v = (randn_bf16((B, T, H, 128), s) for s in (31, 32, 33))
-    junk = torch.full((64 << 20,), 7, dtype=torch.uint8, device=dev)  # recycled by the outputs
-    del junk
     print(f"[preprocess] T={T} block={block} H={H} quant_block={quant_block} pv={int8_pv}", flush=True)
     r, qi, qs, ki, ks, vi = fp.fused_preprocess_routing(q.to(dev), k.to(dev), v.to(dev), tau=0.8,
                                                         scale=128 ** -0.5, block=block, int8_pv=int8_pv,
@@ -778,3 +777,19 @@ def test_preprocess_one_call(pkg, dev, T, block, H, quant_block, int8_pv):
     for name, t in (("qi", qi), ("ki", ki)) + ((("vi", vi),) if int8_pv else ()):
         assert np.array_equal(t.cpu().numpy(), ref[name]), name
     assert np.array_equal(f32(qs), ref["qs"].view(np.uint32)) and np.array_equal(f32(ks), ref["ks"].view(np.uint32))
+
+    npad = (NT // 64 + 1) * 64
+    bfs = [torch.full((B, npad, H, 128), 3.0, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    like = lambda t: None if t is None else torch.full_like(t, 5)  # noqa: E731
+    outs = [like(t) for t in (r.qbar, r.kc_mean, r.kc_var, r.vamax_part, r.vscale, r.threshold, r.counts, r.mask, qi,
+                              qs, ki, ks, vi)]
+    dense = [x.to(dev) for x in (q, k, v)]
+    args = [n for x in dense for n in (capi.ptr(x), x.stride(0), x.stride(1), x.stride(2))]
+    capi.call("solattn_preprocess_int8", *args, B, T, H, 128, block, 128 ** -0.5, 0.8, 0, 0, 0, 0,
+              1 if quant_block else 0, capi.ptr(bfs[0]), capi.ptr(bfs[1]), npad, *(capi.ptr(t) for t in outs),
+              capi.stream(dev))
+    for t, want in zip(bfs, (r.kc, r.vc)):
+        assert torch.equal(t[:, :NT], want[:, :NT]) and not bits(t)[:, NT:].any()
+    for t, want in zip(outs, (r.qbar, r.kc_mean, r.kc_var, r.vamax_part, r.vscale, r.threshold, r.counts, r.mask, qi, qs,
+                              ki, ks, vi)):
+        assert (t is None and want is None) or torch.equal(t, want)

@@ -420,7 +420,7 @@ def main():
                                         "FETCH_SIZE + WRITE_SIZE of this kernel, calibrated on "
                                         "a 512 MiB copy (not measured by this run)")
                      if (args.config, block, H) == (2, 128, 24) else None,
-                     "kernel": f"bf16fwd::fwd_bf16_kernel<{block}>",
+                     "kernel": f"bf16fwd::fwd_bf16_kernel<{block}, {D}>",
                      "algorithmic_flops_per_launch": rflops, "launch_ms": round(fwd_ms, 4)},
         "routed_density": round(density, 4),
         "prep_ms": round(prep_ms, 4),

@@ -4,7 +4,7 @@
 // workgroups per CU). Its work is a sequence of 64-key tiles: pooled tiles
 // (chunks of 64 pooled keys with at least one approximate block) and exact
 // tiles (64 tokens each, BLK/64 per exact block, ascending block order).
-// Tiles are copied global -> LDS (double buffered) and consumed by MFMA:
+// Tiles are copied global -> LDS and consumed by MFMA:
 //   S^T = K . Q^T (v_mfma_f32_32x32x16_bf16): lane l holds query row l%32 and
 //     keys 32m + 8(r/4) + 4(l/32) + r%4 in element r of tile m, so row max and
 //     sum need one exchange between lanes 32 apart;

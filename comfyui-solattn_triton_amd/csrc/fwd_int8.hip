@@ -530,13 +530,15 @@ __device__ __forceinline__ void issue_ki_half(uint32_t dst, const I8Source& is, 
 // every copy has a whole step to land. Two waves per SIMD (four workgroups per
 // CU at block 64, two at block 128).
 //
-// Bound: the VALU. A wave's half step takes about 650 cycles of it (16 exps at a
-// quarter of the rate, 16 fma, 32 conversions and scalings, the packing and row
-// sums) against 384 of its MFMAs, and two waves share a SIMD. Against a two-stage
-// step with a single-buffered V tile at block 64 and a three-stage step over whole
+// Bound: no pipe alone. VALU active 59% of the SIMDs' cycles at 32760 tokens and block
+// 128 (55% at 15990 and block 64), MFMA busy 46% (40%), either 82% (76%); waves wait for
+// copies and barriers in a quarter of theirs. A wave's half step issues about 98 VALU
+// instructions, 16 of them exps (460 cycles), beside 384 cycles of its MFMAs. Against a
+// two-stage step with a single-buffered V tile at block 64 and a three-stage step over whole
 // tiles at block 128: 15990 tokens 825 -> 818 and 747 -> 741 us, 7280 tokens 189 ->
 // 186 and 181 -> 177, 32760 tokens 2757 -> 2748 and 2350 -> 2346, 2040 tokens 68.4
-// -> 67.4 and 72.0 -> 72.1. All exps in the four slots with a score MFMA: 0.9%
+// -> 67.4 and 72.0 -> 72.1; but with one workgroup a CU (block 128, 32760 tokens of one
+// head) 177 -> 193, half tiles waiting for the copies twice as often. All exps in the four slots with a score MFMA: 0.9%
 // faster at block 64, 0.8% slower at block 128.
 template <int BLK, bool UKS>
 __global__ void __launch_bounds__(BLK * 2) __attribute__((amdgpu_waves_per_eu(2)))

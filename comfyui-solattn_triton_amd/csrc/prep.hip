@@ -639,7 +639,7 @@ prep_int8_single_read_kernel(const PrepInt8Args a) {
 // NT^2 * HD fmas a head in the contract's order (21 us at NT 512, 24 heads) and
 // a quarter more to unpack kc. Measured, against one row per thread with the
 // centroids as scalar operands (115 SGPRs spilled to lanes, every cache line
-// fetched in eight 16-byte pieces): NT 512 46-53 -> 37-42 us, NT 591 with 40
+// fetched in eight 16-byte pieces): NT 512 46-53 -> 37-45 us, NT 591 with 40
 // heads 113 -> 85, NT 256 23 -> 19.7, NT 190 21.6 -> 17.5. Eight query blocks a
 // wave were slower (43-51 us at NT 512: half the workgroups), as was taking the
 // centroids by the fma's lane move (row_newbcast; 47-55 us).
